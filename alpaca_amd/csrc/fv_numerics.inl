@@ -247,10 +247,96 @@ __device__ __forceinline__ void cell_quantities(double gamma, double b, const do
   q.H = R(H);
 }
 
-// WENO5::ApplyImplementation (weno5.h:88-158) on ordered v1..v5.  ONE_DIV
-// (FP64 with FMA only) forms the weights with one division, below.
-template <typename R, bool ONE_DIV = false>
-__device__ __forceinline__ R weno5(R v1, R v2, R v3, R v4, R v5) {
+// What the Roe average takes from a cell (eigendecomposition.h:266-283): the
+// square root of the density, the velocities, psi, the enthalpy and p / rho.
+// A face needs them of its two inner cells, so a cell's are used by six
+// faces: the plane-marching kernels form them once per cell and keep them in
+// LDS (PackedQ), the tile kernels form them per face.  The same operations on
+// the same values either way.
+template <typename R> struct FaceQ {
+  R rho, sq, vel[3], psi, H, pod;
+};
+
+template <int DIM, typename R>
+__device__ __forceinline__ FaceQ<R> face_quantities(double gamma, double b, const double *c) {
+  CellQ<R> q;
+  cell_quantities<DIM, R>(gamma, b, c, q);
+  FaceQ<R> f;
+  f.rho = q.rho;
+  f.sq = dsqrt(q.rho);
+  f.vel[0] = q.vel[0];
+  f.vel[1] = q.vel[1];
+  f.vel[2] = q.vel[2];
+  f.psi = q.psi;
+  f.H = q.H;
+  f.pod = q.p * q.one_rho;
+  return f;
+}
+
+// A cell's FaceQ as NQ values.  FP64 keeps 1/rho and forms the velocities from
+// the stencil's momenta again (one exact repetition of a product each, 40
+// bytes per cell); the mixed form keeps the velocities, which are rounded
+// from FP64 products, in FP32 (28 bytes).
+template <typename R> struct PackedQ {
+  static constexpr bool kF64 = std::is_same<R, double>::value;
+  static constexpr int NQ = kF64 ? 5 : 7;
+};
+
+// Writes the FaceQ of the cell with conservatives c to q[0], q[STRIDE], ...
+template <int DIM, typename R, int STRIDE>
+__device__ __forceinline__ void store_packed(double gamma, double b, const double *c, R *q) {
+  if constexpr (PackedQ<R>::kF64) {
+    CellQ<double> w;
+    cell_quantities<DIM, double>(gamma, b, c, w);
+    q[0] = dsqrt(w.rho);
+    q[STRIDE] = w.one_rho;
+    q[2 * STRIDE] = w.psi;
+    q[3 * STRIDE] = w.H;
+    q[4 * STRIDE] = w.p * w.one_rho;
+  } else {
+    FaceQ<R> const f = face_quantities<DIM, R>(gamma, b, c);
+    q[0] = f.sq;
+    q[STRIDE] = f.vel[0];
+    q[2 * STRIDE] = f.vel[1];
+    q[3 * STRIDE] = f.vel[2];
+    q[4 * STRIDE] = f.psi;
+    q[5 * STRIDE] = f.H;
+    q[6 * STRIDE] = f.pod;
+  }
+}
+
+template <int DIM, typename R, int STRIDE>
+__device__ __forceinline__ FaceQ<R> load_packed(const R *q, const double *c) {
+  FaceQ<R> f;
+  f.rho = R(c[kMass]);
+  f.sq = q[0];
+  if constexpr (PackedQ<R>::kF64) {
+    double const one_rho = q[STRIDE];
+    f.vel[0] = c[kMomX] * one_rho;
+    f.vel[1] = c[kMomX + 1] * one_rho;
+    f.vel[2] = DIM == 3 ? c[kMomX + DIM - 1] * one_rho : 0.0;
+    f.psi = q[2 * STRIDE];
+    f.H = q[3 * STRIDE];
+    f.pod = q[4 * STRIDE];
+  } else {
+    f.vel[0] = q[STRIDE];
+    f.vel[1] = q[2 * STRIDE];
+    f.vel[2] = q[3 * STRIDE];
+    f.psi = q[4 * STRIDE];
+    f.H = q[5 * STRIDE];
+    f.pod = q[6 * STRIDE];
+  }
+  return f;
+}
+
+// The FP64-with-FMA form takes its own expressions for the reconstruction and
+// the Riemann problem (fewer operations, no bit parity).
+template <typename R> constexpr bool kLean = kFastArith && std::is_same<R, double>::value;
+// The exact FP64 form.
+template <typename R> constexpr bool kExact = !kFastArith && std::is_same<R, double>::value;
+
+// WENO5::ApplyImplementation (weno5.h:88-158) on ordered v1..v5, mixed form.
+template <typename R> __device__ __forceinline__ R weno5(R v1, R v2, R v3, R v4, R v5) {
   R const c_s1 = R(13.0 / 12.0), c_s2 = R(0.25), eps = R(1.0e-6);
   R const s11 = R(1.0) * v1 + R(-2.0) * v2 + R(1.0) * v3;
   R const s12 = R(1.0) * v1 + R(-4.0) * v2 + R(3.0) * v3;
@@ -267,69 +353,180 @@ __device__ __forceinline__ R weno5(R v1, R v2, R v3, R v4, R v5) {
   R const p1 = R(2.0 / 6.0) * v1 + R(-7.0 / 6.0) * v2 + R(11.0 / 6.0) * v3;
   R const p2 = R(-1.0 / 6.0) * v2 + R(5.0 / 6.0) * v3 + R(2.0 / 6.0) * v4;
   R const p3 = R(2.0 / 6.0) * v3 + R(5.0 / 6.0) * v4 + R(-1.0 / 6.0) * v5;
-  R a1, a2, a3, one_a_sum;
-  if constexpr (ONE_DIV) {
-    static_assert(kFastArith && std::is_same<R, double>::value, "FP64 with FMA only");
-    // FP64 with FMA: the weights d_k / x_k over the common denominator
-    // x1 x2 x3, so that w_k = b_k / (b1 + b2 + b3) with b_k = d_k x_i x_j and
-    // one division replaces four.  Each x_k (>= 1e-12) is first clamped to at
-    // most 2^1000 (an infinite one then gets a weight about 1e-289 of the
-    // others', as its d_k / x_k = 0 would; a NaN one still makes the result
-    // NaN through its stencil polynomial), and all three are scaled by 2^-e,
-    // e the exponent of the largest, into (2^-1041, 1), so the b_k stay at
-    // most 0.6 and their sum positive.  Scaling by a power of two changes no
-    // significand, so for x_k in the normal range the quotient has the bits
-    // of the unscaled one.
-    double const c1 = __builtin_fmin(x1, 0x1p1000), c2 = __builtin_fmin(x2, 0x1p1000),
-                 c3 = __builtin_fmin(x3, 0x1p1000);
-    int const e = __builtin_amdgcn_frexp_exp(__builtin_fmax(__builtin_fmax(c1, c2), c3));
-    double const y1 = __builtin_amdgcn_ldexp(c1, -e), y2 = __builtin_amdgcn_ldexp(c2, -e),
-                 y3 = __builtin_amdgcn_ldexp(c3, -e);
-    double const b1 = 0.1 * y2 * y3, b2 = 0.6 * y1 * y3, b3 = 0.3 * y1 * y2;
-    return fast_div64(b1 * p1 + b2 * p2 + b3 * p3, b1 + b2 + b3);
-  }
-  if constexpr (!kFastArith && std::is_same<R, double>::value) {
-    // x_k = (s_k + 1e-6)^2 >= 1e-12 (s_k >= 0 or NaN).  While every x_k is
-    // below 2^700 the hardware's correctly rounded division of 0.1, 0.6, 0.3
-    // by x_k and of 1 by a1 + a2 + a3 (>= 2^-704) scales nothing and fixes up
-    // nothing, so it is exactly its Newton-Raphson core nr_div64 (v_rcp, two
-    // refinements, quotient, one residual correction): same bits, 3 fewer
-    // instructions per division.  The positive x_k order like the high words
-    // of their bit patterns; NaN and infinity fail the test and take the
-    // full division.
-    auto hi = [](double v) { return (unsigned)((unsigned long long)__double_as_longlong(v) >> 32); };
-    unsigned const hmax = __builtin_elementwise_max(__builtin_elementwise_max(hi(x1), hi(x2)), hi(x3));
-    if (__builtin_expect(hmax < 0x6BB00000u, 1)) {  // 2^700
-      a1 = weno_div(0.1, x1);
-      a2 = weno_div(0.6, x2);
-      a3 = weno_div(0.3, x3);
-      one_a_sum = weno_div(1.0, a1 + a2 + a3);
-    } else {
-      a1 = fdiv(0.1, x1);
-      a2 = fdiv(0.6, x2);
-      a3 = fdiv(0.3, x3);
-      one_a_sum = fdiv(1.0, a1 + a2 + a3);
-    }
-  } else {
-    a1 = fdiv(R(0.1), x1);
-    a2 = fdiv(R(0.6), x2);
-    a3 = fdiv(R(0.3), x3);
-    one_a_sum = fdiv(R(1.0), a1 + a2 + a3);
-  }
+  R const a1 = fdiv(R(0.1), x1);
+  R const a2 = fdiv(R(0.6), x2);
+  R const a3 = fdiv(R(0.3), x3);
+  R const one_a_sum = fdiv(R(1.0), a1 + a2 + a3);
   R const w1 = a1 * one_a_sum;
   R const w2 = a2 * one_a_sum;
   R const w3 = a3 * one_a_sum;
   return w1 * p1 + w2 * p2 + w3 * p3;
 }
-// UpwindLeft {0,+1} and UpwindRight {1,-1} (apply_wrapper.h:48-58).
-template <typename R, bool ONE_DIV = false> __device__ __forceinline__ R weno_left(const R *a) {
-  return weno5<R, ONE_DIV>(a[0], a[1], a[2], a[3], a[4]);
+
+// weno5 in the exact FP64 form, in two halves: the smoothness indicators and
+// polynomials, then the weights.  Two products of the reference are fused
+// where a power of two makes the fused form round the same: v1 + (-2 v2) and
+// v1 + (-4 v2) (the product is exact) and t + 0.25 (s s) for (0.25 s) s
+// (scaling by 0.25 changes no significand, and the sum only enters s + 1e-6).
+// 13 fewer instructions per pair of reconstructions; the same bits for
+// |v| < 2^1022.
+struct Weno5 {
+  double x[3], p[3];
+  __device__ __forceinline__ Weno5(double v1, double v2, double v3, double v4, double v5) {
+    double const c_s1 = 13.0 / 12.0, eps = 1.0e-6;
+    double const t3 = 3.0 * v3;
+    double const s11 = __builtin_fma(-2.0, v2, v1) + v3;
+    double const s12 = __builtin_fma(-4.0, v2, v1) + t3;
+    double const s1 = __builtin_fma(0.25, s12 * s12, c_s1 * s11 * s11);
+    double const s21 = __builtin_fma(-2.0, v3, v2) + v4;
+    double const s22 = v2 - v4;
+    double const s2 = __builtin_fma(0.25, s22 * s22, c_s1 * s21 * s21);
+    double const s31 = __builtin_fma(-2.0, v4, v3) + v5;
+    double const s32 = __builtin_fma(-4.0, v4, t3) + v5;
+    double const s3 = __builtin_fma(0.25, s32 * s32, c_s1 * s31 * s31);
+    x[0] = (s1 + eps) * (s1 + eps);
+    x[1] = (s2 + eps) * (s2 + eps);
+    x[2] = (s3 + eps) * (s3 + eps);
+    p[0] = (2.0 / 6.0) * v1 + (-7.0 / 6.0) * v2 + (11.0 / 6.0) * v3;
+    p[1] = (-1.0 / 6.0) * v2 + (5.0 / 6.0) * v3 + (2.0 / 6.0) * v4;
+    p[2] = (2.0 / 6.0) * v3 + (5.0 / 6.0) * v4 + (-1.0 / 6.0) * v5;
+  }
+  // x_k = (s_k + 1e-6)^2 >= 1e-12 (s_k >= 0 or NaN).  The positive x_k order
+  // like the high words of their bit patterns; NaN and infinity lie above.
+  __device__ __forceinline__ unsigned top() const {
+    auto hi = [](double v) { return (unsigned)((unsigned long long)__double_as_longlong(v) >> 32); };
+    return __builtin_elementwise_max(__builtin_elementwise_max(hi(x[0]), hi(x[1])), hi(x[2]));
+  }
+  // CORE: every x_k is below 2^700.  The hardware's correctly rounded division
+  // of 0.1, 0.6, 0.3 by x_k and of 1 by a1 + a2 + a3 (>= 2^-704) then scales
+  // nothing and fixes up nothing, so it is exactly its Newton-Raphson core
+  // nr_div64 (v_rcp, two refinements, quotient, one residual correction):
+  // same bits, 3 fewer instructions per division.
+  template <bool CORE> __device__ __forceinline__ double value() const {
+    auto div = [](double a, double b) { return CORE ? weno_div(a, b) : fdiv(a, b); };
+    double const a1 = div(0.1, x[0]);
+    double const a2 = div(0.6, x[1]);
+    double const a3 = div(0.3, x[2]);
+    double const one_a_sum = div(1.0, a1 + a2 + a3);
+    double const w1 = a1 * one_a_sum;
+    double const w2 = a2 * one_a_sum;
+    double const w3 = a3 * one_a_sum;
+    return w1 * p[0] + w2 * p[1] + w3 * p[2];
+  }
+};
+
+// UpwindLeft {0,+1} of l and UpwindRight {1,-1} of r (apply_wrapper.h:48-58) in
+// the exact form.  Returns whether every x_k was in the core's range; l[0..4]
+// and r[1..5] are then finite.  PAIRED: one range check for both; otherwise
+// one after the other.  The split decides what the register allocator holds
+// at once: the flux-splitting face (two projections per field) takes 207 VGPRs
+// paired and 256 in sequence, the finite-volume face (one) 241 and 224.
+template <bool PAIRED>
+__device__ __forceinline__ bool weno_pair_exact(const double *l, const double *r, double &left,
+                                                double &right) {
+  auto in_core = [](unsigned top) { return top < 0x6BB00000u; };  // 2^700
+  if constexpr (PAIRED) {
+    Weno5 const a(l[0], l[1], l[2], l[3], l[4]), b(r[5], r[4], r[3], r[2], r[1]);
+    bool const core = in_core(__builtin_elementwise_max(a.top(), b.top()));
+    if (__builtin_expect(core, 1)) {
+      left = a.template value<true>();
+      right = b.template value<true>();
+    } else {
+      left = a.template value<false>();
+      right = b.template value<false>();
+    }
+    return core;
+  } else {
+    auto one = [&](Weno5 const &a, double &v) {
+      bool const core = in_core(a.top());
+      if (__builtin_expect(core, 1))
+        v = a.template value<true>();
+      else
+        v = a.template value<false>();
+      return core;
+    };
+    bool const cl = one(Weno5(l[0], l[1], l[2], l[3], l[4]), left);
+    bool const cr = one(Weno5(r[5], r[4], r[3], r[2], r[1]), right);
+    return cl && cr;
+  }
 }
-template <typename R, bool ONE_DIV = false> __device__ __forceinline__ R weno_right(const R *a) {
-  return weno5<R, ONE_DIV>(a[5], a[4], a[3], a[2], a[1]);
+
+// WENO5 in the FP64-with-FMA form, from the first differences d1..d4 and the
+// second differences D1..D3 of the five values, relative to the middle value:
+//   4 s_k = 13/3 D_k^2 + m_k^2, m = (3 d2 - d1, d2 + d3, 3 d3 - d4),
+//   6 (p_k - v3) = e_k = (5 d2 - 2 d1, d2 + 2 d3, 4 d3 - d4),
+// and the weights w_k = d_k / x_k, x_k = (s_k + 1e-6)^2, over the common
+// denominator x1 x2 x3, so that one division serves all:
+//   v = v3 + 1/6 (z1 e1 + 6 z2 e2 + 3 z3 e3) / (z1 + 6 z2 + 3 z3),
+// z1 = x2 x3, z2 = x1 x3, z3 = x1 x2.  The four times scaled s_k + 1e-6 are
+// scaled by a power of two r (which changes no significand) so that the
+// largest lies in [1/8, 1]; er = 4e-6 r is kept at least 2^-250, so the x_k
+// stay in [2^-500, 1] and the z_k normal.  An infinite s_k is clamped to 1 (its
+// stencil gets a weight 2^-500 of the others', as its d_k / x_k = 0 would); a
+// NaN still makes the result NaN through its e_k.
+// The left and right reconstructions of one array share the differences, the
+// D terms and the scale: 96 instructions for both, against 133 with the
+// candidate polynomials and indicators formed from the values.
+struct WenoScale {
+  double r, er;
+  __device__ __forceinline__ explicit WenoScale(double smax) {
+    unsigned h = (unsigned)((unsigned long long)__double_as_longlong(smax) >> 32);
+    h = __builtin_elementwise_min(__builtin_elementwise_max(h, 0x3EE00000u), 0x7FB00000u);
+    r = __longlong_as_double((long long)((unsigned long long)(0x7FC00000u - (h & 0x7FF00000u)) << 32));
+    er = __builtin_fmax(4.0e-6 * r, 0x1p-250);
+  }
+};
+__device__ __forceinline__ double max3(double a, double b, double c) {
+  return __builtin_fmax(__builtin_fmax(a, b), c);
 }
-// The FP64-with-FMA form reconstructs with one division per WENO5.
-template <typename R> constexpr bool kWenoOneDiv = kFastArith && std::is_same<R, double>::value;
+// 6 (v - v3): indicators s_k (times four), differences d1..d4.
+__device__ __forceinline__ double weno_lean(const WenoScale &w, double s1, double s2, double s3,
+                                            double d1, double d2, double d3, double d4) {
+  auto x = [&w](double s) {
+    double const t = __builtin_fmin(__builtin_fmax(s * w.r + w.er, 0.0), 1.0);
+    return t * t;
+  };
+  double const x1 = x(s1), x2 = x(s2), x3 = x(s3);
+  double const z1 = x2 * x3, z2 = 6.0 * (x1 * x3), z3 = 3.0 * (x1 * x2);
+  double const num = z1 * (5.0 * d2 - 2.0 * d1) + z2 * (d2 + 2.0 * d3) + z3 * (4.0 * d3 - d4);
+  return fast_div64(num, z1 + z2 + z3);
+}
+__device__ __forceinline__ void weno_pair_lean(const double *a, double &left, double &right) {
+  double const d0 = a[1] - a[0], d1 = a[2] - a[1], d2 = a[3] - a[2], d3 = a[4] - a[3],
+               d4 = a[5] - a[4];
+  double const c = 13.0 / 3.0;
+  double const D0 = d1 - d0, D1 = d2 - d1, D2 = d3 - d2, D3 = d4 - d3;
+  double const C0 = c * D0, C1 = c * D1, C2 = c * D2, C3 = c * D3;
+  auto ind = [](double D, double C, double m) { return D * C + m * m; };
+  double const l1 = ind(D0, C0, 3.0 * d1 - d0), l2 = ind(D1, C1, d1 + d2), l3 = ind(D2, C2, 3.0 * d2 - d3);
+  double const r1 = ind(D3, C3, 3.0 * d3 - d4), r2 = ind(D2, C2, d3 + d2), r3 = ind(D1, C1, 3.0 * d2 - d1);
+  WenoScale const w(__builtin_fmax(max3(l1, l2, l3), max3(r1, r2, r3)));
+  left = a[2] + (1.0 / 6.0) * weno_lean(w, l1, l2, l3, d0, d1, d2, d3);
+  right = a[3] - (1.0 / 6.0) * weno_lean(w, r1, r2, r3, d4, d3, d2, d1);
+}
+__device__ __forceinline__ double weno_one_lean(double v1, double v2, double v3, double v4, double v5) {
+  double const d1 = v2 - v1, d2 = v3 - v2, d3 = v4 - v3, d4 = v5 - v4;
+  double const c = 13.0 / 3.0;
+  double const D1 = d2 - d1, D2 = d3 - d2, D3 = d4 - d3;
+  auto ind = [c](double D, double m) { return D * (c * D) + m * m; };
+  double const s1 = ind(D1, 3.0 * d2 - d1), s2 = ind(D2, d2 + d3), s3 = ind(D3, 3.0 * d3 - d4);
+  WenoScale const w(max3(s1, s2, s3));
+  return v3 + (1.0 / 6.0) * weno_lean(w, s1, s2, s3, d1, d2, d3, d4);
+}
+
+// The left reconstruction of l and the right one of r (apply_wrapper.h:48-58).
+template <typename R, bool PAIRED = true>
+__device__ __forceinline__ void weno_pair(const R *l, const R *r, R &left, R &right) {
+  if constexpr (kExact<R>) {
+    (void)weno_pair_exact<true>(l, r, left, right);
+  } else if constexpr (kLean<R>) {
+    left = weno_one_lean(l[0], l[1], l[2], l[3], l[4]);
+    right = weno_one_lean(r[5], r[4], r[3], r[2], r[1]);
+  } else {
+    left = weno5<R>(l[0], l[1], l[2], l[3], l[4]);
+    right = weno5<R>(r[5], r[4], r[3], r[2], r[1]);
+  }
+}
 
 template <int NE, typename R> struct Eig {
   R L[NE][NE];
@@ -425,7 +622,7 @@ __device__ __forceinline__ void roe_right_eigenvectors(Eig<DIM + 2, R> &ev) {
 // t = cell i, n = cell i+1 along DIR.  Returns false (all zero) when a
 // density is not positive.
 template <int DIM, int DIR, typename R, bool kDefer = kDeferRight<R>>
-__device__ __forceinline__ bool roe_eigensystem(R gamma, const CellQ<R> &t, const CellQ<R> &n,
+__device__ __forceinline__ bool roe_eigensystem(R gamma, const FaceQ<R> &t, const FaceQ<R> &n,
                                                 Eig<DIM + 2, R> &ev) {
   constexpr int NE = DIM + 2;
   constexpr int m1 = Minor<DIR>::m1, m2 = Minor<DIR>::m2;
@@ -451,8 +648,8 @@ __device__ __forceinline__ bool roe_eigensystem(R gamma, const CellQ<R> &t, cons
   R const v_n = n.vel[m1];
   R const w_n = DIM == 3 ? n.vel[m2] : R(0.0);
 
-  R const sq_t = dsqrt(t.rho);
-  R const sq_n = dsqrt(n.rho);
+  R const sq_t = t.sq;
+  R const sq_n = n.sq;
   R const rho_div = fdiv(R(1.0), sq_t + sq_n);
   R const rho_roe = sq_t * sq_n;
   R const one_rho_roe = fdiv(R(1.0), rho_roe);
@@ -467,7 +664,7 @@ __device__ __forceinline__ bool roe_eigensystem(R gamma, const CellQ<R> &t, cons
   R const q2 = dams<DIM>(u * u, v * v, w * w);
   R const tmp = dams<DIM>((u_t - u_n) * (u_t - u_n), (v_t - v_n) * (v_t - v_n),
                           (w_t - w_n) * (w_t - w_n));
-  R const pod = ((t.p * t.one_rho) * sq_t + (n.p * n.one_rho) * sq_n) * rho_div +
+  R const pod = (t.pod * sq_t + n.pod * sq_n) * rho_div +
                 R(0.5) * rho_roe * (rho_div * rho_div) * tmp;
   R const cc = psi + g * pod;
   R const one_cc = fdiv(R(1.0), cc);
@@ -635,10 +832,10 @@ __device__ __forceinline__ void advection(const double *c, const Prim<double> &p
 // about 340 registers (one wave per SIMD).
 constexpr int kRoePrefetch = 2;  // stencil cells read ahead for the next field
 
-template <int DIM, int DIR>
+template <int DIM, int DIR, typename QS>
 __device__ __forceinline__ void roe_split_flux_exact(double gamma, double b,
                                                      const double *__restrict__ blk, int off,
-                                                     double *f) {
+                                                     const QS &qs, double *f) {
   constexpr int NE = DIM + 2;
   constexpr int S = axis_stride<DIM, DIR>();
   BlockReader<DIM> const rd(blk);
@@ -655,10 +852,7 @@ __device__ __forceinline__ void roe_split_flux_exact(double gamma, double b,
       Ui[e] = at(off0, 2, e);
       Un[e] = at(off0, 3, e);
     }
-    CellQ<double> qt, qn;
-    cell_quantities<DIM, double>(gamma, b, Ui, qt);
-    cell_quantities<DIM, double>(gamma, b, Un, qn);
-    roe_eigensystem<DIM, DIR, double, true>(gamma, qt, qn, ev);
+    roe_eigensystem<DIM, DIR, double, true>(gamma, qs.left(Ui), qs.right(Un), ev);
   }
   double dep = ev.lam[0];
   double adv[6][NE];
@@ -724,7 +918,9 @@ __device__ __forceinline__ void roe_split_flux_exact(double gamma, double b,
 #pragma unroll
         for (int e = 0; e < NE; ++e) U[m][e] = at(o, m, e);
     }
-    chf[n] = 0.5 * (weno_left(pos) + weno_right(neg));
+    double wl, wr;
+    weno_pair<double>(pos, neg, wl, wr);
+    chf[n] = 0.5 * (wl + wr);
     dep = chf[n];
     if (n + 1 < NE) {
       int o = off0;
@@ -748,9 +944,10 @@ __device__ __forceinline__ void roe_split_flux_exact(double gamma, double b,
 // cell -- load, advection, projection onto every field -- which keeps few
 // values live: 2 waves per SIMD for the FP64-with-FMA kernel, 3 for the mixed
 // one.  Each projection is the expression of the exact form.
-template <int DIM, int DIR, typename R>
+template <int DIM, int DIR, typename R, typename QS>
 __device__ __forceinline__ void roe_split_flux(double gamma64, double b64,
-                                               const double *__restrict__ base, R *f) {
+                                               const double *__restrict__ base, const QS &qs,
+                                               R *f) {
   constexpr int NE = DIM + 2;
   constexpr bool kShift = std::is_same<R, float>::value;
   R const gamma = R(gamma64);
@@ -760,16 +957,13 @@ __device__ __forceinline__ void roe_split_flux(double gamma64, double b64,
       c[e] = base[e * Dims<DIM>::FIELD + (m - 2) * axis_stride<DIM, DIR>()];
   };
   Eig<NE, R> ev;
-  CellQ<R> qt, qn;
   double adv2[NE];  // advection of cell i (FP64; mixed form only)
   R chf[NE];
   {
     double Ui[NE], Un[NE];
     load(2, Ui);
     load(3, Un);
-    cell_quantities<DIM, R>(gamma64, b64, Ui, qt);
-    cell_quantities<DIM, R>(gamma64, b64, Un, qn);
-    roe_eigensystem<DIM, DIR, R, false>(gamma, qt, qn, ev);
+    roe_eigensystem<DIM, DIR, R, false>(gamma, qs.left(Ui), qs.right(Un), ev);
     if constexpr (kShift) {
       Prim<double> pd;
       cons_to_prim<DIM, double>(gamma64, b64, Ui, pd);
@@ -818,9 +1012,11 @@ __device__ __forceinline__ void roe_split_flux(double gamma64, double b64,
       }
     }
 #pragma unroll
-    for (int n = 0; n < NE; ++n)
-      chf[n] = R(0.5) * (weno_left<R, kWenoOneDiv<R>>(pos[n]) +
-                         weno_right<R, kWenoOneDiv<R>>(neg[n]));
+    for (int n = 0; n < NE; ++n) {
+      R wl, wr;
+      weno_pair<R>(pos[n], neg[n], wl, wr);
+      chf[n] = R(0.5) * (wl + wr);
+    }
   }
   R phys[NE];
   to_physical<DIM, DIR>(chf, ev.Rm, phys);
@@ -834,16 +1030,177 @@ __device__ __forceinline__ void roe_split_flux(double gamma64, double b64,
   }
 }
 
+// The reconstruction of the FP64-with-FMA form: the products with the Roe
+// eigenvectors factored through the quantities they share.  With
+//   Y = E - u m_n - v m_1 - w m_2 + (q^2 - H) rho,
+//   A = g/(2c^2) Y + rho/2,  B = (u rho - m_n) / (2c)
+// the amplitudes of the waves u-c, u+c and of the entropy wave are A + B, A - B
+// and -Y/c^2 (15 instructions per cell for all five, against 19 row by row),
+// and back, with a = the five reconstructed amplitudes,
+//   rho = a_- + a_+ + g a_e,  d = c (a_+ - a_-),  m_n = u rho + d, ...
+// The stencil is dead once Y, A, B and the shear amplitudes are formed, and no
+// eigenvector matrix is held.
+template <int DIM, int DIR, typename QS>
+__device__ __forceinline__ void fv_reconstruct_lean(double gamma, const double (&U)[6][DIM + 2],
+                                                    const QS &qs, double *cl, double *cr) {
+  constexpr int m1 = Minor<DIR>::m1, m2 = Minor<DIR>::m2;
+  constexpr int Mp = kMomX + DIR, M1 = kMomX + m1, M2 = kMomX + m2;
+  FaceQ<double> const t = qs.left(U[2]), n = qs.right(U[3]);
+  if (!(t.rho > 0.0) || !(n.rho > 0.0)) {
+    if (t.rho <= 0.0 || n.rho <= 0.0) {
+      // No eigensystem: a zero state, whose face is skipped.
+#pragma unroll
+      for (int e = 0; e < DIM + 2; ++e) cl[e] = cr[e] = 0.0;
+      return;
+    }
+  }
+  double const rho_div = fdiv(1.0, t.sq + n.sq);
+  double const rho_roe = t.sq * n.sq;
+  double const one_rho = fdiv(1.0, rho_roe);
+  auto mean = [&](double a, double b) { return (a * t.sq + b * n.sq) * rho_div; };
+  double const u = mean(t.vel[DIR], n.vel[DIR]), v = mean(t.vel[m1], n.vel[m1]);
+  double const w = DIM == 3 ? mean(t.vel[m2], n.vel[m2]) : 0.0;
+  double const g = gamma - 1.0;
+  double const H = mean(t.H, n.H);
+  double const du = t.vel[DIR] - n.vel[DIR], dv = t.vel[m1] - n.vel[m1];
+  double q2 = u * u + v * v, dq = du * du + dv * dv;
+  if constexpr (DIM == 3) {
+    double const dw = t.vel[m2] - n.vel[m2];
+    q2 += w * w;
+    dq += dw * dw;
+  }
+  double const cc = mean(t.psi + g * t.pod, n.psi + g * n.pod) +
+                    g * (0.5 * rho_roe * (rho_div * rho_div) * dq);
+  double const one_cc = fdiv(1.0, cc);
+  double const c = dsqrt(cc);
+  double const kY = q2 - H, kA = 0.5 * g * one_cc, kB = 0.5 * one_cc * c;
+  double const kBu = kB * u, kv = v * one_rho, kw = w * one_rho;
+
+  double Y[6], B[6], lo[DIM + 2], hi[DIM + 2];
+  {
+    double s1[6], s2[6];
+#pragma unroll
+    for (int m = 0; m < 6; ++m) {
+      s1[m] = kv * U[m][kMass] - one_rho * U[m][M1];
+      Y[m] = U[m][kEnergy] - u * U[m][Mp] - v * U[m][M1] + kY * U[m][kMass];
+      B[m] = kBu * U[m][kMass] - kB * U[m][Mp];
+      if constexpr (DIM == 3) {
+        s2[m] = one_rho * U[m][M2] - kw * U[m][kMass];
+        Y[m] -= w * U[m][M2];
+      }
+    }
+    weno_pair_lean(s1, lo[1], hi[1]);
+    if constexpr (DIM == 3) weno_pair_lean(s2, lo[2], hi[2]);
+  }
+  double A[6], x[6];
+#pragma unroll
+  for (int m = 0; m < 6; ++m) {
+    A[m] = kA * Y[m] + 0.5 * U[m][kMass];
+    x[m] = -one_cc * Y[m];
+  }
+  weno_pair_lean(x, lo[DIM], hi[DIM]);
+#pragma unroll
+  for (int m = 0; m < 6; ++m) x[m] = A[m] + B[m];
+  weno_pair_lean(x, lo[0], hi[0]);
+#pragma unroll
+  for (int m = 0; m < 6; ++m) x[m] = A[m] - B[m];
+  weno_pair_lean(x, lo[DIM + 1], hi[DIM + 1]);
+  auto back = [&](const double *a, double *o) {
+    double const rho = a[0] + a[DIM + 1] + g * a[DIM];
+    double const d = c * (a[DIM + 1] - a[0]);
+    double const t1 = rho_roe * a[1];
+    double e = H * rho + u * d - cc * a[DIM] - v * t1;
+    o[kMass] = rho;
+    o[Mp] = u * rho + d;
+    o[M1] = v * rho - t1;
+    if constexpr (DIM == 3) {
+      double const t2 = rho_roe * a[2];
+      o[M2] = w * rho + t2;
+      e += w * t2;
+    }
+    o[kEnergy] = e;
+  };
+  back(lo, cl);
+  back(hi, cr);
+}
+
+// FP64 square root of a positive argument: nr_sqrt64 without its zero case.
+__device__ __forceinline__ double nr_sqrt64_pos(double x) {
+  double const r = __builtin_amdgcn_rsq(x);
+  double g = x * r;
+  double h = 0.5 * r;
+  double const e = __builtin_fma(-g, h, 0.5);
+  g = __builtin_fma(g, e, g);
+  h = __builtin_fma(h, e, h);
+  return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+}
+
+// The Riemann problem of the FP64-with-FMA form (hllc and einfeldt below): the
+// side of the contact the face lies on is selected before its star state is
+// formed, and that state takes one division: with i = 1 / (S - S*),
+// chi = (S - u) i and p / (rho (S - u)) rho chi = p i.  (The reference's
+// clamped speed differs from S only where it is zero, and it then multiplies
+// the star state by zero.)  1/rho serves the velocities, the pressure and the
+// sound speed.  Five divisions per face instead of twelve.
+template <int DIM, int DIR>
+__device__ __forceinline__ void fv_riemann_lean(double gamma, double b, const double *cl,
+                                                const double *cr, double *f) {
+  constexpr int NE = DIM + 2;
+  constexpr int Mp = kMomX + DIR, M1 = kMomX + Minor<DIR>::m1, M2 = kMomX + Minor<DIR>::m2;
+#pragma unroll
+  for (int e = 0; e < NE; ++e) f[e] = 0.0;
+  double const eps = 2.220446049250313080847263336181640625e-16;  // DBL_EPSILON
+  if (cl[kMass] <= eps || cr[kMass] <= eps) return;
+  auto pressure = [&](const double *c, double one_rho, double &u) {
+    u = c[Mp] * one_rho;
+    double k = c[Mp] * u + c[M1] * (c[M1] * one_rho);
+    if constexpr (DIM == 3) k += c[M2] * (c[M2] * one_rho);
+    return (gamma - 1.0) * (c[kEnergy] - 0.5 * k) - gamma * b;
+  };
+  double const il = fdiv(1.0, cl[kMass]), ir = fdiv(1.0, cr[kMass]);
+  double ul, ur;
+  double const pl = pressure(cl, il, ul), pr = pressure(cr, ir, ur);
+  if (pl <= -b || pr <= -b) return;
+  double const ccl = gamma * (pl + b) * il, ccr = gamma * (pr + b) * ir;
+  double const al = nr_sqrt64_pos(ccl), ar = nr_sqrt64_pos(ccr);
+  double const sql = nr_sqrt64_pos(cl[kMass]), sqr = nr_sqrt64_pos(cr[kMass]);
+  double const rd = fdiv(1.0, sql + sqr);
+  double const um = (ul * sql + ur * sqr) * rd;
+  double const du = ur - ul;
+  double const ce = nr_sqrt64_pos((ccl * sql + ccr * sqr) * rd + 0.5 * (sql * rd) * (sqr * rd) * (du * du));
+  double const sl = __builtin_fmin(um - ce, ul - al), sr = __builtin_fmax(um + ce, ur + ar);
+  double const dl = sl - ul, dr = sr - ur;
+  double const sc = fdiv((pr - pl) + (cl[Mp] * dl - cr[Mp] * dr), cl[kMass] * dl - cr[kMass] * dr);
+  bool const left = sc >= 0.0;
+  double c[NE];
+#pragma unroll
+  for (int e = 0; e < NE; ++e) c[e] = left ? cl[e] : cr[e];
+  double const p = left ? pl : pr, u = left ? ul : ur, d = left ? dl : dr, s = left ? sl : sr;
+  double const sk = left ? __builtin_fmin(sl, 0.0) : __builtin_fmax(sr, 0.0);
+  double const i = fdiv(1.0, s - sc);
+  double const chi = d * i, rchi = c[kMass] * chi;
+  double const n = rchi * sc, chi1 = chi - 1.0;
+  f[kMass] = c[Mp] + sk * (rchi - c[kMass]);
+  f[Mp] = (c[Mp] * u + p) + sk * (n - c[Mp]);
+  f[kEnergy] = u * (c[kEnergy] + p) + sk * (chi1 * c[kEnergy] + (sc - u) * (n + p * i));
+  f[M1] = c[M1] * (u + sk * chi1);
+  if constexpr (DIM == 3) f[M2] = c[M2] * (u + sk * chi1);
+}
+
 // The finite-volume face (FiniteVolumeScheme::ComputeFluxes,
 // finite_volume_scheme.cpp:160-251, with CharacteristicStateReconstruction,
-// characteristic_state_reconstruction.h:60-134) from its stencil Ud (FP64
-// conservatives of cells i-2..i+3 along DIR).  Writes f (zero when the
-// reference skips the face).
-template <int DIM, int DIR, typename R>
-__device__ __forceinline__ void fv_face(double gamma64, double b64, const double (&Ud)[6][DIM + 2],
-                                        R *f) {
+// characteristic_state_reconstruction.h:60-134) in two parts: fv_reconstruct
+// forms the states cl and cr left and right of the face from its stencil Ud
+// (FP64 conservatives of cells i-2..i+3 along DIR), fv_riemann the flux.
+template <int DIM, int DIR, typename R, typename QS>
+__device__ __forceinline__ void fv_reconstruct(double gamma64, const double (&Ud)[6][DIM + 2],
+                                               const QS &qs, R *cl, R *cr) {
+  if constexpr (kLean<R>) {
+    fv_reconstruct_lean<DIM, DIR>(gamma64, Ud, qs, cl, cr);
+    return;
+  }
+  R const gamma = R(gamma64);
   constexpr int NE = DIM + 2;
-  R const gamma = R(gamma64), b = R(b64);
   // Mixed form: the stencil enters the FP32 reconstruction as differences
   // from cell i (taken in FP64), and cell i is added back in FP64 after the
   // back-transform.  Exact arithmetic gives the same flux: the WENO5
@@ -853,35 +1210,54 @@ __device__ __forceinline__ void fv_face(double gamma64, double b64, const double
   // state's magnitude.
   constexpr bool kShift = std::is_same<R, float>::value;
   Eig<NE, R> ev;
-#pragma unroll
-  for (int e = 0; e < NE; ++e) f[e] = R(0.0);
   R U[6][NE];
 #pragma unroll
   for (int m = 0; m < 6; ++m)
 #pragma unroll
     for (int e = 0; e < NE; ++e) U[m][e] = kShift ? R(Ud[m][e] - Ud[2][e]) : R(Ud[m][e]);
-  CellQ<R> qt, qn;
-  cell_quantities<DIM, R>(gamma64, b64, Ud[2], qt);
-  cell_quantities<DIM, R>(gamma64, b64, Ud[3], qn);
-  roe_eigensystem<DIM, DIR>(gamma, qt, qn, ev);
+  roe_eigensystem<DIM, DIR>(gamma, qs.left(Ud[2]), qs.right(Ud[3]), ev);
   R minus[NE], plus[NE];
-#pragma unroll
-  for (int n = 0; n < NE; ++n) {
-    R uc[6];
+  // Row n of L times the stencil; SKIP leaves out the row's structural zeros.
+  // The reference's sum starts at 0.0; the exact form starts at the first
+  // product, which can differ in the sign of a zero only, and no zero's sign
+  // passes the back-transform's sum, which does start at 0.0.
+  auto project = [&](int n, auto skip, R *uc) {
 #pragma unroll
     for (int m = 0; m < 6; ++m) {
       R s = R(0.0);
+      bool first = kExact<R>;
 #pragma unroll
       for (int q = 0; q < NE; ++q) {
         int const l = seq<DIM, DIR>(q);
-        if (!(kSkipZeros<R> && left_zero<DIM, DIR>(n, l))) s += ev.L[n][l] * U[m][l];
+        if (decltype(skip)::value && left_zero<DIM, DIR>(n, l)) continue;
+        s = first ? ev.L[n][l] * U[m][l] : s + ev.L[n][l] * U[m][l];
+        first = false;
       }
       uc[m] = s;
     }
-    minus[n] = weno_left<R, kWenoOneDiv<R>>(uc);
-    plus[n] = weno_right<R, kWenoOneDiv<R>>(uc);
+  };
+  // In the exact form a zero entry's product matters only where a stencil
+  // value is not finite (0 * x is then NaN, as in the reference).  Field 0's
+  // row is dense: if its reconstruction stayed in the core's range, every
+  // stencil value is finite, and the shear rows leave their zeros out.
+  bool finite = true;
+#pragma unroll
+  for (int n = 0; n < NE; ++n) {
+    R uc[6];
+    if constexpr (kExact<R>) {
+      if (n >= 1 && n < DIM) {
+        project(n, std::true_type{}, uc);
+        if (__builtin_expect(!finite, 0)) project(n, std::false_type{}, uc);
+      } else {
+        project(n, std::false_type{}, uc);
+      }
+      bool const core = weno_pair_exact<false>(uc, uc, minus[n], plus[n]);
+      if (n == 0) finite = core;
+    } else {
+      project(n, std::false_type{}, uc);
+      weno_pair<R>(uc, uc, minus[n], plus[n]);
+    }
   }
-  R cl[NE], cr[NE];
   roe_right_eigenvectors<DIM, DIR>(ev);
   to_physical<DIM, DIR>(minus, ev.Rm, cl);
   to_physical<DIM, DIR>(plus, ev.Rm, cr);
@@ -892,16 +1268,6 @@ __device__ __forceinline__ void fv_face(double gamma64, double b64, const double
       cr[e] = R(double(cr[e]) + Ud[2][e]);
     }
   }
-  R const eps = R(2.220446049250313080847263336181640625e-16);  // DBL_EPSILON
-  if (cl[kMass] <= eps || cr[kMass] <= eps) return;
-  Prim<R> pl, pr;
-  cons_to_prim<DIM>(gamma, b, cl, pl);
-  cons_to_prim<DIM>(gamma, b, cr, pr);
-  if (pl.p <= -b || pr.p <= -b) return;
-  R hf[NE];
-  hllc<DIM, DIR>(gamma, b, cl, cr, pl, pr, hf);
-#pragma unroll
-  for (int e = 0; e < NE; ++e) f[e] += hf[e];
 }
 
 // The six-cell stencil of a face: cells off + (m - 2) * stride, m = 0..5,
@@ -918,31 +1284,107 @@ __device__ __forceinline__ void load_stencil(const BlockReader<DIM> &rd, int off
                     e * Dims<DIM>::FIELD * (int)sizeof(double));
 }
 
+// Writes f (zero when the reference skips the face).
+template <int DIM, int DIR, typename R>
+__device__ __forceinline__ void fv_riemann(double gamma64, double b64, const R *cl, const R *cr,
+                                           R *f) {
+  if constexpr (kLean<R>) {
+    fv_riemann_lean<DIM, DIR>(gamma64, b64, cl, cr, f);
+    return;
+  }
+  constexpr int NE = DIM + 2;
+  R const gamma = R(gamma64), b = R(b64);
+#pragma unroll
+  for (int e = 0; e < NE; ++e) f[e] = R(0.0);
+  R const eps = R(2.220446049250313080847263336181640625e-16);  // DBL_EPSILON
+  if (cl[kMass] <= eps || cr[kMass] <= eps) return;
+  Prim<R> pl, pr;
+  cons_to_prim<DIM>(gamma, b, cl, pl);
+  cons_to_prim<DIM>(gamma, b, cr, pr);
+  if (pl.p <= -b || pr.p <= -b) return;
+  R hf[NE];
+  hllc<DIM, DIR>(gamma, b, cl, cr, pl, pr, hf);
+#pragma unroll
+  for (int e = 0; e < NE; ++e) f[e] += hf[e];
+}
+
+template <int DIM, int DIR, typename R, typename QS>
+__device__ __forceinline__ void fv_face(double gamma64, double b64, const double *blk, int off,
+                                        const QS &qs, R *f) {
+  BlockReader<DIM> const rd(blk);
+  double Ud[6][DIM + 2];
+  load_stencil<DIM>(rd, off, axis_stride<DIM, DIR>(), Ud);
+  R cl[DIM + 2], cr[DIM + 2];
+  fv_reconstruct<DIM, DIR, R>(gamma64, Ud, qs, cl, cr);
+  fv_riemann<DIM, DIR, R>(gamma64, b64, cl, cr, f);
+}
+
+// The conservatives of one cell.
+template <int DIM>
+__device__ __forceinline__ void load_cell(const BlockReader<DIM> &rd, int off, double (&c)[DIM + 2]) {
+#pragma unroll
+  for (int e = 0; e < DIM + 2; ++e)
+    c[e] = rd(off * (int)sizeof(double), e * Dims<DIM>::FIELD * (int)sizeof(double));
+}
+
 // One face flux from the six-cell stencil Ud[m] (FP64 conservatives of cells
 // i-2..i+3 along DIR); reconstruction and Riemann arithmetic in R.
 // FV:  FiniteVolumeScheme::ComputeFluxes (finite_volume_scheme.cpp:160-251)
 //      + CharacteristicStateReconstruction (characteristic_state_reconstruction.h:60-134).
 // Roe: FluxSplittingScheme::ComputeFluxes + ComputeAdvection
 //      (flux_splitting_scheme.cpp:42-76, 185-315).
-// Writes f (zero when the reference skips the face).
-template <int DIM, int DIR, int FLUX, typename R>
+// Writes f (zero when the reference skips the face).  qs gives the FaceQ of
+// the cells left and right of the face.
+template <int DIM, int DIR, int FLUX, typename R, typename QS>
 __device__ __forceinline__ void face_flux(double gamma64, double b64,
-                                          const double *__restrict__ blk, int off, R *f) {
+                                          const double *__restrict__ blk, int off, const QS &qs,
+                                          R *f) {
   constexpr int NE = DIM + 2;
   const double *__restrict__ base = blk + off;
 #pragma unroll
   for (int e = 0; e < NE; ++e) f[e] = R(0.0);
   if constexpr (FLUX == 0) {
-    BlockReader<DIM> const rd(blk);
-    double Ud[6][NE];
-    load_stencil<DIM>(rd, off, axis_stride<DIM, DIR>(), Ud);
-    fv_face<DIM, DIR, R>(gamma64, b64, Ud, f);
+    fv_face<DIM, DIR, R>(gamma64, b64, blk, off, qs, f);
   } else if constexpr (std::is_same<R, double>::value && !kFastArith) {
-    roe_split_flux_exact<DIM, DIR>(gamma64, b64, blk, off, f);
+    roe_split_flux_exact<DIM, DIR>(gamma64, b64, blk, off, qs, f);
   } else {
-    roe_split_flux<DIM, DIR, R>(gamma64, b64, base, f);
+    roe_split_flux<DIM, DIR, R>(gamma64, b64, base, qs, f);
   }
 }
+
+// FaceQ sources of a face.  Formed: from the cell's conservatives.  Kept: of
+// both cells from LDS.  KeptThenFormed: the left cell's from LDS, the right
+// cell's formed and written to LDS for the next plane.
+template <int DIM, typename R> struct FormedQ {
+  double gamma, b;
+  __device__ __forceinline__ FaceQ<R> left(const double *c) const {
+    return face_quantities<DIM, R>(gamma, b, c);
+  }
+  __device__ __forceinline__ FaceQ<R> right(const double *c) const {
+    return face_quantities<DIM, R>(gamma, b, c);
+  }
+};
+template <int DIM, typename R, int STRIDE> struct KeptQ {
+  const R *l, *r;
+  __device__ __forceinline__ FaceQ<R> left(const double *c) const {
+    return load_packed<DIM, R, STRIDE>(l, c);
+  }
+  __device__ __forceinline__ FaceQ<R> right(const double *c) const {
+    return load_packed<DIM, R, STRIDE>(r, c);
+  }
+};
+template <int DIM, typename R, int STRIDE> struct KeptThenFormedQ {
+  double gamma, b;
+  const R *l;
+  R *r;
+  __device__ __forceinline__ FaceQ<R> left(const double *c) const {
+    return load_packed<DIM, R, STRIDE>(l, c);
+  }
+  __device__ __forceinline__ FaceQ<R> right(const double *c) const {
+    store_packed<DIM, R, STRIDE>(gamma, b, c, r);
+    return load_packed<DIM, R, STRIDE>(r, c);
+  }
+};
 
 // Loads the six-cell stencil around the face (i,j,k)+1/2 along DIR (halo
 // indices of the cell left of the face) and computes its flux.
@@ -950,5 +1392,5 @@ template <int DIM, int DIR, int FLUX, typename R>
 __device__ __forceinline__ void stencil_flux(const double *__restrict__ blk, int i, int j, int k,
                                              double gamma, double b, R *f) {
   using D = Dims<DIM>;
-  face_flux<DIM, DIR, FLUX, R>(gamma, b, blk, i * D::SX + j * D::SY + k, f);
+  face_flux<DIM, DIR, FLUX, R>(gamma, b, blk, i * D::SX + j * D::SY + k, FormedQ<DIM, R>{gamma, b}, f);
 }
