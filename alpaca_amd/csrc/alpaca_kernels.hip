@@ -13,6 +13,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <cstring>
 #include <map>
@@ -685,6 +686,21 @@ struct ProfileScope {
 
 int hip_status(hipError_t e) { return e == hipSuccess ? ALPACA_OK : ALPACA_ERR_HIP; }
 
+// Compute units of the current device (256 where it cannot be asked), looked
+// up once per device.
+int device_cus() {
+  static std::atomic<int> cus[64];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  int n = cus[dev].load(std::memory_order_relaxed);
+  if (n == 0) {
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1)
+      n = 256;
+    cus[dev].store(n, std::memory_order_relaxed);
+  }
+  return n;
+}
+
 // Implicit contexts of the stream-argument entries: one per (device, stream),
 // created on first use and kept until the process ends.
 std::mutex g_ctx_mutex;
@@ -828,8 +844,39 @@ void launch_stage_kernel(dim3 grid, hipStream_t s, const double *avg, const doub
                        s, avg, init, out, state, a);
 }
 
+// The same by plane marching (3D).
+template <int FLUX, int MODE>
+void launch_march_kernel(int nblocks, hipStream_t s, const double *avg, const double *init,
+                         double *out, alpaca_case_state *state, const StageArgs &a) {
+  using R = std::conditional_t<MODE == kModeMixed, float, double>;
+  using M = exact::MarchShape<R>;
+  dim3 const grid(nblocks * M::SLABS), block(M::PLANE);
+  if constexpr (MODE == kModeExact)
+    hipLaunchKernelGGL((exact::march_stage_kernel<FLUX, R>), grid, block, 0, s, avg, init, out,
+                       state, a);
+  else
+    hipLaunchKernelGGL((fast::march_stage_kernel<FLUX, R>), grid, block, 0, s, avg, init, out, state,
+                       a);
+}
+
 // 2D cases with fewer leaf blocks than this run on 8x8 tiles.
 constexpr int kSmallCaseBlocks = 256;
+
+// Whether a 3D case marches (march_stage_kernel) or runs on 8^3 tiles.  Both
+// kernels spend about the same time per unit of 64 faces and wavefront (HLLC
+// FMA 8.2 and 8.3 us, exact 13.6 and 13.5 us at 256^3), a slab taking 26
+// units and a tile 7, and a CU works through the workgroups it is dealt one
+// after the other.  So the case marches where its slabs fill the CUs at least
+// as evenly: 512 blocks 104 units against 112 (exact 1.50 ms a step against
+// 1.54 ms), but 385 blocks 104 against 91 (FMA 0.84 ms against 0.74 ms), and
+// few blocks never (64: 26 against 14).  The mixed HLLC form keeps the tiles.
+template <int FLUX, int MODE>
+constexpr bool kMarches = !(FLUX == ALPACA_FLUX_HLLC && MODE == kModeMixed);
+bool use_march(int nblocks) {
+  long long const cus = device_cus();
+  auto rounds = [cus](long long groups) { return (groups + cus - 1) / cus; };
+  return rounds(2LL * nblocks) * 26 <= rounds(8LL * nblocks) * 7;
+}
 
 // Tile shape of the fused stage kernel: 8x8x8 cells and 256 threads in 3D,
 // the whole 16x16 block and 128 threads in 2D (8x8 and 256 threads for a case
@@ -856,6 +903,12 @@ void launch_stage_fused(const alpaca_case_desc *d, int stage, const double *avg,
   a.init_copy = init_copy;
   ProfileScope prof(ALPACA_KERNEL_STAGE, s, double(Dims<DIM>::CELLS) * nblocks);
   if constexpr (DIM == 3) {
+    if constexpr (kMarches<FLUX, MODE>) {
+      if (use_march(nblocks)) {
+        launch_march_kernel<FLUX, MODE>(nblocks, s, avg, init, out, state, a);
+        return;
+      }
+    }
     constexpr int TX = 8, TY = 8, TZ = 8, NT = 256;
     constexpr int tiles = (kIC / TX) * (kIC / TY) * (kIC / TZ);
     launch_stage_kernel<3, FLUX, MODE, TX, TY, TZ, NT>(dim3(nblocks * tiles), s, avg, init, out,

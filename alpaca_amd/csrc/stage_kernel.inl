@@ -22,61 +22,135 @@ __device__ __forceinline__ double wave_max64(double v) {
   return v;
 }
 
-// Writes the new value v of equation e of internal cell c3 of block blk of the
-// job's case into the halo slabs that read it: the neighbours' slabs across
-// each near face, or the block's own slab on a zero-gradient side (the first
-// or last internal layer fills all four halo layers) or a symmetry side (the
-// cell at internal depth c fills the halo layer at depth c, the face-normal
-// momentum negated).
+// Writes the new values v of internal cell c3 of block blk of the job's case
+// into the halo slabs that read them: the neighbours' slabs across each near
+// face, or the block's own slab on a zero-gradient side (the first or last
+// internal layer fills all four halo layers) or a symmetry side (the cell at
+// internal depth c fills the halo layer at depth c, the face-normal momentum
+// negated).  A workgroup's cells lie in one block, so each destination block is
+// uniform over the wavefront and addressed by a buffer resource; the cell's
+// offset is formed once for all equations.
 template <int DIM>
-__device__ __forceinline__ void push_halo(const TileJob &j, int blk, const int *bc3, const int *c3,
-                                          int e, double v) {
+__device__ __forceinline__ void push_halos(const TileJob &j, int blk, const int *bc3, const int *c3,
+                                           const double *v) {
   using D = Dims<DIM>;
-  double *__restrict__ out = j.out;
+  constexpr int NE = D::NE;
+  int const cell = (c3[0] + kHS) * D::SX + (c3[1] + kHS) * D::SY + (DIM == 3 ? c3[2] + kHS : 0);
+  auto block = [&j](int b) {
+    return BlockReader<DIM>(j.out + (size_t)__builtin_amdgcn_readfirstlane(b) * D::BLOCK);
+  };
 #pragma unroll
   for (int d = 0; d < DIM; ++d) {
+    int const S = d == 0 ? D::SX : (d == 1 ? D::SY : D::SZ);
     int const c = c3[d];
-    int pos[3] = {c3[0] + kHS, c3[1] + kHS, DIM == 3 ? c3[2] + kHS : 0};
-    double const mirrored = (e == kMomX + d) ? -1.0 * v : v;
-    if (c < kHS) {
-      if (bc3[d] > 0 || j.bc[d] == ALPACA_BC_PERIODIC) {
-        int nb3[3] = {bc3[0], bc3[1], bc3[2]};
-        nb3[d] = bc3[d] > 0 ? bc3[d] - 1 : j.nb[d] - 1;
-        int const nbk = j.base + (nb3[0] * j.nb[1] + nb3[1]) * j.nb[2] + nb3[2];
-        pos[d] = c + kHS + kIC;
-        out[(size_t)nbk * D::BLOCK + e * D::FIELD + pos[0] * D::SX + pos[1] * D::SY + pos[2]] = v;
-      } else if (j.bc[d] == ALPACA_BC_SYMMETRY) {
-        pos[d] = kHS - 1 - c;
-        out[(size_t)blk * D::BLOCK + e * D::FIELD + pos[0] * D::SX + pos[1] * D::SY + pos[2]] =
-            mirrored;
-      } else if (c == 0) {
 #pragma unroll
-        for (int h = 0; h < kHS; ++h) {
-          pos[d] = h;
-          out[(size_t)blk * D::BLOCK + e * D::FIELD + pos[0] * D::SX + pos[1] * D::SY + pos[2]] = v;
-        }
-      }
-    }
-    if (c >= kIC - kHS) {
-      if (bc3[d] < j.nb[d] - 1 || j.bc[d] == ALPACA_BC_PERIODIC) {
+    for (int hi = 0; hi < 2; ++hi) {
+      if (hi ? c < kIC - kHS : c >= kHS) continue;
+      bool const edge = hi ? bc3[d] == j.nb[d] - 1 : bc3[d] == 0;
+      if (!edge || j.bc[d] == ALPACA_BC_PERIODIC) {
         int nb3[3] = {bc3[0], bc3[1], bc3[2]};
-        nb3[d] = bc3[d] < j.nb[d] - 1 ? bc3[d] + 1 : 0;
-        int const nbk = j.base + (nb3[0] * j.nb[1] + nb3[1]) * j.nb[2] + nb3[2];
-        pos[d] = c - kIC + kHS;
-        out[(size_t)nbk * D::BLOCK + e * D::FIELD + pos[0] * D::SX + pos[1] * D::SY + pos[2]] = v;
-      } else if (j.bc[d] == ALPACA_BC_SYMMETRY) {
-        pos[d] = kHS + 2 * kIC - 1 - c;
-        out[(size_t)blk * D::BLOCK + e * D::FIELD + pos[0] * D::SX + pos[1] * D::SY + pos[2]] =
-            mirrored;
-      } else if (c == kIC - 1) {
+        nb3[d] = hi ? (edge ? 0 : bc3[d] + 1) : (edge ? j.nb[d] - 1 : bc3[d] - 1);
+        BlockReader<DIM> const w = block(j.base + (nb3[0] * j.nb[1] + nb3[1]) * j.nb[2] + nb3[2]);
+        int const at = cell + (hi ? -kIC : kIC) * S;
 #pragma unroll
-        for (int h = 0; h < kHS; ++h) {
-          pos[d] = kHS + kIC + h;
-          out[(size_t)blk * D::BLOCK + e * D::FIELD + pos[0] * D::SX + pos[1] * D::SY + pos[2]] = v;
-        }
+        for (int e = 0; e < NE; ++e) w.store(v[e], at, e);
+      } else if (j.bc[d] == ALPACA_BC_SYMMETRY) {
+        BlockReader<DIM> const w = block(blk);
+        int const at = cell + ((hi ? 2 * kIC - 1 : -1) - 2 * c) * S;
+#pragma unroll
+        for (int e = 0; e < NE; ++e) w.store(e == kMomX + d ? -1.0 * v[e] : v[e], at, e);
+      } else if (c == (hi ? kIC - 1 : 0)) {
+        BlockReader<DIM> const w = block(blk);
+#pragma unroll
+        for (int h = 1; h <= kHS; ++h)
+#pragma unroll
+          for (int e = 0; e < NE; ++e) w.store(v[e], cell + (hi ? h : -h) * S, e);
       }
     }
   }
+}
+
+// The step of a stage a cell takes: RK coefficients times the time step and
+// the block's place in its grid.
+struct StageStep {
+  double m0, m1, cdt;
+  int bc3[3];
+  __device__ __forceinline__ StageStep(const TileJob &j, int blk_local) {
+    int const stage = j.stage;
+    m0 = stage == 0 ? 1.0 : (stage == 1 ? 0.25 : 2.0 / 3.0);
+    m1 = stage == 0 ? 0.0 : (stage == 1 ? 0.75 : 1.0 / 3.0);
+    double const cs = stage == 0 ? 1.0 : (stage == 1 ? 0.25 : 2.0 / 3.0);
+    cdt = cs * (0.0 + j.state->dt);
+    bc3[0] = blk_local / (j.nb[1] * j.nb[2]);
+    bc3[1] = (blk_local / j.nb[2]) % j.nb[1];
+    bc3[2] = blk_local % j.nb[2];
+  }
+};
+
+// One internal cell c3 of block blk: the divergence of its flux differences
+// (diff gives them per equation), the RK combination, the new value written
+// and pushed into the halos that read it, and on the last stage the cell's
+// CFL signal.
+template <int DIM, typename DIFF>
+__device__ __forceinline__ void stage_cell(const TileJob &j, const StageStep &st, int blk,
+                                           const int *c3, const DIFF &diff, double &sig,
+                                           bool &bad) {
+  using D = Dims<DIM>;
+  constexpr int NE = D::NE;
+  size_t const first = (size_t)__builtin_amdgcn_readfirstlane(blk) * D::BLOCK;
+  BlockReader<DIM> const avg(j.avg + first), out(j.out + first);
+  int const cell = (c3[0] + kHS) * D::SX + (c3[1] + kHS) * D::SY + (DIM == 3 ? c3[2] + kHS : 0);
+  constexpr int B = (int)sizeof(double);
+  double u[NE], ini[NE], v[NE];
+#pragma unroll
+  for (int e = 0; e < NE; ++e) u[e] = avg(cell * B, e * D::FIELD * B);
+  if (j.stage > 0) {
+    BlockReader<DIM> const init(j.init + first);
+#pragma unroll
+    for (int e = 0; e < NE; ++e) ini[e] = init(cell * B, e * D::FIELD * B);
+  } else if (j.init_copy) {
+    BlockReader<DIM> const copy(j.init_copy + first);
+#pragma unroll
+    for (int e = 0; e < NE; ++e) copy.store(u[e], cell, e);
+  }
+#pragma unroll
+  for (int e = 0; e < NE; ++e) {
+    double dX, dY, dZ = 0.0;
+    diff(e, dX, dY, dZ);
+    double const rhs = 0.0 + (0.0 + dams<DIM>(dX, dY, dZ) * j.inv_dx);
+    double const base = j.stage == 0 ? u[e] : st.m0 * u[e] + st.m1 * ini[e];
+    v[e] = base + st.cdt * rhs;
+    bad |= !__builtin_isfinite(v[e]);
+  }
+#pragma unroll
+  for (int e = 0; e < NE; ++e) out.store(v[e], cell, e);
+  push_halos<DIM>(j, blk, st.bc3, c3, v);
+  if (j.signal) {
+    // The CFL signal is FP64 without contraction in every mode, so a step's
+    // dt does not depend on which kernel reduced the signal.
+    exact::Prim<double> p;
+    exact::cons_to_prim<DIM>(j.gamma, j.b, v, p);
+    double const cso = exact::eos_sos(j.gamma, j.b, p.rho, p.p);
+    double sum;
+    if constexpr (DIM == 2)
+      sum = (__builtin_fabs(p.vel[0]) + cso) + (__builtin_fabs(p.vel[1]) + cso);
+    else
+      sum = exact::cms3(__builtin_fabs(p.vel[0]) + cso, __builtin_fabs(p.vel[1]) + cso,
+                        __builtin_fabs(p.vel[2]) + cso);
+    sig = smax(sig, sum);
+  }
+}
+
+// After a workgroup's cells: the CFL signal into the case record, the
+// non-finite flag.
+__device__ __forceinline__ void stage_finish(const TileJob &j, double sig, bool bad) {
+  if (j.signal) {
+    sig = wave_max64(sig);
+    if ((threadIdx.x & 63) == 0)
+      atomicMax(reinterpret_cast<unsigned long long *>(&j.state->smax),
+                (unsigned long long)__double_as_longlong(sig));
+  }
+  if (bad) atomicOr(&j.state->flags, kFlagNonFinite);
 }
 
 template <int DIM, int TX, int TY, int TZ> struct TileShape {
@@ -98,8 +172,8 @@ template <int DIM, int TX, int TY, int TZ> struct TileShape {
 // ([6][NE][IC][ICZ]: East, West, North, South, Top, Bottom; the boundary-flux
 // save of SpaceSolver::UpdateFluxes, space_solver.cpp:160-182).
 template <int DIM, int FLUX, typename R, int TX, int TY, int TZ, int NT, bool JUMP>
-__device__ __forceinline__ void tile_faces(const double *__restrict__ bb, int x0, int y0, int z0,
-                                           double gamma, double b, R *lds, double *jump) {
+__device__ __forceinline__ void tile_faces(int tid, const double *__restrict__ bb, int x0, int y0,
+                                           int z0, double gamma, double b, R *lds, double *jump) {
   using D = Dims<DIM>;
   using T = TileShape<DIM, TX, TY, TZ>;
   constexpr int NE = D::NE;
@@ -116,7 +190,7 @@ __device__ __forceinline__ void tile_faces(const double *__restrict__ bb, int x0
 #pragma unroll
     for (int e = 0; e < NE; ++e) jump[((loc * NE + e) * kIC + a) * ICZ + c] += double(fl[e]);
   };
-  for (int f = threadIdx.x; f < PX + PY + PZ; f += NT) {
+  for (int f = tid; f < PX + PY + PZ; f += NT) {
     R fl[NE];
     if (f < PX) {
       if (f < NFX) {
@@ -165,8 +239,10 @@ __device__ __forceinline__ void tile_faces(const double *__restrict__ bb, int x0
 // One tile of one block: faces into LDS, barrier, divergence + RK + halo
 // push (+ CFL signal).  blk_local is the block's index within its case.
 // All threads of the workgroup must call it (it contains a barrier).
+// tid is the thread's index in the workgroup.
 template <int DIM, int FLUX, typename R, int TX, int TY, int TZ, int NT>
-__device__ __forceinline__ void stage_tile(const TileJob &j, int blk_local, int tile, R *lds) {
+__device__ __forceinline__ void stage_tile(int tid, const TileJob &j, int blk_local, int tile,
+                                           R *lds) {
   using D = Dims<DIM>;
   using T = TileShape<DIM, TX, TY, TZ>;
   constexpr int NE = D::NE;
@@ -182,68 +258,250 @@ __device__ __forceinline__ void stage_tile(const TileJob &j, int blk_local, int 
   const double *bb = j.avg + (size_t)blk * D::BLOCK;
 
   // 1. Face fluxes of the tile into LDS.
-  tile_faces<DIM, FLUX, R, TX, TY, TZ, NT, false>(bb, x0, y0, z0, j.gamma, j.b, lds, nullptr);
+  tile_faces<DIM, FLUX, R, TX, TY, TZ, NT, false>(tid, bb, x0, y0, z0, j.gamma, j.b, lds, nullptr);
   __syncthreads();
 
   // 2. Divergence + RK combination + halo push (+ CFL signal).
-  double const dt = j.state->dt;
-  int const stage = j.stage;
-  double const m0 = stage == 0 ? 1.0 : (stage == 1 ? 0.25 : 2.0 / 3.0);
-  double const m1 = stage == 0 ? 0.0 : (stage == 1 ? 0.75 : 1.0 / 3.0);
-  double const cs = stage == 0 ? 1.0 : (stage == 1 ? 0.25 : 2.0 / 3.0);
-  double const cdt = cs * (0.0 + dt);
-  int const bc3[3] = {blk_local / (j.nb[1] * j.nb[2]), (blk_local / j.nb[2]) % j.nb[1],
-                      blk_local % j.nb[2]};
+  StageStep const st(j, blk_local);
   double sig = 0.0;
   bool bad = false;
-  for (int c = threadIdx.x; c < T::CELLS; c += NT) {
+  for (int c = tid; c < T::CELLS; c += NT) {
     int const kk = c % TZe, jj = (c / TZe) % TY, ii = c / (TZe * TY);
     int const c3[3] = {x0 + ii, y0 + jj, z0 + kk};
-    size_t const cell = (size_t)blk * D::BLOCK + (c3[0] + kHS) * D::SX + (c3[1] + kHS) * D::SY +
-                        (DIM == 3 ? c3[2] + kHS : 0);
-    double v[NE];
-#pragma unroll
-    for (int e = 0; e < NE; ++e) {
-      double const dX = double(FX[e * NFX + (ii * TY + jj) * TZe + kk]) -
-                        double(FX[e * NFX + ((ii + 1) * TY + jj) * TZe + kk]);
-      double const dY = double(FY[e * NFY + (ii * (TY + 1) + jj) * TZe + kk]) -
-                        double(FY[e * NFY + (ii * (TY + 1) + jj + 1) * TZe + kk]);
-      double dZ = 0.0;
+    auto diff = [&](int e, double &dX, double &dY, double &dZ) {
+      dX = double(FX[e * NFX + (ii * TY + jj) * TZe + kk]) -
+           double(FX[e * NFX + ((ii + 1) * TY + jj) * TZe + kk]);
+      dY = double(FY[e * NFY + (ii * (TY + 1) + jj) * TZe + kk]) -
+           double(FY[e * NFY + (ii * (TY + 1) + jj + 1) * TZe + kk]);
       if constexpr (DIM == 3)
         dZ = double(FZ[e * NFZ + (ii * TY + jj) * (TZ + 1) + kk]) -
              double(FZ[e * NFZ + (ii * TY + jj) * (TZ + 1) + kk + 1]);
-      double const rhs = 0.0 + (0.0 + dams<DIM>(dX, dY, dZ) * j.inv_dx);
-      size_t const idx = cell + (size_t)e * D::FIELD;
-      double const u = j.avg[idx];
-      if (stage == 0 && j.init_copy) j.init_copy[idx] = u;
-      double const base = stage == 0 ? u : m0 * u + m1 * j.init[idx];
-      v[e] = base + cdt * rhs;
-      j.out[idx] = v[e];
-      bad |= !__builtin_isfinite(v[e]);
-      push_halo<DIM>(j, blk, bc3, c3, e, v[e]);
-    }
-    if (j.signal) {
-      // The CFL signal is FP64 without contraction in every mode, so a step's
-      // dt does not depend on which kernel reduced the signal.
-      exact::Prim<double> p;
-      exact::cons_to_prim<DIM>(j.gamma, j.b, v, p);
-      double const cso = exact::eos_sos(j.gamma, j.b, p.rho, p.p);
-      double sum;
-      if constexpr (DIM == 2)
-        sum = (__builtin_fabs(p.vel[0]) + cso) + (__builtin_fabs(p.vel[1]) + cso);
-      else
-        sum = exact::cms3(__builtin_fabs(p.vel[0]) + cso, __builtin_fabs(p.vel[1]) + cso,
-                          __builtin_fabs(p.vel[2]) + cso);
-      sig = smax(sig, sum);
-    }
+    };
+    stage_cell<DIM>(j, st, blk, c3, diff, sig, bad);
   }
-  if (j.signal) {
-    sig = wave_max64(sig);
-    if ((threadIdx.x & 63) == 0)
-      atomicMax(reinterpret_cast<unsigned long long *>(&j.state->smax),
-                (unsigned long long)__double_as_longlong(sig));
+  stage_finish(j, sig, bad);
+}
+
+// ------------------------------------------------------- plane marching ---
+// 3D, large cases: one workgroup of 256 threads per slab of SX = 8 planes of a
+// block, thread (j, k) owning the column of cells (x0 .. x0+7, j, k).  Plane
+// by plane each thread computes the low y face, the low z face and the high x
+// face of its cell; the x flux stays in registers as the next plane's low
+// one, the y and z fluxes of the plane go through LDS.  The faces that close
+// the slab at j = 16 and k = 16 (8 planes x 16 each: two whole waves per
+// direction) are computed before the first plane, by the same code: p = -1
+// runs the y body in waves 0 and 1, the z body in waves 2 and 3, and the x
+// body on the slab's first face.  So every wave computes 26 units of 64 faces
+// for 24 units of cells (8.3% more faces than cells; 8^3 tiles compute 12.5%
+// more in 27 units over 4 waves), and the values the Roe average takes from a
+// cell are formed once per cell (1.5 times, with the slab's rim) instead of
+// six to seven times.
+//
+// LDS, in units of 256 values of R: Q (NQ per buffer, two buffers: the plane's
+// packed cell quantities, the next plane's written by the x faces), HQ (NQ:
+// those of the halo cells at j = -1 and k = -1, all planes), FZ, EX (the closing
+// fluxes) and two buffers of FY (NE each): 70 KB in FP64, two workgroups per
+// CU as the registers allow.  Before plane 0 the two Q buffers hold the
+// quantities of the cells left and right of the closing faces.
+//
+// Bound by FP64 issue with a share of L2 misses.  256^3, one step, against the
+// 8^3 tiles with the same face arithmetic: HLLC exact 12.06 -> 11.30 ms, FMA
+// 7.46 -> 6.82 ms; Roe exact 22.0 -> 21.4 ms, FMA 11.8 -> 11.0 ms, mixed 9.34 ->
+// 8.82 ms.  The mixed HLLC form gains nothing (7.0 ms both ways: it runs 3
+// waves per SIMD either way and pays the barrier) and keeps the tiles.  A
+// wavefront marching an 8^3 tile by itself, without barriers, was slower
+// (HLLC exact 13.3 ms, FMA 9.96 ms): its waves drift apart and their planes
+// no longer share the caches (1.3e8 L2 misses a launch).
+template <typename R> struct MarchShape {
+  static constexpr int SX = 8;
+  static constexpr int SLABS = kIC / SX;
+  static constexpr int PLANE = kIC * kIC;  // cells of a plane = threads
+  static constexpr int NQ = PackedQ<R>::NQ;
+  static constexpr int NE = 5;
+  static constexpr int LDS = (3 * NQ + 4 * NE) * PLANE;
+  static_assert(SX * 2 * kIC == PLANE, "one halo cell and one closing face per thread");
+};
+
+// Barrier of the workgroup that orders LDS accesses only: outstanding global
+// stores are not waited for (no thread reads what another one stored).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// Makes `off` available only once a and b are formed.
+template <typename R> __device__ __forceinline__ void after(int &off, R a, R b) {
+  asm volatile("" : "+v"(off) : "v"(a), "v"(b));
+}
+
+template <int FLUX, typename R>
+__device__ __forceinline__ void stage_march(const TileJob &j, int blk_local, int slab, R *lds) {
+  using D = Dims<3>;
+  using M = MarchShape<R>;
+  constexpr int NE = M::NE, P = M::PLANE, SX = M::SX, NQ = M::NQ;
+  int const tid = threadIdx.x;
+  int const wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  int const x0 = slab * SX;
+  int const blk = j.base + blk_local;
+  const double *bb = j.avg + (size_t)blk * D::BLOCK;
+  BlockReader<3> const rd(bb);
+  R *Q = lds, *HQ = lds + 2 * NQ * P, *FZ = HQ + NQ * P, *EX = FZ + NE * P, *FY2 = EX + NE * P;
+  // Packed quantities of the cell at halo offset `off` into q.
+  auto keep = [&](int off, R *q) {
+    double c[NE];
+#pragma unroll
+    for (int e = 0; e < NE; ++e) c[e] = rd(off * (int)sizeof(double), e * D::FIELD * (int)sizeof(double));
+    store_packed<3, R, P>(j.gamma, j.b, c, q);
+  };
+  // Halo offset of thread t's cell in plane p, and of the cell left of its
+  // closing face (threads 0-127 the y side, 128-255 the z side; plane
+  // (t >> 4) & 7, position t & 15 along the other axis).
+  auto here = [x0](int t, int p) {
+    return (x0 + p + kHS) * D::SX + (t / kIC + kHS) * D::SY + t % kIC + kHS;
+  };
+  auto closing = [x0](int t, bool zside) {
+    int const row = (x0 + ((t >> 4) & 7) + kHS) * D::SX;
+    return zside ? row + ((t & 15) + kHS) * D::SY + kHS + kIC - 1
+                 : row + (kHS + kIC - 1) * D::SY + (t & 15) + kHS;
+  };
+  // Quantities left and right of the closing faces (t = 0, 1) and of the rim
+  // cells at j = -1 and k = -1 (t = 2).
+#pragma unroll 1
+  for (int t = 0; t < 3; ++t) {
+    bool const zside = tid >= P / 2;
+    int const step = zside ? 1 : D::SY;
+    keep(closing(tid, zside) + (t == 2 ? -kIC : t) * step, Q + t * NQ * P + tid);
   }
-  if (bad) atomicOr(&j.state->flags, kFlagNonFinite);
+  __syncthreads();
+  StageStep const st(j, blk_local);
+  double sig = 0.0;
+  bool bad = false;
+  R fx[NE];
+#pragma unroll
+  for (int e = 0; e < NE; ++e) fx[e] = R(0.0);
+  // FV: the stencil of the next face is read while this face's Riemann problem
+  // is solved, whose registers leave room for it.
+  constexpr bool AHEAD = FLUX == 0;
+  // The contracted FP64 form also keeps the column's cells p-2 .. p+2 in
+  // registers for the x faces (203 VGPRs).  Reading them again for each of the
+  // six faces that use a cell misses the XCD's 4 MB L2, which the 64 slabs in
+  // flight fill (256^3: 9.4e7 L2 misses a launch against 3.8e7 for tiles; the
+  // step takes 7.27 ms with the reads and 6.82 ms with the column).  The exact
+  // form has no registers for it (111 spilled: 13.8 ms instead of 12.0).
+  constexpr bool COLUMN = AHEAD && kLean<R>;
+  double U[6][NE], X[6][NE];
+  int p = -1;
+  if constexpr (AHEAD) load_stencil<3>(rd, closing(tid, false), D::SY, U);
+  if constexpr (COLUMN) load_stencil<3>(rd, here(tid, p), D::SX, X);
+#pragma unroll 1
+  for (; p < SX; ++p) {
+    // The thread's indices pass through empty asm statements, so that no
+    // address is formed ahead of the loop and held in registers through it
+    // (and the first pass stays in the loop: one copy of each face body).
+    asm volatile("" : "+s"(p));
+    bool const inner = p >= 0;
+    R *FY = FY2 + (p & 1) * NE * P;
+    if (inner || wave < 2) {
+      int t = tid;
+      asm volatile("" : "+v"(t));
+      int const yj = t / kIC, yk = t % kIC;
+      const R *q = Q + (p & 1) * NQ * P;
+      R fl[NE];
+      KeptQ<3, R, P> const qs{inner ? (yj > 0 ? q + t - kIC : HQ + p * kIC + yk) : Q + t,
+                              inner ? q + t : Q + NQ * P + t};
+      if constexpr (AHEAD) {
+        R cl[NE], cr[NE];
+        fv_reconstruct<3, 1, R>(j.gamma, U, qs, cl, cr);
+        int off = here(t, p) - 1;
+        after(off, cl[NE - 1], cr[NE - 1]);
+        load_stencil<3>(rd, off, 1, U);
+        fv_riemann<3, 1, R>(j.gamma, j.b, cl, cr, fl);
+      } else {
+        int const off = inner ? here(t, p) - D::SY : closing(t, false);
+        face_flux<3, 1, FLUX, R>(j.gamma, j.b, bb, off, qs, fl);
+      }
+      R *o = (inner ? FY : EX) + t;
+#pragma unroll
+      for (int e = 0; e < NE; ++e) o[e * P] = fl[e];
+    }
+    if (inner || wave >= 2) {
+      int t = tid;
+      asm volatile("" : "+v"(t));
+      int const zj = t / kIC, zk = t % kIC;
+      const R *q = Q + (p & 1) * NQ * P;
+      R fl[NE];
+      KeptQ<3, R, P> const qs{inner ? (zk > 0 ? q + t - 1 : HQ + P / 2 + p * kIC + zj) : Q + t,
+                              inner ? q + t : Q + NQ * P + t};
+      if constexpr (AHEAD) {
+        if (!inner) load_stencil<3>(rd, closing(t, true), 1, U);
+        R cl[NE], cr[NE];
+        fv_reconstruct<3, 2, R>(j.gamma, U, qs, cl, cr);
+        int off = here(t, p);
+        after(off, cl[NE - 1], cr[NE - 1]);
+        if constexpr (COLUMN)
+          load_cell<3>(rd, off + 3 * D::SX, X[5]);
+        else
+          load_stencil<3>(rd, off, D::SX, U);
+        fv_riemann<3, 2, R>(j.gamma, j.b, cl, cr, fl);
+      } else {
+        int const off = inner ? here(t, p) - 1 : closing(t, true);
+        face_flux<3, 2, FLUX, R>(j.gamma, j.b, bb, off, qs, fl);
+      }
+      R *o = (inner ? FZ : EX) + t;
+#pragma unroll
+      for (int e = 0; e < NE; ++e) o[e * P] = fl[e];
+    }
+    R fh[NE];
+    {
+      int t = tid;
+      asm volatile("" : "+v"(t));
+      if (!inner) {
+        lds_barrier();  // the closing faces have read both Q buffers
+        keep(here(t, p), Q + NQ * P + t);
+        if constexpr (AHEAD && !COLUMN) load_stencil<3>(rd, here(t, p), D::SX, U);
+      }
+      KeptThenFormedQ<3, R, P> const qs{j.gamma, j.b, Q + (p & 1) * NQ * P + t,
+                                        Q + ((p + 1) & 1) * NQ * P + t};
+      if constexpr (AHEAD) {
+        R cl[NE], cr[NE];
+        fv_reconstruct<3, 0, R>(j.gamma, COLUMN ? X : U, qs, cl, cr);
+        if constexpr (COLUMN) {
+#pragma unroll
+          for (int m = 0; m < 5; ++m)
+#pragma unroll
+            for (int e = 0; e < NE; ++e) X[m][e] = X[m + 1][e];
+        }
+        int off = here(t, p) + D::SX - D::SY;
+        after(off, cl[NE - 1], cr[NE - 1]);
+        load_stencil<3>(rd, off, D::SY, U);
+        fv_riemann<3, 0, R>(j.gamma, j.b, cl, cr, fh);
+      } else {
+        face_flux<3, 0, FLUX, R>(j.gamma, j.b, bb, here(t, p), qs, fh);
+      }
+    }
+    // The plane's y fluxes and the next plane's quantities.  The z fluxes pass
+    // between lanes of one wave, and the y fluxes have two buffers, so one
+    // barrier per plane is enough.
+    lds_barrier();
+    if (inner) {
+      int t = tid;
+      asm volatile("" : "+v"(t));
+      int const cj = t / kIC, ck = t % kIC;
+      int const c3[3] = {x0 + p, cj, ck};
+      const R *yh = cj < kIC - 1 ? FY + t + kIC : EX + p * kIC + ck;
+      const R *zh = ck < kIC - 1 ? FZ + t + 1 : EX + P / 2 + p * kIC + cj;
+      auto diff = [&](int e, double &dX, double &dY, double &dZ) {
+        dX = double(fx[e]) - double(fh[e]);
+        dY = double(FY[e * P + t]) - double(yh[e * P]);
+        dZ = double(FZ[e * P + t]) - double(zh[e * P]);
+      };
+      stage_cell<3>(j, st, blk, c3, diff, sig, bad);
+    }
+#pragma unroll
+    for (int e = 0; e < NE; ++e) fx[e] = fh[e];
+  }
+  stage_finish(j, sig, bad);
 }
 
 // Waves per SIMD the register allocator is held to in the single-case
@@ -256,23 +514,13 @@ template <int DIM, int FLUX, typename R>
 constexpr int kMinWaves = (DIM == 2 && FLUX == 0 && !kFastArith && std::is_same<R, double>::value) ? 3
                           : (FLUX == 1 && !kFastArith && std::is_same<R, double>::value) ? 2 : 1;
 
-// The persistent batch kernel holds only the exact flux-splitting variant (to
-// 2 waves per SIMD, which its field-by-field face allows).
-template <int FLUX, typename R>
-constexpr int kBatchMinWaves = (FLUX == 1 && !kFastArith && std::is_same<R, double>::value) ? 2 : 1;
+// The persistent batch kernel: as above.
+template <int DIM, int FLUX, typename R>
+constexpr int kBatchMinWaves = kMinWaves<DIM, FLUX, R>;
 
-// Single case: one workgroup per (block, tile).
-template <int DIM, int FLUX, typename R, int TX, int TY, int TZ, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kMinWaves<DIM, FLUX, R>, 8))) void stage_kernel(const double *__restrict__ avg,
-                                                   const double *init, double *out,
-                                                   alpaca_case_state *state, StageArgs a) {
-  using T = TileShape<DIM, TX, TY, TZ>;
-  static_assert(NT % 64 == 0, "whole wavefronts");
-  __shared__ R lds[T::LDS];
-  unsigned const g = xcd_remap_group(blockIdx.x, gridDim.x);
-  int const blk = g / T::TILES;
-  if (blk >= a.nblocks) return;  // uniform over the workgroup
-  if (a.guard && (state->flags & kFlagDone)) return;
+// The job of a single case's stage.
+__device__ __forceinline__ TileJob stage_job(const double *avg, const double *init, double *out,
+                                             alpaca_case_state *state, const StageArgs &a) {
   TileJob j;
   j.avg = avg;
   j.init = init;
@@ -290,7 +538,38 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kMinWaves<DI
   j.inv_dx = a.inv_dx;
   j.stage = a.stage;
   j.signal = a.signal;
-  stage_tile<DIM, FLUX, R, TX, TY, TZ, NT>(j, blk, g % T::TILES, lds);
+  return j;
+}
+
+// Single case: one workgroup per (block, tile).
+template <int DIM, int FLUX, typename R, int TX, int TY, int TZ, int NT>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kMinWaves<DIM, FLUX, R>, 8))) void stage_kernel(const double *__restrict__ avg,
+                                                   const double *init, double *out,
+                                                   alpaca_case_state *state, StageArgs a) {
+  using T = TileShape<DIM, TX, TY, TZ>;
+  static_assert(NT % 64 == 0, "whole wavefronts");
+  __shared__ R lds[T::LDS];
+  unsigned const g = xcd_remap_group(blockIdx.x, gridDim.x);
+  int const blk = g / T::TILES;
+  if (blk >= a.nblocks) return;  // uniform over the workgroup
+  if (a.guard && (state->flags & kFlagDone)) return;
+  TileJob const j = stage_job(avg, init, out, state, a);
+  stage_tile<DIM, FLUX, R, TX, TY, TZ, NT>(threadIdx.x, j, blk, g % T::TILES, lds);
+}
+
+// Single 3D case by plane marching: one workgroup per (block, slab).
+template <int FLUX, typename R>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMinWaves<3, FLUX, R>, 8))) void march_stage_kernel(
+    const double *__restrict__ avg, const double *init, double *out, alpaca_case_state *state,
+    StageArgs a) {
+  constexpr unsigned SLABS = MarchShape<R>::SLABS;
+  __shared__ R lds[MarchShape<R>::LDS];
+  unsigned const g = xcd_remap_group(blockIdx.x, gridDim.x);
+  int const blk = g / SLABS;
+  if (blk >= a.nblocks) return;  // uniform over the workgroup
+  if (a.guard && (state->flags & kFlagDone)) return;
+  TileJob const j = stage_job(avg, init, out, state, a);
+  stage_march<FLUX, R>(j, blk, g % SLABS, lds);
 }
 
 // Right-hand side of listed blocks of a pool (SpaceSolver::UpdateFluxes in
@@ -324,7 +603,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kMinWaves<DI
   int const y0 = ((tile / NTZ) % NTY) * TY;
   int const x0 = (tile / (NTZ * NTY)) * TX;
   double *jb = jump + (size_t)blk * SURF;
-  tile_faces<DIM, FLUX, R, TX, TY, TZ, NT, true>(avg + (size_t)blk * D::BLOCK, x0, y0, z0, gamma,
+  tile_faces<DIM, FLUX, R, TX, TY, TZ, NT, true>(threadIdx.x, avg + (size_t)blk * D::BLOCK, x0, y0, z0, gamma,
                                                  b, lds, jb);
   if constexpr (DIM == 2) {
     for (int t = threadIdx.x; t < 2 * NE * kIC; t += NT) jb[4 * NE * kIC + t] += 0.0;
@@ -366,6 +645,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kMinWaves<DI
   }
 }
 
+// A value that is the same in every lane, in scalar registers.
+__device__ __forceinline__ int in_sgpr(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ double in_sgpr(double v) {
+  long long const b = __double_as_longlong(v);
+  unsigned const lo = __builtin_amdgcn_readfirstlane((int)b);
+  unsigned const hi = __builtin_amdgcn_readfirstlane((int)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
 // Every tile of every listed block of every case of an ensemble, one
 // persistent kernel per RK stage: the grid is sized to the device and each
 // workgroup walks the work list (read from device memory, so a captured
@@ -373,7 +661,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kMinWaves<DI
 // split into 8 contiguous ranges, one per XCD (group g runs on XCD g % 8),
 // so a case's blocks share an L2.  Units of stopped cases are skipped.
 template <int DIM, int FLUX, typename R, int TX, int TY, int TZ, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kBatchMinWaves<FLUX, R>, 8))) void batch_stage_kernel(
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kBatchMinWaves<DIM, FLUX, R>, 8))) void batch_stage_kernel(
     const double *__restrict__ avg, const double *init, double *out, const CaseSlot *slots,
     alpaca_case_state *states, const WorkItem *items, const int *n_items, int stage) {
   using T = TileShape<DIM, TX, TY, TZ>;
@@ -395,7 +683,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kBatchMinWav
   unsigned const units_here = items_here * T::TILES;
   for (unsigned w = m; w < units_here; w += per_xcd) {
     unsigned const u = (xcd + kXcd * (w / T::TILES)) * T::TILES + w % T::TILES;
-    WorkItem const it = items[u / T::TILES];
+    WorkItem it = items[u / T::TILES];
+    it.case_id = in_sgpr(it.case_id);
+    it.block = in_sgpr(it.block);
     alpaca_case_state *st = states + it.case_id;
     // Another workgroup may flag the case during this stage: decide once per
     // workgroup so every thread takes the same branch around the barriers.
@@ -411,18 +701,22 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kBatchMinWav
     j.out = out;
     j.state = st;
     j.init_copy = nullptr;
-    j.base = cs.base;
+    j.base = in_sgpr(cs.base);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      j.nb[d] = cs.nb[d];
-      j.bc[d] = cs.bc[d];
+      j.nb[d] = in_sgpr(cs.nb[d]);
+      j.bc[d] = in_sgpr(cs.bc[d]);
     }
-    j.gamma = cs.gamma;
-    j.b = cs.b;
-    j.inv_dx = cs.inv_dx;
+    j.gamma = in_sgpr(cs.gamma);
+    j.b = in_sgpr(cs.b);
+    j.inv_dx = in_sgpr(cs.inv_dx);
     j.stage = stage;
     j.signal = stage == 2;
-    stage_tile<DIM, FLUX, R, TX, TY, TZ, NT>(j, it.block, u % T::TILES, lds);
+    // Through an empty asm statement, so that nothing that follows from the
+    // thread's index is formed ahead of the loop and held through it.
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    stage_tile<DIM, FLUX, R, TX, TY, TZ, NT>(tid, j, it.block, u % T::TILES, lds);
     __syncthreads();  // LDS is reused by the next unit
   }
 }
