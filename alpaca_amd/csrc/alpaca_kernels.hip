@@ -5,9 +5,9 @@
 //   face_flux_kernel<DIM,DIR,FLUX,R>  one thread per cell face; six-cell
 //       stencil read straight from the haloed block (coalesced along k);
 //       Roe eigensystem + characteristic WENO5 + HLLC or Roe splitting.
-//   combine_kernel<DIM>  one thread per internal cell: flux divergence with
-//       the reference's ConsistencyManagedSum, times 1/dx, fused with the
-//       SSP-RK3 combination and the non-finite check.
+//       Only the per-block convective-flux entry writes face fluxes out.
+//   stage_kernel, march_stage_kernel (stage_kernel.inl)  a whole RK stage:
+//       faces, flux divergence, RK combination, halos.
 //   halo_kernel<DIM>  face halo slabs from neighbours / zero-gradient / symmetry.
 //   signal_kernel<DIM> + dt_kernel  CFL reduction and time step.
 #include <hip/hip_runtime.h>
@@ -22,6 +22,7 @@
 
 #include "../../include/alpaca_gpu.h"
 #include "fv_device.h"
+#include "launch_shapes.h"
 
 // Opaque context of the per-block entries (include/alpaca_gpu.h): the HIP
 // stream its calls are queued on and the face-flux scratch they use, so
@@ -116,124 +117,6 @@ __global__ __launch_bounds__(kThreads) void face_flux_kernel(const double *__res
   double *o = flux_out + ((size_t)blk * DIM + DIR) * NE * NF + f;
 #pragma unroll
   for (int e = 0; e < NE; ++e) o[e * NF] = fl[e];
-}
-
-// ------------------------------------------------------- jump fluxes ---
-// The boundary-flux save of SpaceSolver::UpdateFluxes (space_solver.cpp:
-// 160-182): the fluxes of a block's six boundary faces ADDED into its jump
-// surfaces [6][NE][IC][ICZ] (SurfaceBuffer: East, West, North, South, Top,
-// Bottom).  One thread per surface entry; in 2D the z faces do not exist and
-// Bottom/Top receive += 0.0, as from the reference's zeroed z face array.
-template <int DIM>
-__global__ __launch_bounds__(kThreads) void jump_flux_kernel(const double *__restrict__ flux,
-                                                             double *__restrict__ jump,
-                                                             int nblocks) {
-  using D = Dims<DIM>;
-  constexpr int NE = D::NE;
-  constexpr int NF = faces_per_dir<DIM>();
-  constexpr int ICZ = D::ICZ;
-  constexpr int FACE = NE * kIC * ICZ;
-  size_t const t = (size_t)blockIdx.x * kThreads + threadIdx.x;
-  if (t >= (size_t)nblocks * 6 * FACE) return;
-  int const blk = int(t / (6 * FACE));
-  int const loc = int((t / FACE) % 6);
-  int const r = int(t % FACE);
-  int const e = r / (kIC * ICZ), i = (r / ICZ) % kIC, j = r % ICZ;
-  const double *fx = flux + ((size_t)blk * DIM + 0) * NE * NF + (size_t)e * NF;
-  const double *fy = flux + ((size_t)blk * DIM + 1) * NE * NF + (size_t)e * NF;
-  double v = 0.0;
-  switch (loc) {
-    case 0: v = fx[(kIC * kIC + i) * ICZ + j]; break;        // East: x face IC
-    case 1: v = fx[i * ICZ + j]; break;                        // West: x face 0
-    case 2: v = fy[(i * (kIC + 1) + kIC) * ICZ + j]; break;  // North: y face IC
-    case 3: v = fy[(i * (kIC + 1)) * ICZ + j]; break;          // South: y face 0
-    default:
-      if constexpr (DIM == 3) {
-        const double *fz = flux + ((size_t)blk * DIM + 2) * NE * NF + (size_t)e * NF;
-        v = fz[(i * kIC + j) * (kIC + 1) + (loc == 4 ? kIC : 0)];  // Top / Bottom
-      }
-  }
-  jump[t] += v;
-}
-
-// ------------------------------------------------------------- combine ---
-struct StageCoef {
-  double m0, m1, c;
-};
-__host__ __device__ inline StageCoef stage_coef(int stage) {
-  // RungeKutta3TVD buffer and time-step multipliers (runge_kutta_3_TVD.h:39-59).
-  if (stage == 0) return {1.0, 0.0, 1.0};
-  if (stage == 1) return {0.25, 0.75, 0.25};
-  return {2.0 / 3.0, 1.0 / 3.0, 2.0 / 3.0};
-}
-
-// Flux divergence (space_solver.cpp:131-153) fused with PrepareBufferFor-
-// Integration and IntegrateConservatives (time_integrator.h:98-113, 434-457).
-// MODE 0: RK stage; MODE 1: write the right-hand side itself.
-template <int DIM, int MODE>
-__global__ __launch_bounds__(kThreads) void combine_kernel(
-    const double *__restrict__ flux, const double *__restrict__ avg, const double *init,
-    double *out, int nblocks, int stage, double inv_dx, alpaca_case_state *state) {
-  using D = Dims<DIM>;
-  constexpr int NE = D::NE;
-  constexpr int NF = faces_per_dir<DIM>();
-  constexpr int ICZ = D::ICZ;
-  constexpr int cells = D::CELLS;
-  constexpr int groups_per_block = (cells + kThreads - 1) / kThreads;
-  unsigned const g = xcd_remap_group(blockIdx.x, gridDim.x);
-  int const blk = g / groups_per_block;
-  int const c = (g % groups_per_block) * kThreads + threadIdx.x;
-  if (blk >= nblocks || c >= cells) return;
-  int const kk = c % ICZ;
-  int const jj = (c / ICZ) % kIC;
-  int const ii = c / (ICZ * kIC);
-  const double *fx = flux + ((size_t)blk * DIM + 0) * NE * NF;
-  const double *fy = flux + ((size_t)blk * DIM + 1) * NE * NF;
-  const double *fz = DIM == 3 ? flux + ((size_t)blk * DIM + 2) * NE * NF : nullptr;
-  // Face a along a direction lies between internal cells a-1 and a.
-  int const x_lo = (ii * kIC + jj) * ICZ + kk;           // fx [17][16][16|1]
-  int const x_hi = ((ii + 1) * kIC + jj) * ICZ + kk;
-  int const y_lo = (ii * (kIC + 1) + jj) * ICZ + kk;     // fy [16][17][16|1]
-  int const y_hi = (ii * (kIC + 1) + jj + 1) * ICZ + kk;
-  int const z_lo = (ii * kIC + jj) * (kIC + 1) + kk;     // fz [16][16][17]
-  int const z_hi = z_lo + 1;
-  size_t const cell = (size_t)blk * D::BLOCK + (ii + kHS) * D::SX + (jj + kHS) * D::SY +
-                      (DIM == 3 ? kk + kHS : 0);
-  double dt = 0.0;
-  StageCoef co{1.0, 0.0, 1.0};
-  if constexpr (MODE == 0) {
-    dt = state->dt;
-    co = stage_coef(stage);
-  }
-  double const timestep = 0.0 + dt;
-  double const cdt = co.c * timestep;
-  bool bad = false;
-#pragma unroll
-  for (int e = 0; e < NE; ++e) {
-    double const dx_ = fx[e * NF + x_lo] - fx[e * NF + x_hi];
-    double const dy_ = fy[e * NF + y_lo] - fy[e * NF + y_hi];
-    double dz_ = 0.0;
-    if constexpr (DIM == 3) dz_ = fz[e * NF + z_lo] - fz[e * NF + z_hi];
-    double const rhs = 0.0 + (0.0 + exact::dams<DIM>(dx_, dy_, dz_) * inv_dx);
-    size_t const idx = cell + (size_t)e * D::FIELD;
-    if constexpr (MODE == 0) {
-      double const u = avg[idx];
-      double a = u;
-      if (stage == 0) {
-        if (init) const_cast<double *>(init)[idx] = u;
-      } else {
-        a = co.m0 * u + co.m1 * init[idx];
-      }
-      double const v = a + cdt * rhs;
-      out[idx] = v;
-      bad |= !__builtin_isfinite(v);
-    } else {
-      out[idx] = rhs;
-    }
-  }
-  if constexpr (MODE == 0) {
-    if (bad) atomicOr(&state->flags, 1);
-  }
 }
 
 // ---------------------------------------------------------------- halos ---
@@ -504,13 +387,6 @@ __global__ void dt_kernel(alpaca_case_state *state, double cell_size, int guard 
   state->dt = dt;
   state->smax = 0;
   if (dt < 2.220446049250313080847263336181640625e-16 && dt > 0.0) state->flags |= 2;
-}
-
-// Zero fill of n doubles (grid-stride): used in place of hipMemsetAsync so
-// that a caller may capture the per-block entries in a HIP graph.
-__global__ __launch_bounds__(kThreads) void zero_kernel(double *p, size_t n) {
-  size_t const stride = (size_t)gridDim.x * kThreads;
-  for (size_t t = (size_t)blockIdx.x * kThreads + threadIdx.x; t < n; t += stride) p[t] = 0.0;
 }
 
 // The listed blocks of a pool, 16 bytes per thread and step (grid-stride; a
@@ -798,37 +674,6 @@ void launch_faces(const alpaca_case_desc *d, int nblocks, const double *in, doub
     launch_faces_flux<DIM, ALPACA_FLUX_ROE>(d, nblocks, in, fl, s);
 }
 
-// Faces into the scratch fl (flux_doubles<DIM>(nblocks) doubles), then the
-// divergence (mode 1) or divergence + RK combination (mode 0) into out.
-template <int DIM>
-int stage_impl(const alpaca_case_desc *d, int nblocks, int stage, int mode, const double *avg,
-               double *init, double *out, alpaca_case_state *state, hipStream_t s, double *fl,
-               double *jump = nullptr) {
-  launch_faces<DIM>(d, nblocks, avg, fl, s);
-  constexpr int cells = Dims<DIM>::CELLS;
-  constexpr int gpb = (cells + kThreads - 1) / kThreads;
-  dim3 grid((unsigned)(nblocks * gpb));
-  double const inv_dx = 1.0 / d->cell_size;
-  ProfileScope prof(ALPACA_KERNEL_COMBINE, s, double(cells) * nblocks);
-  if (mode == 0) {
-    double *ini = (init && init != avg) ? init : nullptr;
-    if (stage > 0) ini = init;
-    hipLaunchKernelGGL((combine_kernel<DIM, 0>), grid, dim3(kThreads), 0, s, fl, avg, ini, out,
-                       nblocks, stage, inv_dx, state);
-  } else {
-    hipLaunchKernelGGL((combine_kernel<DIM, 1>), grid, dim3(kThreads), 0, s, fl, avg, nullptr,
-                       out, nblocks, 0, inv_dx, state);
-  }
-  if (jump) {
-    size_t const total = (size_t)nblocks * 6 * Dims<DIM>::NE * kIC * Dims<DIM>::ICZ;
-    hipLaunchKernelGGL((jump_flux_kernel<DIM>), dim3((unsigned)((total + kThreads - 1) / kThreads)),
-                       dim3(kThreads), 0, s, fl, jump, nblocks);
-  }
-  return hip_status(hipGetLastError());
-}
-
-// Tile shape of the fused stage kernel: 8x8x8 cells and 256 threads in 3D,
-// the whole 16x16 block and 128 threads in 2D.
 // Fused stage kernel of an arithmetic mode.
 template <int DIM, int FLUX, int MODE, int TX, int TY, int TZ, int NT>
 void launch_stage_kernel(dim3 grid, hipStream_t s, const double *avg, const double *init,
@@ -859,9 +704,6 @@ void launch_march_kernel(int nblocks, hipStream_t s, const double *avg, const do
                        a);
 }
 
-// 2D cases with fewer leaf blocks than this run on 8x8 tiles.
-constexpr int kSmallCaseBlocks = 256;
-
 // Whether a 3D case marches (march_stage_kernel) or runs on 8^3 tiles.  Both
 // kernels spend about the same time per unit of 64 faces and wavefront (HLLC
 // FMA 8.2 and 8.3 us, exact 13.6 and 13.5 us at 256^3), a slab taking 26
@@ -878,9 +720,6 @@ bool use_march(int nblocks) {
   return rounds(2LL * nblocks) * 26 <= rounds(8LL * nblocks) * 7;
 }
 
-// Tile shape of the fused stage kernel: 8x8x8 cells and 256 threads in 3D,
-// the whole 16x16 block and 128 threads in 2D (8x8 and 256 threads for a case
-// of fewer than kSmallCaseBlocks blocks).
 template <int DIM, int FLUX, int MODE>
 void launch_stage_fused(const alpaca_case_desc *d, int stage, const double *avg,
                         const double *init, double *out, double *init_copy,
@@ -909,64 +748,14 @@ void launch_stage_fused(const alpaca_case_desc *d, int stage, const double *avg,
         return;
       }
     }
-    constexpr int TX = 8, TY = 8, TZ = 8, NT = 256;
-    constexpr int tiles = (kIC / TX) * (kIC / TY) * (kIC / TZ);
-    launch_stage_kernel<3, FLUX, MODE, TX, TY, TZ, NT>(dim3(nblocks * tiles), s, avg, init, out,
-                                                       state, a);
-  } else if (nblocks >= kSmallCaseBlocks) {
-    launch_stage_kernel<2, FLUX, MODE, 16, 16, 1, 128>(dim3(nblocks), s, avg, init, out, state, a);
-  } else {
-    // Fewer blocks than CUs: four 8x8 tiles per block spread the case over
-    // four times as many workgroups, and 256 threads give every thread at
-    // most one of a tile's faces (the same faces and sums per cell).
-    launch_stage_kernel<2, FLUX, MODE, 8, 8, 1, 256>(dim3(nblocks * 4), s, avg, init, out, state, a);
   }
-}
-
-// Right-hand side with the jump-flux save over listed pool blocks: the fused
-// tile kernel (faces in LDS), tile shapes as for the fused stage kernel.
-template <int DIM, int FLUX, int MODE>
-void launch_rhs_tiles(const alpaca_case_desc *d, const double *avg, double *rhs, double *jump,
-                      const int *list, int n, int capacity, hipStream_t s) {
-  constexpr int TX = DIM == 3 ? 8 : 16, TY = DIM == 3 ? 8 : 16, TZ = DIM == 3 ? 8 : 1;
-  constexpr int NT = DIM == 3 ? 256 : 128;
-  constexpr int tiles = exact::TileShape<DIM, TX, TY, TZ>::TILES;
-  dim3 const grid((unsigned)((size_t)n * tiles));
-  double const inv_dx = 1.0 / d->cell_size;
-  ProfileScope prof(ALPACA_KERNEL_STAGE, s, double(Dims<DIM>::CELLS) * n);
-  if constexpr (MODE == kModeExact)
-    hipLaunchKernelGGL((exact::rhs_tile_kernel<DIM, FLUX, double, TX, TY, TZ, NT>), grid, dim3(NT),
-                       0, s, avg, rhs, jump, list, n, capacity, d->gamma, d->background_pressure,
-                       inv_dx);
-  else if constexpr (MODE == kModeFma)
-    hipLaunchKernelGGL((fast::rhs_tile_kernel<DIM, FLUX, double, TX, TY, TZ, NT>), grid, dim3(NT),
-                       0, s, avg, rhs, jump, list, n, capacity, d->gamma, d->background_pressure,
-                       inv_dx);
-  else
-    hipLaunchKernelGGL((fast::rhs_tile_kernel<DIM, FLUX, float, TX, TY, TZ, NT>), grid, dim3(NT),
-                       0, s, avg, rhs, jump, list, n, capacity, d->gamma, d->background_pressure,
-                       inv_dx);
-}
-
-template <int DIM>
-void rhs_tiles(const alpaca_case_desc *d, const double *avg, double *rhs, double *jump,
-               const int *list, int n, int capacity, hipStream_t s) {
-  int const p = d->precision;
-  if (d->flux == ALPACA_FLUX_HLLC) {
-    if (p == ALPACA_MIXED)
-      launch_rhs_tiles<DIM, ALPACA_FLUX_HLLC, kModeMixed>(d, avg, rhs, jump, list, n, capacity, s);
-    else if (p == ALPACA_FP64_FMA)
-      launch_rhs_tiles<DIM, ALPACA_FLUX_HLLC, kModeFma>(d, avg, rhs, jump, list, n, capacity, s);
-    else
-      launch_rhs_tiles<DIM, ALPACA_FLUX_HLLC, kModeExact>(d, avg, rhs, jump, list, n, capacity, s);
-  } else {
-    if (p == ALPACA_MIXED)
-      launch_rhs_tiles<DIM, ALPACA_FLUX_ROE, kModeMixed>(d, avg, rhs, jump, list, n, capacity, s);
-    else if (p == ALPACA_FP64_FMA)
-      launch_rhs_tiles<DIM, ALPACA_FLUX_ROE, kModeFma>(d, avg, rhs, jump, list, n, capacity, s);
-    else
-      launch_rhs_tiles<DIM, ALPACA_FLUX_ROE, kModeExact>(d, avg, rhs, jump, list, n, capacity, s);
-  }
+  constexpr bool wide = FLUX == ALPACA_FLUX_HLLC && MODE != kModeExact;
+  with_shape<DIM>(nblocks, device_cus(), wide, [&](auto shape) {
+    using S = decltype(shape);
+    constexpr int tiles = exact::TileShape<DIM, S::TX, S::TY, S::TZ>::TILES;
+    launch_stage_kernel<DIM, FLUX, MODE, S::TX, S::TY, S::TZ, S::NT>(dim3(nblocks * tiles), s, avg,
+                                                                     init, out, state, a);
+  });
 }
 
 template <int DIM>
@@ -1137,64 +926,17 @@ int alpaca_ctx_convective_fluxes(alpaca_context *ctx, const alpaca_case_desc *de
 
 }  // extern "C"
 
-// Face-flux scratch of alpaca_right_hand_side_noalloc: one array per GPU,
-// part of the library's code object, so each GPU the library runs on holds
-// it (64 MiB) until the process ends.  Host code never passes this name to a
-// kernel (on the host it is only a stand-in for the symbol): it uses the
-// device address that noalloc_scratch() obtains per device.
-constexpr size_t kNoallocScratchDoubles = ALPACA_RHS_NOALLOC_SCRATCH_BYTES / sizeof(double);
-static __device__ __align__(256) double scratch[kNoallocScratchDoubles];
-static_assert(ALPACA_RHS_NOALLOC_MAX_BLOCKS_3D * alpaca::flux_doubles<3>(1) <= kNoallocScratchDoubles &&
-                  (ALPACA_RHS_NOALLOC_MAX_BLOCKS_3D + 1) * alpaca::flux_doubles<3>(1) >
-                      kNoallocScratchDoubles,
-              "3D block limit of the no-allocation scratch");
-static_assert(ALPACA_RHS_NOALLOC_MAX_BLOCKS_2D * alpaca::flux_doubles<2>(1) <= kNoallocScratchDoubles &&
-                  (ALPACA_RHS_NOALLOC_MAX_BLOCKS_2D + 1) * alpaca::flux_doubles<2>(1) >
-                      kNoallocScratchDoubles,
-              "2D block limit of the no-allocation scratch");
-
 namespace alpaca {
 namespace {
 
-// Right-hand side of nblocks blocks with the face fluxes in fl: zero the
-// output blocks, faces, divergence, and (jump != null) the boundary-flux save.
-int rhs_with_scratch(const alpaca_case_desc *desc, int nblocks, const double *d_avg, double *d_rhs,
-                     double *d_jump, double *fl, hipStream_t s) {
-  size_t const n = alpaca_block_doubles(desc->dim) * (size_t)nblocks;
-  unsigned const groups = (unsigned)std::min<size_t>((n + kThreads - 1) / kThreads, 65536);
-  hipLaunchKernelGGL(zero_kernel, dim3(groups), dim3(kThreads), 0, s, d_rhs, n);
-  if (desc->dim == 2)
-    return stage_impl<2>(desc, nblocks, 0, 1, d_avg, nullptr, d_rhs, nullptr, s, fl, d_jump);
-  return stage_impl<3>(desc, nblocks, 0, 1, d_avg, nullptr, d_rhs, nullptr, s, fl, d_jump);
-}
-
-int rhs_context(alpaca_context *ctx, const alpaca_case_desc *desc, int nblocks,
-                const double *d_avg, double *d_rhs, double *d_jump) {
-  double *fl = nullptr;
-  size_t const n = desc->dim == 2 ? flux_doubles<2>(nblocks) : flux_doubles<3>(nblocks);
-  int st = context_scratch(ctx, n * sizeof(double), &fl);
-  if (st != ALPACA_OK) return st;
-  return rhs_with_scratch(desc, nblocks, d_avg, d_rhs, d_jump, fl, ctx->stream);
-}
-
-// Device address of `scratch` on the current device, looked up once per
-// device (hipGetSymbolAddress with that device current) and kept.
-constexpr int kMaxDevices = 64;
-std::mutex g_noalloc_mutex;
-double *g_noalloc_ptr[kMaxDevices] = {};
-
-int noalloc_scratch(double **out) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return ALPACA_ERR_HIP;
-  if (dev < 0 || dev >= kMaxDevices) return ALPACA_ERR_UNSUPPORTED;
-  std::lock_guard<std::mutex> lock(g_noalloc_mutex);
-  if (!g_noalloc_ptr[dev]) {
-    void *p = nullptr;
-    if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p) return ALPACA_ERR_HIP;
-    g_noalloc_ptr[dev] = static_cast<double *>(p);
-  }
-  *out = g_noalloc_ptr[dev];
-  return ALPACA_OK;
+// Right-hand side of the first n blocks, or of those listed of a pool.
+int right_hand_side(const alpaca_case_desc *desc, int n, const double *d_avg, double *d_rhs,
+                    double *d_jump, hipStream_t s, BlockList list = {}) {
+  ProfileScope prof(ALPACA_KERNEL_STAGE, s,
+                    double(desc->dim == 2 ? Dims<2>::CELLS : Dims<3>::CELLS) * n);
+  launch_rhs(desc, d_avg, d_rhs, d_jump, list.list, n, list.list ? list.capacity : n, device_cus(),
+             s);
+  return hip_status(hipGetLastError());
 }
 
 }  // namespace
@@ -1208,7 +950,7 @@ int alpaca_ctx_right_hand_side(alpaca_context *ctx, const alpaca_case_desc *desc
   if (st != ALPACA_OK) return st;
   if (!ctx || nblocks < 1 || nblocks > kMaxBlocks || !d_avg || !d_rhs || d_avg == d_rhs)
     return ALPACA_ERR_INVALID;
-  return rhs_context(ctx, desc, nblocks, d_avg, d_rhs, nullptr);
+  return right_hand_side(desc, nblocks, d_avg, d_rhs, nullptr, ctx->stream);
 }
 
 int alpaca_ctx_right_hand_side_jump_fluxes(alpaca_context *ctx, const alpaca_case_desc *desc,
@@ -1219,7 +961,7 @@ int alpaca_ctx_right_hand_side_jump_fluxes(alpaca_context *ctx, const alpaca_cas
   if (!ctx || nblocks < 1 || nblocks > kMaxBlocks || !d_avg || !d_rhs || !d_jump_fluxes ||
       d_avg == d_rhs)
     return ALPACA_ERR_INVALID;
-  return rhs_context(ctx, desc, nblocks, d_avg, d_rhs, d_jump_fluxes);
+  return right_hand_side(desc, nblocks, d_avg, d_rhs, d_jump_fluxes, ctx->stream);
 }
 
 int alpaca_ctx_right_hand_side_jump_fluxes_list(alpaca_context *ctx, const alpaca_case_desc *desc,
@@ -1233,11 +975,8 @@ int alpaca_ctx_right_hand_side_jump_fluxes_list(alpaca_context *ctx, const alpac
     return ALPACA_ERR_INVALID;
   if (n == 0) return ALPACA_OK;
   if (!d_list) return ALPACA_ERR_INVALID;
-  if (desc->dim == 2)
-    rhs_tiles<2>(desc, d_avg, d_rhs, d_jump_fluxes, d_list, n, capacity, ctx->stream);
-  else
-    rhs_tiles<3>(desc, d_avg, d_rhs, d_jump_fluxes, d_list, n, capacity, ctx->stream);
-  return hip_status(hipGetLastError());
+  return right_hand_side(desc, n, d_avg, d_rhs, d_jump_fluxes, ctx->stream,
+                         BlockList{d_list, capacity});
 }
 
 int alpaca_swap_blocks_list(int dim, double *d_a, double *d_b, int capacity, const int *d_list,
@@ -1280,9 +1019,7 @@ int alpaca_right_hand_side(const alpaca_case_desc *desc, int nblocks, const doub
   if (st != ALPACA_OK) return st;
   if (nblocks < 1 || nblocks > kMaxBlocks || !d_avg || !d_rhs || d_avg == d_rhs)
     return ALPACA_ERR_INVALID;
-  alpaca_context *ctx = nullptr;
-  if ((st = stream_context(static_cast<hipStream_t>(stream), &ctx)) != ALPACA_OK) return st;
-  return rhs_context(ctx, desc, nblocks, d_avg, d_rhs, nullptr);
+  return right_hand_side(desc, nblocks, d_avg, d_rhs, nullptr, static_cast<hipStream_t>(stream));
 }
 
 int alpaca_right_hand_side_jump_fluxes(const alpaca_case_desc *desc, int nblocks,
@@ -1292,9 +1029,7 @@ int alpaca_right_hand_side_jump_fluxes(const alpaca_case_desc *desc, int nblocks
   if (st != ALPACA_OK) return st;
   if (nblocks < 1 || nblocks > kMaxBlocks || !d_avg || !d_rhs || !d_jump_fluxes || d_avg == d_rhs)
     return ALPACA_ERR_INVALID;
-  alpaca_context *ctx = nullptr;
-  if ((st = stream_context(static_cast<hipStream_t>(stream), &ctx)) != ALPACA_OK) return st;
-  return rhs_context(ctx, desc, nblocks, d_avg, d_rhs, d_jump_fluxes);
+  return right_hand_side(desc, nblocks, d_avg, d_rhs, d_jump_fluxes, static_cast<hipStream_t>(stream));
 }
 
 int alpaca_right_hand_side_noalloc(const alpaca_case_desc *desc, int nblocks, const double *d_avg,
@@ -1304,10 +1039,8 @@ int alpaca_right_hand_side_noalloc(const alpaca_case_desc *desc, int nblocks, co
   if (nblocks < 1 || !d_avg || !d_rhs || d_avg == d_rhs) return ALPACA_ERR_INVALID;
   if (nblocks > (desc->dim == 2 ? ALPACA_RHS_NOALLOC_MAX_BLOCKS_2D : ALPACA_RHS_NOALLOC_MAX_BLOCKS_3D))
     return ALPACA_ERR_CAPACITY;
-  double *fl = nullptr;
-  if ((st = noalloc_scratch(&fl)) != ALPACA_OK) return st;
   g_prof_suppressed = true;
-  st = rhs_with_scratch(desc, nblocks, d_avg, d_rhs, nullptr, fl, static_cast<hipStream_t>(stream));
+  st = right_hand_side(desc, nblocks, d_avg, d_rhs, nullptr, static_cast<hipStream_t>(stream));
   g_prof_suppressed = false;
   return st;
 }

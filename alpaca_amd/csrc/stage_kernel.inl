@@ -167,8 +167,8 @@ template <int DIM, int TX, int TY, int TZ> struct TileShape {
 
 // Face fluxes of one tile (first cell x0, y0, z0 of block bb) into LDS:
 // every face of the tile, a flat loop whose per-direction ranges are padded
-// to 64 so each wavefront works on a single direction.  JUMP: a face on the
-// block's boundary is also added into the block's jump-flux surfaces
+// to 64 so each wavefront works on a single direction.  JUMP with a pointer: a
+// face on the block's boundary is also added into its jump-flux surfaces
 // ([6][NE][IC][ICZ]: East, West, North, South, Top, Bottom; the boundary-flux
 // save of SpaceSolver::UpdateFluxes, space_solver.cpp:160-182).
 template <int DIM, int FLUX, typename R, int TX, int TY, int TZ, int NT, bool JUMP>
@@ -201,7 +201,7 @@ __device__ __forceinline__ void tile_faces(int tid, const double *__restrict__ b
         for (int e = 0; e < NE; ++e) FX[e * NFX + f] = fl[e];
         if constexpr (JUMP) {
           int const gx = x0 + ia;
-          if (gx == 0 || gx == kIC) save(gx == kIC ? 0 : 1, y0 + jj, z0 + k, fl);
+          if (jump && (gx == 0 || gx == kIC)) save(gx == kIC ? 0 : 1, y0 + jj, z0 + k, fl);
         }
       }
     } else if (f < PX + PY) {
@@ -214,7 +214,7 @@ __device__ __forceinline__ void tile_faces(int tid, const double *__restrict__ b
         for (int e = 0; e < NE; ++e) FY[e * NFY + r] = fl[e];
         if constexpr (JUMP) {
           int const gy = y0 + ja;
-          if (gy == 0 || gy == kIC) save(gy == kIC ? 2 : 3, x0 + i, z0 + k, fl);
+          if (jump && (gy == 0 || gy == kIC)) save(gy == kIC ? 2 : 3, x0 + i, z0 + k, fl);
         }
       }
     } else {
@@ -228,7 +228,7 @@ __device__ __forceinline__ void tile_faces(int tid, const double *__restrict__ b
           for (int e = 0; e < NE; ++e) FZ[e * NFZ + r] = fl[e];
           if constexpr (JUMP) {
             int const gz = z0 + ka;
-            if (gz == 0 || gz == kIC) save(gz == kIC ? 4 : 5, x0 + i, y0 + jj, fl);
+            if (jump && (gz == 0 || gz == kIC)) save(gz == kIC ? 4 : 5, x0 + i, y0 + jj, fl);
           }
         }
       }
@@ -572,14 +572,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMinWaves<3
   stage_march<FLUX, R>(j, blk, g % SLABS, lds);
 }
 
-// Right-hand side of listed blocks of a pool (SpaceSolver::UpdateFluxes in
-// full, space_solver.cpp:50-182), one workgroup per (list entry, tile):
-// the tile's faces into LDS, those on the block's boundary also added into
-// its jump-flux surfaces; after the barrier each internal cell's flux
+// Right-hand side of n blocks (SpaceSolver::UpdateFluxes, space_solver.cpp:
+// 50-182): those listed of a pool, or, without a list, blocks 0 .. n-1.  One
+// workgroup per (block, tile): the tile's faces into LDS, those on the block's
+// boundary also added into its jump-flux surfaces (jump not null); after the
+// barrier each internal cell's flux
 // divergence (ConsistencyManagedSum, space_solver.cpp:131-153) is written to
 // the block's right-hand-side buffer, and the tile's share of the block's
 // halo cells is set to zero (the whole output block is written, as by the
-// unfused per-block entry).  In 2D the Top and Bottom surfaces receive += 0.0,
+// per-block right-hand side that the reference clears first).  In 2D the Top and Bottom surfaces receive += 0.0,
 // as from the reference's zeroed z face array.  List entries outside
 // [0, capacity) are skipped (uniformly over the workgroup).
 template <int DIM, int FLUX, typename R, int TX, int TY, int TZ, int NT>
@@ -597,15 +598,15 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kMinWaves<DI
   unsigned const g = xcd_remap_group(blockIdx.x, gridDim.x);
   int const item = int(g / T::TILES), tile = int(g % T::TILES);
   if (item >= n) return;
-  int const blk = list[item];
+  int const blk = list ? list[item] : item;
   if (blk < 0 || blk >= capacity) return;  // uniform over the workgroup
   int const z0 = DIM == 3 ? (tile % NTZ) * TZ : 0;
   int const y0 = ((tile / NTZ) % NTY) * TY;
   int const x0 = (tile / (NTZ * NTY)) * TX;
-  double *jb = jump + (size_t)blk * SURF;
+  double *jb = jump ? jump + (size_t)blk * SURF : nullptr;
   tile_faces<DIM, FLUX, R, TX, TY, TZ, NT, true>(threadIdx.x, avg + (size_t)blk * D::BLOCK, x0, y0, z0, gamma,
                                                  b, lds, jb);
-  if constexpr (DIM == 2) {
+  if (DIM == 2 && jb) {
     for (int t = threadIdx.x; t < 2 * NE * kIC; t += NT) jb[4 * NE * kIC + t] += 0.0;
   }
   __syncthreads();

@@ -212,15 +212,11 @@ int alpaca_copy_blocks_list(int dim, const double *d_src, double *d_dst, int cap
 /* (ii) without allocation.  No counterpart in the reference: for callers that
  * cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc).  The same results, bit for bit, as
- * alpaca_right_hand_side; the face fluxes go to a fixed 64 MiB scratch array
- * that the library holds on each GPU it runs on until the process ends, so
- * the call makes no hipMalloc/hipFree and no other allocating call (the
- * profiling hooks record nothing for it).  At most
- * ALPACA_RHS_NOALLOC_MAX_BLOCKS_3D / _2D blocks per call; larger calls return
- * ALPACA_ERR_CAPACITY and launch nothing.  Every call on one GPU shares that
- * GPU's array, which keeps the last call's face fluxes (each call writes all
- * the faces it reads): calls that overlap on one GPU (different streams, or
- * host threads without ordering) race. */
+ * alpaca_right_hand_side, which needs no scratch either; here the profiling
+ * hooks, whose events allocate, record nothing.  At most
+ * ALPACA_RHS_NOALLOC_MAX_BLOCKS_3D / _2D blocks per call (the blocks whose face
+ * fluxes take ALPACA_RHS_NOALLOC_SCRATCH_BYTES); larger calls return
+ * ALPACA_ERR_CAPACITY and launch nothing. */
 #define ALPACA_RHS_NOALLOC_SCRATCH_BYTES (64u << 20)
 #define ALPACA_RHS_NOALLOC_MAX_BLOCKS_3D 128
 #define ALPACA_RHS_NOALLOC_MAX_BLOCKS_2D 3855
