@@ -329,9 +329,13 @@ __global__ __launch_bounds__(kThreads) void halo_list_kernel(double *blocks, int
 
 // ----------------------------------------------------------- time step ---
 
-// Per block: max over internal cells of sum_d(|u_d| + c)
-// (modular_algorithm_assembler.cpp:1840-1869), then an atomic max on the
-// IEEE bits (non-negative doubles order like their bit patterns).
+// Max over the internal cells of n blocks of sum_d(|u_d| + c)
+// (modular_algorithm_assembler.cpp:1840-1869), raised into the record as IEEE
+// bits (non-negative doubles order like their bit patterns).  The cells are
+// dealt in chunks of 256, a workgroup striding over them: one raise of the
+// record per workgroup, and the chunks of few 3D blocks spread over the chip.
+// One workgroup and one atomic per block took 194 us for 2048^2 cells (the
+// atomics on one address; reading the cells takes 30 us).
 template <int DIM>
 __global__ __launch_bounds__(kThreads) void signal_kernel(const double *__restrict__ in, int nblocks,
                                                           double gamma, double b,
@@ -339,13 +343,14 @@ __global__ __launch_bounds__(kThreads) void signal_kernel(const double *__restri
   using D = Dims<DIM>;
   constexpr int NE = D::NE;
   constexpr int ICZ = D::ICZ;
+  constexpr int CHUNKS = D::CELLS / kThreads;  // per block
+  static_assert(CHUNKS * kThreads == D::CELLS, "whole chunks");
   __shared__ double part[kThreads / 64];
-  int const blk = blockIdx.x;
-  if (blk >= nblocks) return;
-  int const mem = list.block(blk);  // uniform over the workgroup
-  if (mem < 0) return;
   double s = 0.0;
-  for (int c = threadIdx.x; c < D::CELLS; c += kThreads) {
+  for (long long q = blockIdx.x; q < (long long)nblocks * CHUNKS; q += gridDim.x) {
+    int const mem = list.block(int(q / CHUNKS));  // uniform over the workgroup
+    if (mem < 0) continue;
+    int const c = int(q % CHUNKS) * kThreads + threadIdx.x;
     int const kk = c % ICZ, jj = (c / ICZ) % kIC, ii = c / (ICZ * kIC);
     const double *p = in + (size_t)mem * D::BLOCK + (ii + kHS) * D::SX + (jj + kHS) * D::SY +
                       (DIM == 3 ? kk + kHS : 0);
@@ -370,23 +375,38 @@ __global__ __launch_bounds__(kThreads) void signal_kernel(const double *__restri
     double m = part[0];
 #pragma unroll
     for (int w = 1; w < kThreads / 64; ++w) m = exact::smax(m, part[w]);
-    atomicMax(reinterpret_cast<unsigned long long *>(&state->smax),
-              (unsigned long long)__double_as_longlong(m));
+    exact::raise_signal(state, m);
   }
 }
 
-// dt = CFL / (S / dx), end-time clamp, minimum-step health check
-// (modular_algorithm_assembler.cpp:1932-1982; ComputeLoop :137-140).
+// The record's next time step: dt = CFL / (S / dx), end-time clamp,
+// minimum-step health check (modular_algorithm_assembler.cpp:1932-1982;
+// ComputeLoop :137-140).
+__device__ __forceinline__ void next_dt(alpaca_case_state &r, double cell_size) {
+  double const s = __longlong_as_double((long long)r.smax);
+  double const rate = exact::fdiv(s, cell_size);
+  double dt = rate == 0.0 ? 1.7976931348623157e308 : exact::fdiv(r.cfl, rate);
+  if (r.time + dt > r.t_end) dt = exact::smax(r.t_end - r.time, 0.0);
+  r.dt = dt;
+  r.smax = 0;
+  if (dt < 2.220446049250313080847263336181640625e-16 && dt > 0.0) r.flags |= 2;
+}
+
+// The end of a step in the record.
+__device__ __forceinline__ void finish_step(alpaca_case_state &r) {
+  r.time += 0.0 + r.dt;
+  r.steps += 1;
+  if (!(r.time < r.t_end)) r.flags |= kFlagDone;
+}
+
+// The kernels that change the record read and write it as a whole, in one
+// round trip to memory; they follow the launches that raise smax or set flags.
 __global__ void dt_kernel(alpaca_case_state *state, double cell_size, int guard = 0) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  if (guard && (state->flags & kFlagDone)) return;
-  double const s = __longlong_as_double((long long)state->smax);
-  double const rate = exact::fdiv(s, cell_size);
-  double dt = rate == 0.0 ? 1.7976931348623157e308 : exact::fdiv(state->cfl, rate);
-  if (state->time + dt > state->t_end) dt = exact::smax(state->t_end - state->time, 0.0);
-  state->dt = dt;
-  state->smax = 0;
-  if (dt < 2.220446049250313080847263336181640625e-16 && dt > 0.0) state->flags |= 2;
+  alpaca_case_state r = *state;
+  if (guard && (r.flags & kFlagDone)) return;
+  next_dt(r, cell_size);
+  *state = r;
 }
 
 // The listed blocks of a pool, 16 bytes per thread and step (grid-stride; a
@@ -454,10 +474,10 @@ __global__ __launch_bounds__(kThreads) void exact_ops_kernel(const double *__res
 // time is no longer below t_end.  guard: a record already done is left alone.
 __global__ void finish_step_kernel(alpaca_case_state *state, int guard = 0) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  if (guard && (state->flags & kFlagDone)) return;
-  state->time += 0.0 + state->dt;
-  state->steps += 1;
-  if (!(state->time < state->t_end)) state->flags |= kFlagDone;
+  alpaca_case_state r = *state;
+  if (guard && (r.flags & kFlagDone)) return;
+  finish_step(r);
+  *state = r;
 }
 
 // finish_step_kernel followed by dt_kernel for the next step, both guarded,
@@ -465,20 +485,11 @@ __global__ void finish_step_kernel(alpaca_case_state *state, int guard = 0) {
 // step boundary inside alpaca_advance.
 __global__ void finish_and_dt_kernel(alpaca_case_state *state, double cell_size) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  if (state->flags & kFlagDone) return;
-  state->time += 0.0 + state->dt;
-  state->steps += 1;
-  if (!(state->time < state->t_end)) {
-    state->flags |= kFlagDone;
-    return;
-  }
-  double const s = __longlong_as_double((long long)state->smax);
-  double const rate = exact::fdiv(s, cell_size);
-  double dt = rate == 0.0 ? 1.7976931348623157e308 : exact::fdiv(state->cfl, rate);
-  if (state->time + dt > state->t_end) dt = exact::smax(state->t_end - state->time, 0.0);
-  state->dt = dt;
-  state->smax = 0;
-  if (dt < 2.220446049250313080847263336181640625e-16 && dt > 0.0) state->flags |= 2;
+  alpaca_case_state r = *state;
+  if (r.flags & kFlagDone) return;
+  finish_step(r);
+  if (!(r.flags & kFlagDone)) next_dt(r, cell_size);
+  *state = r;
 }
 
 __global__ void state_init_kernel(alpaca_case_state *state, double time, double t_end, double cfl) {
@@ -806,7 +817,10 @@ template <int DIM>
 int timestep_impl(const alpaca_case_desc *d, const double *avg, alpaca_case_state *state,
                   hipStream_t s, int nblocks, BlockList list = {}, int guard = 0) {
   ProfileScope prof(ALPACA_KERNEL_TIMESTEP, s, double(Dims<DIM>::CELLS) * nblocks);
-  hipLaunchKernelGGL((signal_kernel<DIM>), dim3(nblocks), dim3(kThreads), 0, s, avg, nblocks,
+  // Eight workgroups of four wavefronts fill a CU.
+  long long const chunks = (long long)nblocks * (Dims<DIM>::CELLS / kThreads);
+  unsigned const groups = (unsigned)std::min<long long>(chunks, 8LL * device_cus());
+  hipLaunchKernelGGL((signal_kernel<DIM>), dim3(groups), dim3(kThreads), 0, s, avg, nblocks,
                      d->gamma, d->background_pressure, state, list);
   hipLaunchKernelGGL(dt_kernel, dim3(1), dim3(64), 0, s, state, d->cell_size, guard);
   return hip_status(hipGetLastError());
