@@ -198,47 +198,17 @@ struct Range {
   int count[3];  // predicted parent cells per axis (child count / 2)
 };
 
-// The 2^DIM predicted child values of the parent cell at LDS index `o` of a
-// window (Lds layout): out[dx | dy << 1 | dz << 2].  In 2D the
-// z terms are the reference's zero-initialised Qz, Qxz, Qyz, Qxyz, and enter
-// the sums as such (their signs matter for signed zeros).
-template <int DIM, typename L = Lds<DIM>>
-__device__ __forceinline__ void predict_cell(const double *__restrict__ s, int o,
-                                             double out[1 << DIM]) {
-  constexpr int sx = L::SX, sy = L::SY;
-  constexpr double c0 = -22.0 / 128.0, c1 = 3.0 / 128.0;
-  constexpr double c00 = c0 * c0, c01 = c0 * c1, c10 = c01, c11 = c1 * c1;
-  constexpr double c000 = c00 * c0, c001 = c00 * c1, c010 = c001, c011 = c0 * c11;
-  constexpr double c100 = c001, c101 = c011, c110 = c011, c111 = c1 * c11;
-#define P(a, b, c) s[o + (a) * sx + (b) * sy + (c)]
-  double Qz = 0.0, Qxz = 0.0, Qyz = 0.0, Qxyz = 0.0;
-  double const Qx = c0 * (P(1, 0, 0) - P(-1, 0, 0)) + c1 * (P(2, 0, 0) - P(-2, 0, 0));
-  double const Qy = c0 * (P(0, 1, 0) - P(0, -1, 0)) + c1 * (P(0, 2, 0) - P(0, -2, 0));
-  double const Qxy =
-      (c00 * ((P(1, 1, 0) + P(-1, -1, 0)) - (P(-1, 1, 0) + P(1, -1, 0))) +
-       c11 * ((P(2, 2, 0) + P(-2, -2, 0)) - (P(-2, 2, 0) + P(2, -2, 0)))) +
-      (c01 * ((P(1, 2, 0) + P(-1, -2, 0)) - (P(-1, 2, 0) + P(1, -2, 0))) +
-       c10 * ((P(2, 1, 0) + P(-2, -1, 0)) - (P(-2, 1, 0) + P(2, -1, 0))));
-  if constexpr (DIM == 3) {
-    Qz = c0 * (P(0, 0, 1) - P(0, 0, -1)) + c1 * (P(0, 0, 2) - P(0, 0, -2));
-    Qxz = (c00 * ((P(1, 0, 1) + P(-1, 0, -1)) - (P(-1, 0, 1) + P(1, 0, -1))) +
-           c11 * ((P(2, 0, 2) + P(-2, 0, -2)) - (P(-2, 0, 2) + P(2, 0, -2)))) +
-          (c01 * ((P(1, 0, 2) + P(-1, 0, -2)) - (P(-1, 0, 2) + P(1, 0, -2))) +
-           c10 * ((P(2, 0, 1) + P(-2, 0, -1)) - (P(-2, 0, 1) + P(2, 0, -1))));
-    Qyz = (c00 * ((P(0, 1, 1) + P(0, -1, -1)) - (P(0, -1, 1) + P(0, 1, -1))) +
-           c11 * ((P(0, 2, 2) + P(0, -2, -2)) - (P(0, -2, 2) + P(0, 2, -2)))) +
-          (c01 * ((P(0, 1, 2) + P(0, -1, -2)) - (P(0, -1, 2) + P(0, 1, -2))) +
-           c10 * ((P(0, 2, 1) + P(0, -2, -1)) - (P(0, -2, 1) + P(0, 2, -1))));
-    // The four antisymmetric differences over the corners (+-a, +-b, +-c).
-#define G(a, b, c)                                     \
-  cms4(P(a, b, c) - P(-(a), -(b), -(c)), P(-(a), -(b), c) - P(a, b, -(c)), \
-       P(a, -(b), -(c)) - P(-(a), b, c), P(-(a), b, -(c)) - P(a, -(b), c))
-    Qxyz = cms4(c000 * G(1, 1, 1) + c111 * G(2, 2, 2), c001 * G(1, 1, 2) + c110 * G(2, 2, 1),
-                c011 * G(1, 2, 2) + c100 * G(2, 1, 1), c010 * G(1, 2, 1) + c101 * G(2, 1, 2));
-#undef G
-  }
-  double const p = P(0, 0, 0);
-#undef P
+constexpr double kC0 = -22.0 / 128.0, kC1 = 3.0 / 128.0;
+constexpr double kC00 = kC0 * kC0, kC01 = kC0 * kC1, kC10 = kC01, kC11 = kC1 * kC1;
+constexpr double kC000 = kC00 * kC0, kC001 = kC00 * kC1, kC010 = kC001, kC011 = kC0 * kC11;
+constexpr double kC100 = kC001, kC101 = kC011, kC110 = kC011, kC111 = kC1 * kC11;
+
+// The predicted children of a parent cell from its value p and its
+// polynomial's terms: out[dx | dy << 1 | dz << 2].
+template <int DIM>
+__device__ __forceinline__ void form_children(double p, double Qx, double Qy, double Qz, double Qxy,
+                                              double Qxz, double Qyz, double Qxyz,
+                                              double out[1 << DIM]) {
   out[0] = p + dams<DIM>(Qx, Qy, Qz) + dams<DIM>(Qxy, Qxz, Qyz) + Qxyz;
   out[1] = p + dams<DIM>(-Qx, Qy, Qz) + dams<DIM>(-Qxy, -Qxz, Qyz) - Qxyz;
   out[2] = p + dams<DIM>(Qx, -Qy, Qz) + dams<DIM>(-Qxy, Qxz, -Qyz) - Qxyz;
@@ -248,6 +218,119 @@ __device__ __forceinline__ void predict_cell(const double *__restrict__ s, int o
     out[5] = p + cms3(-Qx, Qy, -Qz) + cms3(-Qxy, Qxz, -Qyz) + Qxyz;
     out[6] = p + cms3(Qx, -Qy, -Qz) + cms3(-Qxy, -Qxz, Qyz) + Qxyz;
     out[7] = p + cms3(-Qx, -Qy, -Qz) + cms3(Qxy, Qxz, Qyz) - Qxyz;
+  }
+}
+
+// 2D: the predicted children of the parent cell at LDS index `o` of a window.
+// The z terms are the reference's zero-initialised Qz, Qxz, Qyz, Qxyz, and
+// enter the sums as such (their signs matter for signed zeros).
+template <typename L = Lds<2>>
+__device__ __forceinline__ void predict_cell(const double *__restrict__ s, int o, double out[4]) {
+#define P(a, b) s[o + (a) * L::SX + (b) * L::SY]
+  double const Qx = kC0 * (P(1, 0) - P(-1, 0)) + kC1 * (P(2, 0) - P(-2, 0));
+  double const Qy = kC0 * (P(0, 1) - P(0, -1)) + kC1 * (P(0, 2) - P(0, -2));
+  double const Qxy = (kC00 * ((P(1, 1) + P(-1, -1)) - (P(-1, 1) + P(1, -1))) +
+                      kC11 * ((P(2, 2) + P(-2, -2)) - (P(-2, 2) + P(2, -2)))) +
+                     (kC01 * ((P(1, 2) + P(-1, -2)) - (P(-1, 2) + P(1, -2))) +
+                      kC10 * ((P(2, 1) + P(-2, -1)) - (P(-2, 1) + P(2, -1))));
+  form_children<2>(P(0, 0), Qx, Qy, 0.0, Qxy, 0.0, 0.0, 0.0, out);
+#undef P
+}
+
+// Makes the values be formed here.
+__device__ __forceinline__ void formed(double &a, double &b) { asm volatile("" : "+v"(a), "+v"(b)); }
+
+// 3D: the predicted children of the two parent cells at LDS indices o and
+// o + 1 (o even).  Both stencils lie in 25 rows of six values along z, each read
+// once by three 16-byte accesses, in the order in which the terms use them: 600
+// bytes of LDS a cell.  The fences make the compiler form a group's results
+// before the next group's rows are read (it moves both otherwise, and 100
+// registers spill).
+// (A thread per cell read 125 values, 1000 bytes, as
+// 8-byte accesses: LDS-bound, 7600 cycles per wavefront of cells where the 428
+// FP64 instructions issue in 1700.)
+template <typename L>
+__device__ __forceinline__ void predict_pair(const double *__restrict__ s, int o,
+                                             double (&out)[2][8]) {
+  struct Row {
+    double v[6];
+    __device__ __forceinline__ Row(const double *q) {
+      double2 const a = reinterpret_cast<const double2 *>(q)[0];
+      double2 const b = reinterpret_cast<const double2 *>(q)[1];
+      double2 const c = reinterpret_cast<const double2 *>(q)[2];
+      v[0] = a.x, v[1] = a.y, v[2] = b.x, v[3] = b.y, v[4] = c.x, v[5] = c.y;
+    }
+  };
+  auto row = [s, o](int a, int b) { return Row(s + (o - 2 + a * L::SX + b * L::SY)); };
+  double Qx[2], Qy[2], Qz[2], Qxy[2], Qxz[2], Qyz[2], Qxyz[2], p[2];
+  {
+    // The four antisymmetric differences over the corners (+-a, +-b, +-c),
+    // c = 1, 2, and the diagonal difference of the rows (+-a, +-b).
+    struct Corner {
+      double g[2][2], d[2];
+    };
+    auto corner = [&row](int a, int b) {
+      Row const pp = row(a, b), mm = row(-a, -b), mp = row(-a, b), pm = row(a, -b);
+      Corner k;
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        int const z = n + 2;
+        k.d[n] = (pp.v[z] + mm.v[z]) - (mp.v[z] + pm.v[z]);
+#pragma unroll
+        for (int c = 1; c <= 2; ++c)
+          k.g[n][c - 1] = cms4(pp.v[z + c] - mm.v[z - c], mm.v[z + c] - pp.v[z - c],
+                               pm.v[z - c] - mp.v[z + c], mp.v[z - c] - pm.v[z + c]);
+      }
+#pragma unroll
+      for (int n = 0; n < 2; ++n) formed(k.g[n][0], k.g[n][1]), formed(k.d[n], k.g[n][1]);
+      __builtin_amdgcn_sched_barrier(0);
+      return k;
+    };
+    double q0[2], q1[2], xy[2];
+    {
+      Corner const k11 = corner(1, 1);
+      Corner const k22 = corner(2, 2);
+#pragma unroll
+      for (int n = 0; n < 2; ++n) {
+        xy[n] = kC00 * k11.d[n] + kC11 * k22.d[n];
+        q0[n] = kC000 * k11.g[n][0] + kC111 * k22.g[n][1];
+        q1[n] = kC001 * k11.g[n][1] + kC110 * k22.g[n][0];
+      }
+    }
+    Corner const k12 = corner(1, 2);
+    Corner const k21 = corner(2, 1);
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      Qxy[n] = xy[n] + (kC01 * k12.d[n] + kC10 * k21.d[n]);
+      Qxyz[n] = cms4(q0[n], q1[n], kC011 * k12.g[n][1] + kC100 * k21.g[n][0],
+                     kC010 * k12.g[n][0] + kC101 * k21.g[n][1]);
+    }
+  }
+  // The planes of an axis and z.
+  auto plane = [&row](int a, int b, double (&Q)[2], double (&Qd)[2]) {
+    Row const p1 = row(a, b), m1 = row(-a, -b), p2 = row(2 * a, 2 * b), m2 = row(-2 * a, -2 * b);
+    auto diag = [](const Row &p, const Row &m, int z, int c) {
+      return (p.v[z + c] + m.v[z - c]) - (m.v[z + c] + p.v[z - c]);
+    };
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      int const z = n + 2;
+      Q[n] = kC0 * (p1.v[z] - m1.v[z]) + kC1 * (p2.v[z] - m2.v[z]);
+      Qd[n] = (kC00 * diag(p1, m1, z, 1) + kC11 * diag(p2, m2, z, 2)) +
+              (kC01 * diag(p1, m1, z, 2) + kC10 * diag(p2, m2, z, 1));
+      formed(Q[n], Qd[n]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  plane(1, 0, Qx, Qxz);
+  plane(0, 1, Qy, Qyz);
+  Row const line = row(0, 0);
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+    int const z = n + 2;
+    Qz[n] = kC0 * (line.v[z + 1] - line.v[z - 1]) + kC1 * (line.v[z + 2] - line.v[z - 2]);
+    p[n] = line.v[z];
+    form_children<3>(p[n], Qx[n], Qy[n], Qz[n], Qxy[n], Qxz[n], Qyz[n], Qxyz[n], out[n]);
   }
 }
 
@@ -334,7 +417,7 @@ __device__ __forceinline__ void predict_range(double *s, double *__restrict__ bl
   for (int t = threadIdx.x; t < tasks; t += kStencilThreads) {
     int const a = t / (r.count[1] * nz), b = (t / nz) % r.count[1], c = t % nz;
     double v[1 << DIM];
-    predict_cell<DIM>(s, Window<DIM>::centre(a, b, c), v);
+    predict_cell(s, Window<DIM>::centre(a, b, c), v);
     int const ci = r.start[0] + 2 * a, cj = r.start[1] + 2 * b;
     int const ck = DIM == 3 ? r.start[2] + 2 * c : 0;
     store_children<DIM>(child + ci * D::SX + cj * D::SY + ck, v);
@@ -394,7 +477,7 @@ __device__ __forceinline__ void predict_range_equations(double *s, double *__res
     for (int t = threadIdx.x; t < tasks; t += kStencilThreads) {
       int const a = t / (r.count[1] * nz), b = (t / nz) % r.count[1], c = t % nz;
       double v[1 << DIM];
-      predict_cell<DIM, L>(cur, Window<DIM>::template centre<L>(a, b, c), v);
+      predict_cell<L>(cur, Window<DIM>::template centre<L>(a, b, c), v);
       int const ci = r.start[0] + 2 * a, cj = r.start[1] + 2 * b;
       int const ck = DIM == 3 ? r.start[2] + 2 * c : 0;
       store_children<DIM>(out + ci * D::SX + cj * D::SY + ck, v);
@@ -478,6 +561,147 @@ __global__ __launch_bounds__(kStencilThreads) void jump_halo_kernel(
   predict_range_equations<DIM>(s, blocks, l, r);
 }
 
+// ------------------------------------------------------------ 3D predictions
+
+// Quotients of numbers below 4096 by a divisor up to 256 that is the same for
+// the whole workgroup: n * ceil(2^21 / d) >> 21 is exact there, both factors fit
+// 24 bits, and the product 32 where n < 4096 and d >= 5, or n < 1024.
+struct SmallDiv {
+  unsigned d, m;
+  __device__ __forceinline__ explicit SmallDiv(int by)
+      : d((unsigned)by), m(((1u << 21) + d - 1) / d) {}
+  __device__ __forceinline__ int quotient(int n) const { return int(__umul24((unsigned)n, m) >> 21); }
+};
+
+// One field's parent window of NT threads into LDS (layout L).  N > 0: the
+// window of N predicted parent cells per axis.  Loads are issued eight at a time.
+template <int NT, int N, typename L>
+__device__ __forceinline__ void stage_window3(double *s, const double *__restrict__ field,
+                                              const Window<3> &win, int tid) {
+  using D = Dims<3>;
+  int const w1 = N ? N + 4 : win.w[1], w2 = N ? N + 4 : win.w[2];
+  int const n = N ? (N + 4) * (N + 4) * (N + 4) : win.w[0] * w1 * w2;
+  SmallDiv const by2(w2), by1(w1);
+  const double *base = field + win.p0[0] * D::SX + win.p0[1] * D::SY + win.p0[2];
+  constexpr int K = 8;
+  for (int first = tid; first < n; first += K * NT) {
+    double v[K];
+    int to[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      int const t = first + k * NT;
+      int const row = N ? t / (N + 4) : by2.quotient(t);
+      int const a = N ? row / (N + 4) : by1.quotient(row);
+      int const b = row - a * w1, c = t - row * w2;
+      to[k] = a * L::SX + b * L::SY + c;
+      if (t < n) v[k] = base[a * D::SX + b * D::SY + c];
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      if (first + k * NT < n) s[to[k]] = v[k];
+  }
+}
+
+// Children of a pair of parent cells (c even) from `q`, the child's cell
+// (2a, 2b, 2c): four adjacent doubles per row, or the first two alone.
+__device__ __forceinline__ void store_pair(double *q, const double (&v)[2][8], bool second) {
+  store_children<3>(q, v[0]);
+  if (second) store_children<3>(q + 2, v[1]);
+}
+
+// One field of one link by NT threads: the window into s, then the pairs of
+// predicted parent cells along z.  N > 0: N predicted cells per axis.
+template <int NT, int W, int N, typename F>
+__device__ __forceinline__ void for_pairs(const Range &r, int tid, const F &f) {
+  using L = LdsW<3, W>;
+  int const c1 = N ? N : r.count[1], pz = N ? N / 2 : (r.count[2] + 1) / 2;
+  int const tasks = N ? N * N * (N / 2) : r.count[0] * c1 * pz;
+  SmallDiv const byz(pz), byy(c1);
+  for (int t = tid; t < tasks; t += NT) {
+    int a, b, c;
+    if constexpr (N == 8 && W == 12) {
+      // Four threads read 16 consecutive banks of a window row; rows b and b + 2
+      // and planes a and a + 1 of this layout lie 16 and 32 banks further, so a
+      // quarter wavefront of these four rows reads without bank conflicts.
+      c = 2 * (t & 3);
+      b = ((t >> 2) & 1) * 2 + ((t >> 4) & 1) + ((t >> 5) & 1) * 4;
+      a = ((t >> 3) & 1) + 2 * (t >> 6);
+    } else {
+      int const q = N ? t / (N / 2) : byz.quotient(t);
+      a = N ? q / N : byy.quotient(q);
+      b = q - a * c1;
+      c = 2 * (t - q * pz);
+    }
+    f(a, b, c, Window<3>::template centre<L>(a, b, c));
+  }
+}
+
+template <int NT, int W, int N>
+__device__ __forceinline__ void predict_field3(double *s, double *__restrict__ blocks,
+                                               const alpaca_mr_link &l, int e, const Range &r,
+                                               int tid) {
+  using D = Dims<3>;
+  using L = LdsW<3, W>;
+  Window<3> const win(r, l.position);
+  double *child = blocks + (size_t)l.child * D::BLOCK + (size_t)e * D::FIELD;
+  // The internal cells of a child row cover its first and last 64-byte segment
+  // in part, and a partial write of a segment that is in no cache is a
+  // read-modify-write in memory, so both are read first (the values are not
+  // used).  2560 links: 343 us without, 303 us with; whole rows would take 177.
+  double edge[2];
+  if constexpr (N == 8) {
+    static_assert(NT == kIC * kIC, "one child row per thread");
+    const double *q = child + (kHS + tid / kIC) * D::SX + (kHS + tid % kIC) * D::SY;
+    edge[0] = q[0];
+    edge[1] = q[kTC - 1];
+  }
+  stage_window3<NT, N, L>(s, blocks + (size_t)l.parent * D::BLOCK + (size_t)e * D::FIELD, win, tid);
+  if constexpr (N == 8) asm volatile("" ::"v"(edge[0]), "v"(edge[1]));
+  __syncthreads();
+  for_pairs<NT, W, N>(r, tid, [&](int a, int b, int c, int o) {
+    double v[2][8];
+    predict_pair<L>(s, o, v);
+    store_pair(child + (r.start[0] + 2 * a) * D::SX + (r.start[1] + 2 * b) * D::SY + r.start[2] + 2 * c,
+               v, c + 1 < r.count[2]);
+  });
+}
+
+// One workgroup per (link, equation), the equations and siblings of a parent
+// on one XCD.  N = 8 (the internal cells): 256 threads, one pair each; N = 12 (the
+// whole block): 448 threads, two each; N = 0: any range.  A workgroup stages one
+// field, so others' arithmetic covers its loads.  Bound by the writes: without
+// them 2560 links' internal cells take 118 us.
+template <int W, int N> constexpr int kPredictThreads = W == 12 ? 256 : 448;
+
+template <int W, int N>
+__global__ __launch_bounds__((kPredictThreads<W, N>)) __attribute__((amdgpu_waves_per_eu(4, 8))) void prediction3_kernel(
+    double *__restrict__ blocks, int nblocks, const alpaca_mr_link *__restrict__ links, Range r) {
+  constexpr int NE = Dims<3>::NE;
+  __shared__ __align__(16) double s[LdsW<3, W>::SIZE];
+  unsigned const g = xcd_remap_group(blockIdx.x, gridDim.x);
+  alpaca_mr_link const l = links[g / NE];
+  if (!link_ok<3>(l, nblocks)) return;
+  if constexpr (N > 0) {
+#pragma unroll
+    for (int a = 0; a < 3; ++a) r.count[a] = N;
+  }
+  predict_field3<kPredictThreads<W, N>, W, N>(s, blocks, l, int(g % NE), r, threadIdx.x);
+}
+
+// The jump halos of 3D links (jump_halo_kernel): a slab has at most 64 pairs of
+// parent cells, so one wavefront per (link, equation).
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void jump_halo3_kernel(double *__restrict__ blocks, int nblocks,
+                                                        const alpaca_mr_link *__restrict__ links,
+                                                        const int *__restrict__ locations) {
+  constexpr int NE = Dims<3>::NE;
+  __shared__ __align__(16) double s[LdsW<3, 12>::SIZE];
+  unsigned const g = xcd_remap_group(blockIdx.x, gridDim.x);
+  alpaca_mr_link const l = links[g / NE];
+  Range r;
+  if (!link_ok<3>(l, nblocks) || !location_range<3>(locations[g / NE], r)) return;
+  predict_field3<64, 12, 0>(s, blocks, l, int(g % NE), r, threadIdx.x);
+}
+
 // ------------------------------------------------------------------ details
 
 struct Thresholds {
@@ -501,84 +725,110 @@ struct Thresholds {
 // L-two sums are reduced as a tree (lanes, then waves) instead of the
 // reference's cell order: they agree to rounding, and a NaN or infinite term
 // gives a NaN or infinite sum either way.
+// The two fields' windows are staged together (64 KB in 3D, two workgroups of
+// seven wavefronts per CU: 3456 children in two pairs of parent cells a thread
+// and field, 96% of the threads at work); a pair's child cells are read before its
+// prediction is formed.
+template <int DIM> constexpr int kDetailThreads = DIM == 3 ? 448 : 192;
+
+// A child's relative detail between its value x and the prediction v.
+template <int NORM> __device__ __forceinline__ void add_detail(double x, double v, double &m, double &acc) {
+  if constexpr (NORM == 0) {
+    m = __builtin_fmax(m, __builtin_fabs(x - v) / __builtin_fabs(x));
+  } else if constexpr (NORM == 1) {
+    acc += __builtin_fabs(x - v) / __builtin_fabs(x);
+  } else {
+    double const q = (x - v) / x;
+    acc = acc + q * q;
+  }
+}
+
 template <int DIM, int NORM>
-__global__ __launch_bounds__(kStencilThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) void details_kernel(
+__global__ __launch_bounds__(kDetailThreads<DIM>) __attribute__((amdgpu_waves_per_eu(4, 8))) void details_kernel(
     const double *__restrict__ blocks, int nblocks, const alpaca_mr_link *__restrict__ links,
     Thresholds th, double *__restrict__ details, int *__restrict__ decisions) {
   using D = Dims<DIM>;
-  constexpr int HZ = DIM == 3 ? kTC / 2 : 1;
-  constexpr int TASKS = (kTC / 2) * (kTC / 2) * HZ;
-  constexpr int kWaves = kStencilThreads / 64;
+  constexpr int NT = kDetailThreads<DIM>;
+  constexpr int H = kTC / 2;
+  constexpr int kWaves = NT / 64;
   constexpr double kOneNumberOfCells = 1.0 / double(kTC * kTC * D::TZ);
-  __shared__ double s[Lds<DIM>::SIZE];
-  // The window's first entries take the per-wave partial results once it is
-  // consumed (one LDS allocation of 32 KiB keeps five workgroups per CU).
-  double *part = s;
-  alpaca_mr_link const l = links[blockIdx.x];
+  __shared__ __align__(16) double s[2][Lds<DIM>::SIZE];
+  __shared__ double part[2][kWaves];
+  unsigned const g = xcd_remap_group(blockIdx.x, gridDim.x);
+  alpaca_mr_link const l = links[g];
   if (!link_ok<DIM>(l, nblocks)) {
     if (threadIdx.x == 0) {
-      details[blockIdx.x] = __builtin_nan("");
-      if (decisions) decisions[blockIdx.x] = -1;
+      details[g] = __builtin_nan("");
+      if (decisions) decisions[g] = -1;
     }
     return;
   }
-  Range const full{{0, 0, 0}, {kTC / 2, kTC / 2, HZ}};
+  Range const full{{0, 0, 0}, {H, H, DIM == 3 ? H : 1}};
   Window<DIM> const win(full, l.position);
-  double m = 0.0;
+#pragma unroll
   for (int e = kMass; e <= kEnergy; ++e) {
-    if (e != kMass) __syncthreads();  // the previous field's window is consumed
-    stage_window<DIM>(s, blocks + (size_t)l.parent * D::BLOCK + (size_t)e * D::FIELD, win);
-    __syncthreads();
+    const double *field = blocks + (size_t)l.parent * D::BLOCK + (size_t)e * D::FIELD;
+    if constexpr (DIM == 3)
+      stage_window3<NT, H, Lds<3>>(s[e], field, win, threadIdx.x);
+    else
+      stage_window<DIM>(s[e], field, win);
+  }
+  __syncthreads();
+  double m = 0.0;
+#pragma unroll 1
+  for (int e = kMass; e <= kEnergy; ++e) {
     const double *child = blocks + (size_t)l.child * D::BLOCK + (size_t)e * D::FIELD;
     double acc = 0.0;
-    for (int t = threadIdx.x; t < TASKS; t += kStencilThreads) {
-      int const a = t / ((kTC / 2) * HZ), b = (t / HZ) % (kTC / 2), c = t % HZ;
-      double v[1 << DIM];
-      predict_cell<DIM>(s, Window<DIM>::centre(a, b, c), v);
-      double x[1 << DIM];
-      load_children<DIM>(child + 2 * a * D::SX + 2 * b * D::SY + (DIM == 3 ? 2 * c : 0), x);
+    if constexpr (DIM == 3) {
+      for_pairs<NT, 16, H>(full, threadIdx.x, [&](int a, int b, int c, int o) {
+        const double *q = child + 2 * a * D::SX + 2 * b * D::SY + 2 * c;
+        double x[2][8], v[2][8];
+        load_children<3>(q, x[0]);
+        load_children<3>(q + 2, x[1]);
+        predict_pair<Lds<3>>(s[e], o, v);
 #pragma unroll
-      for (int n = 0; n < (1 << DIM); ++n) {
-        if constexpr (NORM == 0) {
-          m = __builtin_fmax(m, __builtin_fabs(x[n] - v[n]) / __builtin_fabs(x[n]));
-        } else if constexpr (NORM == 1) {
-          acc += __builtin_fabs(x[n] - v[n]) / __builtin_fabs(x[n]);
-        } else {
-          double const q = (x[n] - v[n]) / x[n];
-          acc = acc + q * q;
-        }
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+          for (int n = 0; n < 8; ++n) add_detail<NORM>(x[k][n], v[k][n], m, acc);
+      });
+    } else {
+      for (int t = threadIdx.x; t < H * H; t += NT) {
+        int const a = t / H, b = t % H;
+        double x[4], v[4];
+        predict_cell(s[e], Window<2>::centre(a, b, 0), v);
+        load_children<2>(child + 2 * a * D::SX + 2 * b * D::SY, x);
+#pragma unroll
+        for (int n = 0; n < 4; ++n) add_detail<NORM>(x[n], v[n], m, acc);
       }
     }
     if constexpr (NORM != 0) {
 #pragma unroll
       for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-      __syncthreads();  // every thread is done with the window
-      if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = acc;
-      __syncthreads();
-      if (threadIdx.x == 0) {
-        double sum = part[0];
-#pragma unroll
-        for (int w = 1; w < kWaves; ++w) sum += part[w];
-        double const val =
-            NORM == 1 ? sum * kOneNumberOfCells : __builtin_sqrt(sum) * kOneNumberOfCells;
-        m = __builtin_fmax(m, val);
-      }
+      if ((threadIdx.x & 63) == 0) part[e][threadIdx.x >> 6] = acc;
     }
   }
   if constexpr (NORM == 0) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) m = __builtin_fmax(m, __shfl_xor(m, off, 64));
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-#pragma unroll
-      for (int w = 1; w < kWaves; ++w) m = __builtin_fmax(m, part[w]);
-      m = __builtin_fmax(part[0], m);
-    }
+    if ((threadIdx.x & 63) == 0) part[0][threadIdx.x >> 6] = m;
   }
+  __syncthreads();
   if (threadIdx.x == 0) {
-    details[blockIdx.x] = m;
+    if constexpr (NORM == 0) {
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) m = __builtin_fmax(part[0][w], m);
+    } else {
+#pragma unroll
+      for (int e = kMass; e <= kEnergy; ++e) {
+        double sum = part[e][0];
+#pragma unroll
+        for (int w = 1; w < kWaves; ++w) sum += part[e][w];
+        double const val =
+            NORM == 1 ? sum * kOneNumberOfCells : __builtin_sqrt(sum) * kOneNumberOfCells;
+        m = __builtin_fmax(m, val);
+      }
+    }
+    details[g] = m;
     if (decisions) {
       int dec = -1;
       if (l.level >= 0 && l.level < th.nlevels) {
@@ -588,7 +838,7 @@ __global__ __launch_bounds__(kStencilThreads) __attribute__((amdgpu_waves_per_eu
         double const eps_refine = eps_coarsen * 32.0;
         dec = m <= eps_coarsen ? 2 : (m >= eps_refine ? 1 : 0);
       }
-      decisions[blockIdx.x] = dec;
+      decisions[g] = dec;
     }
   }
 }
@@ -619,34 +869,51 @@ template <int DIM> int average_jump_impl(double *surfaces, int nblocks, const al
 
 template <int DIM> int prediction_impl(double *blocks, int nblocks, const alpaca_mr_link *links,
                                        int nlinks, const Range &r, hipStream_t s) {
-  dim3 grid((unsigned)nlinks * Dims<DIM>::NE);
-  bool const full = r.start[0] == 0 && r.start[1] == 0 && r.start[2] == 0 &&
-                    r.count[0] == kTC / 2 && r.count[1] == kTC / 2 &&
-                    r.count[2] == (DIM == 3 ? kTC / 2 : 1);
-  if (!full && small_window(r))
+  dim3 const grid((unsigned)nlinks * Dims<DIM>::NE);
+  auto all = [&r](int n) {
+    return r.count[0] == n && r.count[1] == n && r.count[2] == (DIM == 3 ? n : 1);
+  };
+  if constexpr (DIM == 3) {
+    if (all(8) && r.start[0] == kHS && r.start[1] == kHS && r.start[2] == kHS)
+      hipLaunchKernelGGL((prediction3_kernel<12, 8>), grid, dim3(kPredictThreads<12, 8>), 0, s,
+                         blocks, nblocks, links, r);
+    else if (all(12))
+      hipLaunchKernelGGL((prediction3_kernel<16, 12>), grid, dim3(kPredictThreads<16, 12>), 0, s,
+                         blocks, nblocks, links, r);
+    else if (small_window(r))
+      hipLaunchKernelGGL((prediction3_kernel<12, 0>), grid, dim3(kPredictThreads<12, 0>), 0, s,
+                         blocks, nblocks, links, r);
+    else
+      hipLaunchKernelGGL((prediction3_kernel<16, 0>), grid, dim3(kPredictThreads<16, 0>), 0, s,
+                         blocks, nblocks, links, r);
+  } else if (small_window(r)) {
     hipLaunchKernelGGL((prediction_small_kernel<DIM>), dim3((unsigned)nlinks),
                        dim3(kStencilThreads), 0, s, blocks, nblocks, links, r);
-  else if (full)
+  } else if (all(12)) {
     hipLaunchKernelGGL((prediction_kernel<DIM, true>), grid, dim3(kStencilThreads), 0, s, blocks,
                        nblocks, links, r);
-  else
+  } else {
     hipLaunchKernelGGL((prediction_kernel<DIM, false>), grid, dim3(kStencilThreads), 0, s, blocks,
                        nblocks, links, r);
+  }
   return hip_status(hipGetLastError());
 }
 
 template <int DIM> int jump_halo_impl(double *blocks, int nblocks, const alpaca_mr_link *links,
                                       const int *locations, int nlinks, hipStream_t s) {
-  dim3 grid((unsigned)nlinks);
-  hipLaunchKernelGGL((jump_halo_kernel<DIM>), grid, dim3(kStencilThreads), 0, s, blocks, nblocks,
-                     links, locations);
+  if constexpr (DIM == 3)
+    hipLaunchKernelGGL(jump_halo3_kernel, dim3((unsigned)nlinks * Dims<3>::NE), dim3(64), 0, s, blocks,
+                       nblocks, links, locations);
+  else
+    hipLaunchKernelGGL((jump_halo_kernel<DIM>), dim3((unsigned)nlinks), dim3(kStencilThreads), 0, s,
+                       blocks, nblocks, links, locations);
   return hip_status(hipGetLastError());
 }
 
 template <int DIM> int details_impl(const double *blocks, int nblocks, const alpaca_mr_link *links,
                                     int nlinks, int norm, const Thresholds &th, double *details,
                                     int *decisions, hipStream_t s) {
-  dim3 const grid((unsigned)nlinks), block(kStencilThreads);
+  dim3 const grid((unsigned)nlinks), block(kDetailThreads<DIM>);
   if (norm == ALPACA_MR_NORM_L1)
     hipLaunchKernelGGL((details_kernel<DIM, 1>), grid, block, 0, s, blocks, nblocks, links, th,
                        details, decisions);
