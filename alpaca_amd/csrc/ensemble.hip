@@ -82,6 +82,19 @@ __global__ void ens_set_flags_kernel(alpaca_case_state *states, int i, int set, 
 //   3D: 0 = 8x8x8 cells / 256 threads, 1 = 16x8x8 / 512
 //   2D: 0 = 16x16 / 128, 1 = 16x16 / 256, 2 = 16x8 / 128
 template <int DIM> constexpr int num_tiles_configs() { return DIM == 3 ? 2 : 3; }
+// And those the ensemble chooses by itself: 2D: 3 = 8x8 / 256, 4 = 16x8 / 192
+constexpr int kMaxTileConfigs = 5;
+
+// The configuration of an ensemble that was given none, from the blocks it
+// holds: as launch_shapes.h chooses for a single case (whose line for one
+// workgroup per CU does not carry over to several classes at once).  290 blocks
+// in each of two classes, exact and mixed HLLC, side by side: 49 us a stage with
+// configuration 0, 28 to 40 us with 4.
+int auto_tile_config(int dim, long long blocks, long long cus) {
+  if (dim == 3) return 0;
+  if (4 * blocks <= 5 * cus) return 3;
+  return blocks < 6 * cus ? 4 : 0;
+}
 
 template <int DIM, int FLUX, int TX, int TY, int TZ, int NT>
 void launch_batch_tile(int groups, hipStream_t s, const double *avg, const double *init,
@@ -115,6 +128,12 @@ void launch_batch(int tile_config, int groups, hipStream_t s, const double *avg,
                                                          items, n, stage, mode);
     else if (tile_config == 2)
       launch_batch_tile<2, FLUX, 16, 8, 1, 128>(groups, s, avg, init, out, slots, states,
+                                                        items, n, stage, mode);
+    else if (tile_config == 3)
+      launch_batch_tile<2, FLUX, 8, 8, 1, 256>(groups, s, avg, init, out, slots, states,
+                                                       items, n, stage, mode);
+    else if (tile_config == 4)
+      launch_batch_tile<2, FLUX, 16, 8, 1, 192>(groups, s, avg, init, out, slots, states,
                                                         items, n, stage, mode);
     else
       launch_batch_tile<2, FLUX, 16, 16, 1, 128>(groups, s, avg, init, out, slots, states,
@@ -160,11 +179,12 @@ struct alpaca_ensemble {
   std::vector<CaseSlot> h_slots;
   std::vector<alpaca_case_desc> h_desc;
   std::vector<int> h_active;
+  bool tuned = false;  // set_tuning gave the configuration
   int tile_config = 0;
   int groups_per_cu = 0;  // 0: default from occupancy
   int num_cus = 256;
-  hipGraphExec_t exec = nullptr;
-  hipGraph_t graph = nullptr;
+  hipGraphExec_t exec[kMaxTileConfigs] = {};  // the captured step per configuration
+  hipGraph_t graph[kMaxTileConfigs] = {};
   std::mutex mu;
 };
 
@@ -231,7 +251,7 @@ void pool_capacity(alpaca_ensemble *e, int *free_blocks, int *largest) {
 
 int default_groups_per_cu(int dim, int tile_config) {
   if (dim == 3) return tile_config == 1 ? 1 : 2;
-  return tile_config == 1 ? 3 : 6;
+  return tile_config == 1 || tile_config == 3 ? 3 : (tile_config == 4 ? 4 : 6);
 }
 
 int upload_lists(alpaca_ensemble *e) {
@@ -254,23 +274,23 @@ int upload_lists(alpaca_ensemble *e) {
 }
 
 // One class's persistent stage kernel on stream s.
-void launch_class(alpaca_ensemble *e, int c, int groups, hipStream_t s, int stage) {
+void launch_class(alpaca_ensemble *e, int tile_config, int c, int groups, hipStream_t s, int stage) {
   double *const ins[3] = {e->u, e->s1, e->s2};
   double *const outs[3] = {e->s1, e->s2, e->u};
   int const flux = c / 3, mode = c % 3;
   if (e->dim == 3) {
     if (flux == 0)
-      launch_batch<3, 0>(e->tile_config, groups, s, ins[stage], e->u, outs[stage], e->d_slots,
+      launch_batch<3, 0>(tile_config, groups, s, ins[stage], e->u, outs[stage], e->d_slots,
                          e->d_states, e->d_items[c], e->d_counts + c, stage, mode);
     else
-      launch_batch<3, 1>(e->tile_config, groups, s, ins[stage], e->u, outs[stage], e->d_slots,
+      launch_batch<3, 1>(tile_config, groups, s, ins[stage], e->u, outs[stage], e->d_slots,
                          e->d_states, e->d_items[c], e->d_counts + c, stage, mode);
   } else {
     if (flux == 0)
-      launch_batch<2, 0>(e->tile_config, groups, s, ins[stage], e->u, outs[stage], e->d_slots,
+      launch_batch<2, 0>(tile_config, groups, s, ins[stage], e->u, outs[stage], e->d_slots,
                          e->d_states, e->d_items[c], e->d_counts + c, stage, mode);
     else
-      launch_batch<2, 1>(e->tile_config, groups, s, ins[stage], e->u, outs[stage], e->d_slots,
+      launch_batch<2, 1>(tile_config, groups, s, ins[stage], e->u, outs[stage], e->d_slots,
                          e->d_states, e->d_items[c], e->d_counts + c, stage, mode);
   }
 }
@@ -281,8 +301,8 @@ void launch_class(alpaca_ensemble *e, int c, int groups, hipStream_t s, int stag
 // join before the next stage), so one class's tail overlaps the others'
 // work -- then the per-case finish.  Classes touch disjoint cases, so the
 // branches never write the same block.
-int record_step(alpaca_ensemble *e) {
-  int const g0 = e->groups_per_cu > 0 ? e->groups_per_cu : default_groups_per_cu(e->dim, e->tile_config);
+int record_step(alpaca_ensemble *e, int tile_config) {
+  int const g0 = e->groups_per_cu > 0 ? e->groups_per_cu : default_groups_per_cu(e->dim, tile_config);
   int groups = g0 * e->num_cus;
   groups = (groups + 7) / 8 * 8;
   int const nc = e->max_cases;
@@ -298,7 +318,7 @@ int record_step(alpaca_ensemble *e) {
       int const c = cls[i];
       hipStream_t s = i == 0 ? e->stream : e->aux[c];
       if (i > 0 && hipStreamWaitEvent(s, e->fork[stage], 0) != hipSuccess) return ALPACA_ERR_HIP;
-      launch_class(e, c, groups, s, stage);
+      launch_class(e, tile_config, c, groups, s, stage);
       if (i > 0 && hipEventRecord(e->join[stage][c], s) != hipSuccess) return ALPACA_ERR_HIP;
     }
     for (int i = 1; i < ncls; ++i)
@@ -310,27 +330,30 @@ int record_step(alpaca_ensemble *e) {
   return hip_ok(hipGetLastError());
 }
 
-void drop_graph(alpaca_ensemble *e) {
-  if (e->exec) (void)hipGraphExecDestroy(e->exec);
-  if (e->graph) (void)hipGraphDestroy(e->graph);
-  e->exec = nullptr;
-  e->graph = nullptr;
+void drop_graph(alpaca_ensemble *e, int tile_config) {
+  if (e->exec[tile_config]) (void)hipGraphExecDestroy(e->exec[tile_config]);
+  if (e->graph[tile_config]) (void)hipGraphDestroy(e->graph[tile_config]);
+  e->exec[tile_config] = nullptr;
+  e->graph[tile_config] = nullptr;
+}
+void drop_graphs(alpaca_ensemble *e) {
+  for (int t = 0; t < kMaxTileConfigs; ++t) drop_graph(e, t);
 }
 
-int capture_step(alpaca_ensemble *e) {
-  drop_graph(e);
+int capture_step(alpaca_ensemble *e, int tile_config) {
+  drop_graph(e, tile_config);
   if (hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
     return ALPACA_ERR_HIP;
-  int const st = record_step(e);
+  int const st = record_step(e, tile_config);
   hipGraph_t g = nullptr;
   hipError_t const end = hipStreamEndCapture(e->stream, &g);
   if (st != ALPACA_OK || end != hipSuccess) {
     if (g) (void)hipGraphDestroy(g);
     return st != ALPACA_OK ? st : ALPACA_ERR_HIP;
   }
-  e->graph = g;
-  if (hipGraphInstantiate(&e->exec, g, nullptr, nullptr, 0) != hipSuccess) {
-    drop_graph(e);
+  e->graph[tile_config] = g;
+  if (hipGraphInstantiate(&e->exec[tile_config], g, nullptr, nullptr, 0) != hipSuccess) {
+    drop_graph(e, tile_config);
     return ALPACA_ERR_HIP;
   }
   return ALPACA_OK;
@@ -470,7 +493,7 @@ int alpaca_ensemble_create_shared(alpaca_ensemble *peer, int dim, int max_cases,
 int alpaca_ensemble_destroy(alpaca_ensemble *e) {
   if (!e) return ALPACA_ERR_INVALID;
   if (e->stream) (void)hipStreamSynchronize(e->stream);
-  drop_graph(e);
+  drop_graphs(e);
   (void)hipFree(e->d_slots);
   (void)hipFree(e->d_states);
   (void)hipFree(e->d_counts);
@@ -575,11 +598,10 @@ int alpaca_ensemble_set_tuning(alpaca_ensemble *e, int tile_config, int groups_p
   int const ntc = e->dim == 3 ? num_tiles_configs<3>() : num_tiles_configs<2>();
   if (tile_config < 0 || tile_config >= ntc) return ALPACA_ERR_INVALID;
   std::lock_guard<std::mutex> lock(e->mu);
-  if (tile_config != e->tile_config || groups_per_cu != e->groups_per_cu) {
-    e->tile_config = tile_config;
-    e->groups_per_cu = groups_per_cu;
-    drop_graph(e);
-  }
+  if (groups_per_cu != e->groups_per_cu) drop_graphs(e);
+  e->tuned = true;
+  e->tile_config = tile_config;
+  e->groups_per_cu = groups_per_cu;
   return ALPACA_OK;
 }
 
@@ -588,9 +610,12 @@ int alpaca_ensemble_step(alpaca_ensemble *e, int nsteps) {
   std::lock_guard<std::mutex> lock(e->mu);
   int st = upload_lists(e);
   if (st != ALPACA_OK) return st;
-  if (!e->exec && (st = capture_step(e)) != ALPACA_OK) return st;
+  size_t blocks = 0;
+  for (auto const &items : e->h_items) blocks += items.size();
+  int const t = e->tuned ? e->tile_config : auto_tile_config(e->dim, (long long)blocks, e->num_cus);
+  if (!e->exec[t] && (st = capture_step(e, t)) != ALPACA_OK) return st;
   for (int n = 0; n < nsteps; ++n)
-    if (hipGraphLaunch(e->exec, e->stream) != hipSuccess) return ALPACA_ERR_HIP;
+    if (hipGraphLaunch(e->exec[t], e->stream) != hipSuccess) return ALPACA_ERR_HIP;
   return ALPACA_OK;
 }
 
