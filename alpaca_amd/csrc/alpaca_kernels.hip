@@ -723,12 +723,42 @@ void launch_march_kernel(int nblocks, hipStream_t s, const double *avg, const do
 // as evenly: 512 blocks 104 units against 112 (exact 1.50 ms a step against
 // 1.54 ms), but 385 blocks 104 against 91 (FMA 0.84 ms against 0.74 ms), and
 // few blocks never (64: 26 against 14).  The mixed HLLC form keeps the tiles.
+// HLLC with FMA marches from 8 blocks per CU only: below, tiles with 512 threads
+// are faster (512 blocks 290 us a stage against 307 marching, 4096 blocks 2364
+// against 2322).
 template <int FLUX, int MODE>
 constexpr bool kMarches = !(FLUX == ALPACA_FLUX_HLLC && MODE == kModeMixed);
-bool use_march(int nblocks) {
+template <int FLUX, int MODE> bool use_march(int nblocks) {
   long long const cus = device_cus();
+  if (FLUX == ALPACA_FLUX_HLLC && MODE == kModeFma && nblocks < 8 * cus) return false;
   auto rounds = [cus](long long groups) { return (groups + cus - 1) / cus; };
   return rounds(2LL * nblocks) * 26 <= rounds(8LL * nblocks) * 7;
+}
+
+// Whether a 2D case runs on pair_stage_kernel.  Four of its workgroups fill a CU, so
+// it is ahead where the pairs are resident at once or nearly so, and where there
+// are many (exact HLLC, one stage, us, against 16x16 tiles): 1600 blocks 69 and 74,
+// 2025 71 and 91, 2500 90 and 103, 3249 127 and 123, 4900 165 and 170, 16384 529
+// and 550.  The other forms gain at many blocks only (16384: HLLC FMA 307 and
+// 325, mixed 291 and 301, Roe mixed 382 and 396); the Roe form with FMA, whose
+// registers hold 16 wavefronts a CU, loses (534 and 484).
+template <int FLUX, int MODE> bool use_pairs(long long nblocks) {
+  long long const cus = device_cus();
+  if (FLUX == ALPACA_FLUX_ROE && MODE == kModeFma) return false;
+  if (nblocks >= 32 * cus) return true;
+  return MODE == kModeExact && nblocks >= 6 * cus && (nblocks <= 10 * cus || nblocks >= 16 * cus);
+}
+
+template <int FLUX, int MODE>
+void launch_pair_kernel(int nblocks, hipStream_t s, const double *avg, const double *init,
+                        double *out, alpaca_case_state *state, const StageArgs &a) {
+  dim3 const grid((nblocks + 1) / 2), block(exact::kPairThreads);
+  if constexpr (MODE == kModeExact)
+    hipLaunchKernelGGL((exact::pair_stage_kernel<FLUX, double>), grid, block, 0, s, avg, init, out,
+                       state, a);
+  else
+    hipLaunchKernelGGL((fast::pair_stage_kernel<FLUX, std::conditional_t<MODE == kModeMixed, float, double>>),
+                       grid, block, 0, s, avg, init, out, state, a);
 }
 
 template <int DIM, int FLUX, int MODE>
@@ -754,10 +784,16 @@ void launch_stage_fused(const alpaca_case_desc *d, int stage, const double *avg,
   ProfileScope prof(ALPACA_KERNEL_STAGE, s, double(Dims<DIM>::CELLS) * nblocks);
   if constexpr (DIM == 3) {
     if constexpr (kMarches<FLUX, MODE>) {
-      if (use_march(nblocks)) {
+      if (use_march<FLUX, MODE>(nblocks)) {
         launch_march_kernel<FLUX, MODE>(nblocks, s, avg, init, out, state, a);
         return;
       }
+    }
+  }
+  if constexpr (DIM == 2) {
+    if (use_pairs<FLUX, MODE>(nblocks)) {
+      launch_pair_kernel<FLUX, MODE>(nblocks, s, avg, init, out, state, a);
+      return;
     }
   }
   constexpr bool wide = FLUX == ALPACA_FLUX_HLLC && MODE != kModeExact;

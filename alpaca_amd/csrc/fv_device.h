@@ -90,14 +90,15 @@ constexpr int round_up64(int n) { return (n + 63) / 64 * 64; }
 // address lives in scalar registers, a thread passes one byte offset in a
 // VGPR and the field/stencil part as a scalar offset, so an access costs no
 // 64-bit address arithmetic.  The block pointer must be uniform over the
-// wavefront.  num_records is the block's size in bytes; every offset the
+// wavefront.  num_records is the block's size in bytes (in 2D of two blocks: a
+// wavefront of pair_stage_kernel may read from both); every offset the
 // kernels form stays inside it, and voffset and soffset are never negative.
 template <int DIM> struct BlockReader {
   __amdgpu_buffer_rsrc_t r;
   typedef unsigned int u2 __attribute__((ext_vector_type(2)));
   __device__ __forceinline__ explicit BlockReader(const double *blk)
       : r(__builtin_amdgcn_make_buffer_rsrc(const_cast<double *>(blk), (short)0,
-                                            (int)(Dims<DIM>::BLOCK * sizeof(double)),
+                                            (int)((DIM == 2 ? 2 : 1) * Dims<DIM>::BLOCK * sizeof(double)),
                                             0x00020000)) {}
   __device__ __forceinline__ double operator()(int voffset_bytes, int soffset_bytes) const {
     u2 const v = __builtin_amdgcn_raw_buffer_load_b64(r, voffset_bytes, soffset_bytes, 0);

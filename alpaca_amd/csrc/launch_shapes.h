@@ -20,11 +20,11 @@ template <int X, int Y, int Z, int N> struct ShapeTag {
 // and there the large tile wins, which computes the fewest shared faces twice and
 // wastes the fewest lanes of its wavefronts' last faces.  Lines in multiples
 // of the compute units, measured with 256 (one stage, exact HLLC, us):
-//   2D blocks           6    64   100   150   225   300   529  1035  1600  9025
+//   2D blocks           6    64   100   150   225   300   529  1035  1521  9025
 //     8x8   256 thr   7.9   8.3  11.7  14.7  18.0  21.1  33.5  58.5  83.9   453
 //     16x16 640      14.2  14.4  14.7  15.1  15.3  27.1  39.1  65.2  90.6   486
 //     16x8  192      11.6  12.0  12.1  18.7  18.7  24.3  30.8  50.0  68.7   358
-//     16x16 128      25.5  26.0  26.1  25.9  26.1  40.0  42.2  58.4  75.2   328
+//     16x16 128      25.5  26.0  26.1  25.9  26.1  40.0  42.2  58.4  59.9   328
 //   3D blocks           2     8    12    24    48    64   128   512
 //     4x4x4 384      12.8  24.4  35.6  67.0   130   173   344  1437
 //     8x4x4 576      18.7  20.6  37.1  54.3   105   138   267  1142
@@ -44,7 +44,7 @@ template <int DIM, typename F> void with_shape(long long n, long long cus, bool 
       f(ShapeTag<16, 16, 1, 640>{});  // one workgroup per CU, one face per thread
     else if (4 * n <= 5 * cus)
       f(ShapeTag<8, 8, 1, 256>{});
-    else if (n < 6 * cus)  // fewer 16x16 tiles than fit the chip at once
+    else if (2 * n < 9 * cus)
       f(ShapeTag<16, 8, 1, 192>{});
     else
       f(ShapeTag<16, 16, 1, 128>{});

@@ -588,6 +588,67 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMinWaves<3
   stage_march<FLUX, R>(j, blk, g % SLABS, lds);
 }
 
+// Large 2D cases: one workgroup of 192 threads per two blocks adjacent in
+// memory.  A block has 272 faces per direction, 4.25 wavefronts, so a block by itself
+// takes 10 units of 64 faces; two take 18, six for each of three wavefronts, and
+// the four workgroups that the LDS of a CU holds are the 12 wavefronts its
+// registers hold.  A wavefront's faces may lie in both blocks, its cells lie in one.
+// 2048^2 cells, one stage: exact HLLC 550 -> 529 us against a block per workgroup,
+// exact Roe 806 -> 755 us.
+constexpr int kPairThreads = 192;
+
+template <int FLUX, typename R>
+__global__ __launch_bounds__(kPairThreads) __attribute__((amdgpu_waves_per_eu(kMinWaves<2, FLUX, R>, 8))) void pair_stage_kernel(
+    const double *__restrict__ avg, const double *init, double *out, alpaca_case_state *state,
+    StageArgs a) {
+  using D = Dims<2>;
+  constexpr int NE = D::NE, NT = kPairThreads;
+  constexpr int NF = (kIC + 1) * kIC;  // faces of a block per direction
+  constexpr int P = round_up64(2 * NF);
+  __shared__ R lds[2 * NE * 2 * NF];
+  R *FX = lds, *FY = lds + NE * 2 * NF;
+  int const pair = 2 * int(xcd_remap_group(blockIdx.x, gridDim.x));
+  if (pair >= a.nblocks) return;  // uniform over the workgroup
+  if (a.guard && (state->flags & kFlagDone)) return;
+  TileJob const j = stage_job(avg, init, out, state, a);
+  int const faces = pair + 1 < a.nblocks ? 2 * NF : NF;
+  const double *bb = avg + (size_t)pair * D::BLOCK;
+  FormedQ<2, R> const qs{a.gamma, a.b};
+  for (int f = threadIdx.x; f < 2 * P; f += NT) {
+    bool const y = f >= P;  // uniform over the wavefront
+    int const r = y ? f - P : f;
+    if (r >= faces) continue;
+    int const second = r >= NF, q = second ? r - NF : r;
+    R fl[NE];
+    if (!y) {  // [17][16]
+      int const off = (q / kIC + kHS - 1) * D::SX + (q % kIC + kHS) * D::SY;
+      face_flux<2, 0, FLUX, R>(a.gamma, a.b, bb, off + second * D::BLOCK, qs, fl);
+    } else {  // [16][17]
+      int const off = (q / (kIC + 1) + kHS) * D::SX + (q % (kIC + 1) + kHS - 1) * D::SY;
+      face_flux<2, 1, FLUX, R>(a.gamma, a.b, bb, off + second * D::BLOCK, qs, fl);
+    }
+    R *o = (y ? FY : FX) + r;
+#pragma unroll
+    for (int e = 0; e < NE; ++e) o[e * 2 * NF] = fl[e];
+  }
+  __syncthreads();
+  double sig = 0.0;
+  bool bad = false;
+  int const cells = faces / NF * D::CELLS;
+  for (int c = threadIdx.x; c < cells; c += NT) {
+    int const second = __builtin_amdgcn_readfirstlane(c / D::CELLS);
+    int const ii = c / kIC % kIC, jj = c % kIC;
+    int const c3[3] = {ii, jj, 0};
+    const R *fx = FX + second * NF + ii * kIC + jj, *fy = FY + second * NF + ii * (kIC + 1) + jj;
+    auto diff = [&](int e, double &dX, double &dY, double &) {
+      dX = double(fx[e * 2 * NF]) - double(fx[e * 2 * NF + kIC]);
+      dY = double(fy[e * 2 * NF]) - double(fy[e * 2 * NF + 1]);
+    };
+    stage_cell<2>(j, StageStep(j, pair + second), pair + second, c3, diff, sig, bad);
+  }
+  stage_finish<NT>(j, sig, bad);
+}
+
 // Right-hand side of n blocks (SpaceSolver::UpdateFluxes, space_solver.cpp:
 // 50-182): those listed of a pool, or, without a list, blocks 0 .. n-1.  One
 // workgroup per (block, tile): the tile's faces into LDS, those on the block's
