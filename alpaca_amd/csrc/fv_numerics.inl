@@ -419,8 +419,8 @@ struct Weno5 {
 // the exact form.  Returns whether every x_k was in the core's range; l[0..4]
 // and r[1..5] are then finite.  PAIRED: one range check for both; otherwise
 // one after the other.  The split decides what the register allocator holds
-// at once: the flux-splitting face (two projections per field) takes 207 VGPRs
-// paired and 256 in sequence, the finite-volume face (one) 241 and 224.
+// at once (the finite-volume face, with one projection per field, takes 241 VGPRs
+// paired and 224 in sequence).
 template <bool PAIRED>
 __device__ __forceinline__ bool weno_pair_exact(const double *l, const double *r, double &left,
                                                 double &right) {
@@ -818,20 +818,20 @@ __device__ __forceinline__ void advection(const double *c, const Prim<double> &p
 // exact FP64 form (flux_splitting_scheme.cpp:42-76, 185-315), added into f.
 // Every value is formed by the reference's operations in the reference's
 // order; only the time at which each is formed differs, which without
-// contraction changes no bit.  To keep two waves per SIMD the face is
-// processed in a fixed sequence with few values live: the eigensystem of
-// cells i and i+1, then the advection of the six stencil cells one cell at a
-// time (kept in registers), then field by field the characteristic
-// projections and WENO5, with the conservatives read again from the block for
-// each field (the L1 and L2 serve the re-reads).  The reads go through a
-// buffer resource (no address arithmetic).  Each group of reads (and each
-// field's row of L) takes its inputs through an empty asm statement that
-// also consumes the previous group's last result, so the compiler neither
-// merges the re-reads nor hoists one field's work above the previous one's:
-// left to itself it forms the products of all fields at once and needs
-// about 340 registers (one wave per SIMD).
-constexpr int kRoePrefetch = 2;  // stencil cells read ahead for the next field
-
+// contraction changes no bit.  The eigensystem of cells i and i+1, then the stencil
+// cell by cell: its conservatives (read one cell ahead, through a buffer
+// resource: no address arithmetic), its advection and its projections onto every
+// field, then WENO5 field by field.  The projections are what is held, 60 doubles in
+// 3D, beside L; empty asm statements make each cell's be formed before the next
+// cell's and each field's reconstruction before the next field's, so that two
+// wavefronts per SIMD fit (left to itself the compiler forms the products of all
+// cells at once).  Field by field, with the stencil read again for each
+// field, a face had 220 reads instead of 40 and waited for them 29% of the
+// time: 128^3, one step, 2778 -> 1892 us; 24 blocks, two steps, 338 -> 262 us.
+// The shear rows of L leave their structural zeros out: a sum that starts at 0.0 is
+// never -0, so a zero product changes it only where a stencil value is not
+// finite (0 * x is then NaN).  Row 0 is dense, so if its reconstruction stayed in the
+// core's range, every value is finite; otherwise the zero products are added.
 template <int DIM, int DIR, typename QS>
 __device__ __forceinline__ void roe_split_flux_exact(double gamma, double b,
                                                      const double *__restrict__ blk, int off,
@@ -841,94 +841,89 @@ __device__ __forceinline__ void roe_split_flux_exact(double gamma, double b,
   BlockReader<DIM> const rd(blk);
   // Byte offset of stencil cell 0 (cell i-2, inside the haloed block).
   int const off0 = (off - 2 * S) * (int)sizeof(double);
-  auto at = [&rd](int o, int m, int e) {
-    return rd(o, (e * Dims<DIM>::FIELD + m * S) * (int)sizeof(double));
+  auto read = [&rd](int o, int m, double *c) {
+#pragma unroll
+    for (int e = 0; e < NE; ++e) c[e] = rd(o, (e * Dims<DIM>::FIELD + m * S) * (int)sizeof(double));
   };
   Eig<NE, double> ev;
   {
     double Ui[NE], Un[NE];
-#pragma unroll
-    for (int e = 0; e < NE; ++e) {
-      Ui[e] = at(off0, 2, e);
-      Un[e] = at(off0, 3, e);
-    }
+    read(off0, 2, Ui);
+    read(off0, 3, Un);
     roe_eigensystem<DIM, DIR, double, true>(gamma, qs.left(Ui), qs.right(Un), ev);
   }
-  double dep = ev.lam[0];
-  double adv[6][NE];
-#pragma unroll
-  for (int m = 0; m < 6; ++m) {
-    int o = off0;
-    asm volatile("" : "+v"(o) : "v"(dep));
-    double U[NE];
-#pragma unroll
-    for (int e = 0; e < NE; ++e) U[e] = at(o, m, e);
-    Prim<double> P;
-    cons_to_prim<DIM, double>(gamma, b, U, P);
-    advection<DIM, DIR>(U, P, adv[m]);
-    dep = adv[m][NE - 1];
-  }
-  // Conservatives of the stencil for the field being projected; the first
-  // kRoePrefetch cells of the next field are read while this field's WENO5
-  // runs, the rest after it.
-  double U[6][NE];
+  double pos[NE][6], neg[NE][6];
+  double dep = ev.lam[0], U[NE], ahead[NE];
   {
     int o = off0;
     asm volatile("" : "+v"(o) : "v"(dep));
-#pragma unroll
-    for (int m = 0; m < 6; ++m)
-#pragma unroll
-      for (int e = 0; e < NE; ++e) U[m][e] = at(o, m, e);
+    read(o, 0, ahead);
   }
-  double chf[NE];
 #pragma unroll
-  for (int n = 0; n < NE; ++n) {
-    // The field's row of L and its eigenvalue pass through an asm statement
-    // that consumes the previous field's result, so no product of this field
-    // is formed before the previous field is done.
-    double lam = ev.lam[n], Lr[5];
+  for (int m = 0; m < 6; ++m) {
 #pragma unroll
-    for (int l = 0; l < NE; ++l) Lr[l] = ev.L[n][l];
-    if constexpr (NE == 5)
-      asm volatile("" : "+v"(lam), "+v"(Lr[0]), "+v"(Lr[1]), "+v"(Lr[2]), "+v"(Lr[3]),
-                   "+v"(Lr[4]) : "v"(dep));
-    else
-      asm volatile("" : "+v"(lam), "+v"(Lr[0]), "+v"(Lr[1]), "+v"(Lr[2]), "+v"(Lr[3])
-                   : "v"(dep));
-    double pos[6], neg[6];
+    for (int e = 0; e < NE; ++e) U[e] = ahead[e];
+    if (m < 5) {
+      int o = off0;
+      asm volatile("" : "+v"(o) : "v"(dep));
+      read(o, m + 1, ahead);
+    }
+    Prim<double> P;
+    cons_to_prim<DIM, double>(gamma, b, U, P);
+    double adv[NE];
+    advection<DIM, DIR>(U, P, adv);
 #pragma unroll
-    for (int m = 0; m < 6; ++m) {
+    for (int n = 0; n < NE; ++n) {
       double sp = 0.0, sn = 0.0;
 #pragma unroll
       for (int q = 0; q < NE; ++q) {
         int const l = seq<DIM, DIR>(q);
-        double const uct = U[m][l] * Lr[l];
-        double const act = adv[m][l] * Lr[l];
-        sp += (act + lam * uct);
-        sn += (act - lam * uct);
+        if (left_zero<DIM, DIR>(n, l)) continue;
+        double const uct = U[l] * ev.L[n][l];
+        double const act = adv[l] * ev.L[n][l];
+        sp += (act + ev.lam[n] * uct);
+        sn += (act - ev.lam[n] * uct);
       }
-      pos[m] = sp;
-      neg[m] = sn;
+      pos[n][m] = sp;
+      neg[n][m] = sn;
     }
-    if (n + 1 < NE) {
-      int o = off0;
-      asm volatile("" : "+v"(o) : "v"(pos[5]), "v"(neg[5]));
 #pragma unroll
-      for (int m = 0; m < kRoePrefetch; ++m)
+    for (int n = 0; n < NE; ++n) asm volatile("" : "+v"(pos[n][m]), "+v"(neg[n][m]));
+    dep = neg[NE - 1][m];
+  }
+  double chf[NE];
 #pragma unroll
-        for (int e = 0; e < NE; ++e) U[m][e] = at(o, m, e);
-    }
+  for (int n = 0; n < NE; ++n) {
     double wl, wr;
-    weno_pair<double>(pos, neg, wl, wr);
+    bool const core = weno_pair_exact<true>(pos[n], neg[n], wl, wr);
     chf[n] = 0.5 * (wl + wr);
-    dep = chf[n];
+    if (n == 0 && __builtin_expect(!core, 0)) {
+#pragma unroll 1
+      for (int m = 0; m < 6; ++m) {
+        int o = off0 + m * S * (int)sizeof(double);
+        double c[NE], adv[NE];
+        read(o, 0, c);
+        Prim<double> P;
+        cons_to_prim<DIM, double>(gamma, b, c, P);
+        advection<DIM, DIR>(c, P, adv);
+#pragma unroll
+        for (int k = 1; k < DIM; ++k) {
+          double z = 0.0;
+#pragma unroll
+          for (int l = 0; l < NE; ++l)
+            if (left_zero<DIM, DIR>(k, l)) z += adv[l] * 0.0 + ev.lam[k] * (c[l] * 0.0);
+#pragma unroll
+          for (int i = 0; i < 6; ++i) {
+            pos[k][i] += i == m ? z : 0.0;
+            neg[k][i] += i == m ? z : 0.0;
+          }
+        }
+      }
+    }
     if (n + 1 < NE) {
-      int o = off0;
-      asm volatile("" : "+v"(o) : "v"(dep));
 #pragma unroll
-      for (int m = kRoePrefetch; m < 6; ++m)
-#pragma unroll
-        for (int e = 0; e < NE; ++e) U[m][e] = at(o, m, e);
+      for (int m = 0; m < 6; ++m)
+        asm volatile("" : "+v"(pos[n + 1][m]), "+v"(neg[n + 1][m]) : "v"(chf[n]));
     }
   }
   roe_right_eigenvectors<DIM, DIR, double, true>(ev);

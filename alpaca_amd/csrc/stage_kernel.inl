@@ -520,15 +520,12 @@ __device__ __forceinline__ void stage_march(const TileJob &j, int blk_local, int
   stage_finish<P>(j, sig, bad);
 }
 
-// Waves per SIMD the register allocator is held to in the single-case
-// kernel.  The exact FP64 2D HLLC kernel needs 178 VGPRs unconstrained (2
-// waves); held to 168 it fits 3 waves with 12 spilled registers (2048^2
-// cells: 2.16e9 -> 2.36e9 cell-updates/s).  The persistent batch kernel
-// spills 34-64 registers under the same hold and runs slower with it, so it
-// and every other variant keep the default.
+// Waves per SIMD the register allocator is held to.  The exact FP64 2D kernels
+// fit 3 waves without spilling; the exact 3D flux-splitting kernels need 211
+// to 217 VGPRs (2 waves).
 template <int DIM, int FLUX, typename R>
-constexpr int kMinWaves = (DIM == 2 && FLUX == 0 && !kFastArith && std::is_same<R, double>::value) ? 3
-                          : (FLUX == 1 && !kFastArith && std::is_same<R, double>::value) ? 2 : 1;
+constexpr int kMinWaves = kFastArith || !std::is_same<R, double>::value ? 1
+                          : DIM == 2 ? 3 : (FLUX == 1 ? 2 : 1);
 
 // The persistent batch kernel: as above.
 template <int DIM, int FLUX, typename R>
