@@ -339,7 +339,8 @@ __global__ __launch_bounds__(kThreads) void halo_list_kernel(double *blocks, int
 template <int DIM>
 __global__ __launch_bounds__(kThreads) void signal_kernel(const double *__restrict__ in, int nblocks,
                                                           double gamma, double b,
-                                                          alpaca_case_state *state, BlockList list) {
+                                                          alpaca_case_state *state, BlockList list,
+                                                          double *partials) {
   using D = Dims<DIM>;
   constexpr int NE = D::NE;
   constexpr int ICZ = D::ICZ;
@@ -375,7 +376,10 @@ __global__ __launch_bounds__(kThreads) void signal_kernel(const double *__restri
     double m = part[0];
 #pragma unroll
     for (int w = 1; w < kThreads / 64; ++w) m = exact::smax(m, part[w]);
-    exact::raise_signal(state, m);
+    if (partials)
+      partials[blockIdx.x] = m;
+    else
+      exact::raise_signal(state, m);
   }
 }
 
@@ -399,12 +403,31 @@ __device__ __forceinline__ void finish_step(alpaca_case_state &r) {
   if (!(r.time < r.t_end)) r.flags |= kFlagDone;
 }
 
+// The larger of the record's signal and the n partial signals of the launch
+// before, by one workgroup of kReduceThreads; thread 0 gets it.
+constexpr int kReduceThreads = 512;
+__device__ __forceinline__ void take_partials(alpaca_case_state &r, const double *partials, int n) {
+  __shared__ double part[kReduceThreads / 64];
+  double s = 0.0;
+  for (int t = threadIdx.x; t < n; t += kReduceThreads) s = exact::smax(s, partials[t]);
+  s = exact::wave_max64(s);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kReduceThreads / 64; ++w) s = exact::smax(s, part[w]);
+  r.smax = (uint64_t)__double_as_longlong(
+      exact::smax(__longlong_as_double((long long)r.smax), s));
+}
+
 // The kernels that change the record read and write it as a whole, in one
 // round trip to memory; they follow the launches that raise smax or set flags.
-__global__ void dt_kernel(alpaca_case_state *state, double cell_size, int guard = 0) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__global__ __launch_bounds__(kReduceThreads) void dt_kernel(alpaca_case_state *state,
+                                                            double cell_size, int guard,
+                                                            const double *partials, int n) {
   alpaca_case_state r = *state;
   if (guard && (r.flags & kFlagDone)) return;
+  take_partials(r, partials, n);
+  if (threadIdx.x != 0) return;
   next_dt(r, cell_size);
   *state = r;
 }
@@ -483,10 +506,14 @@ __global__ void finish_step_kernel(alpaca_case_state *state, int guard = 0) {
 // finish_step_kernel followed by dt_kernel for the next step, both guarded,
 // in one launch (the same operations on the record in the same order): the
 // step boundary inside alpaca_advance.
-__global__ void finish_and_dt_kernel(alpaca_case_state *state, double cell_size) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+__global__ __launch_bounds__(kReduceThreads) void finish_and_dt_kernel(alpaca_case_state *state,
+                                                                       double cell_size,
+                                                                       const double *partials,
+                                                                       int n) {
   alpaca_case_state r = *state;
-  if (r.flags & kFlagDone) return;
+  if (r.flags & kFlagDone) return;  // the same for all threads
+  take_partials(r, partials, n);
+  if (threadIdx.x != 0) return;
   finish_step(r);
   if (!(r.flags & kFlagDone)) next_dt(r, cell_size);
   *state = r;
@@ -702,7 +729,7 @@ void launch_stage_kernel(dim3 grid, hipStream_t s, const double *avg, const doub
 
 // The same by plane marching (3D).
 template <int FLUX, int MODE>
-void launch_march_kernel(int nblocks, hipStream_t s, const double *avg, const double *init,
+unsigned launch_march_kernel(int nblocks, hipStream_t s, const double *avg, const double *init,
                          double *out, alpaca_case_state *state, const StageArgs &a) {
   using R = std::conditional_t<MODE == kModeMixed, float, double>;
   using M = exact::MarchShape<R>;
@@ -713,6 +740,7 @@ void launch_march_kernel(int nblocks, hipStream_t s, const double *avg, const do
   else
     hipLaunchKernelGGL((fast::march_stage_kernel<FLUX, R>), grid, block, 0, s, avg, init, out, state,
                        a);
+  return grid.x;
 }
 
 // Whether a 3D case marches (march_stage_kernel) or runs on 8^3 tiles.  Both
@@ -750,7 +778,7 @@ template <int FLUX, int MODE> bool use_pairs(long long nblocks) {
 }
 
 template <int FLUX, int MODE>
-void launch_pair_kernel(int nblocks, hipStream_t s, const double *avg, const double *init,
+unsigned launch_pair_kernel(int nblocks, hipStream_t s, const double *avg, const double *init,
                         double *out, alpaca_case_state *state, const StageArgs &a) {
   dim3 const grid((nblocks + 1) / 2), block(exact::kPairThreads);
   if constexpr (MODE == kModeExact)
@@ -759,12 +787,15 @@ void launch_pair_kernel(int nblocks, hipStream_t s, const double *avg, const dou
   else
     hipLaunchKernelGGL((fast::pair_stage_kernel<FLUX, std::conditional_t<MODE == kModeMixed, float, double>>),
                        grid, block, 0, s, avg, init, out, state, a);
+  return grid.x;
 }
 
+// Returns the number of workgroups, which is that of the partial signals.
 template <int DIM, int FLUX, int MODE>
-void launch_stage_fused(const alpaca_case_desc *d, int stage, const double *avg,
+unsigned launch_stage_fused(const alpaca_case_desc *d, int stage, const double *avg,
                         const double *init, double *out, double *init_copy,
-                        alpaca_case_state *state, int signal, hipStream_t s, bool guard) {
+                        alpaca_case_state *state, int signal, double *partials, hipStream_t s,
+                        bool guard) {
   int const nblocks = case_blocks(d);
   StageArgs a;
   a.nb[0] = d->nb[0];
@@ -779,52 +810,51 @@ void launch_stage_fused(const alpaca_case_desc *d, int stage, const double *avg,
   a.nblocks = nblocks;
   a.stage = stage;
   a.signal = signal;
+  a.partials = partials;
   a.guard = guard;
   a.init_copy = init_copy;
   ProfileScope prof(ALPACA_KERNEL_STAGE, s, double(Dims<DIM>::CELLS) * nblocks);
   if constexpr (DIM == 3) {
     if constexpr (kMarches<FLUX, MODE>) {
       if (use_march<FLUX, MODE>(nblocks)) {
-        launch_march_kernel<FLUX, MODE>(nblocks, s, avg, init, out, state, a);
-        return;
+        return launch_march_kernel<FLUX, MODE>(nblocks, s, avg, init, out, state, a);
       }
     }
   }
   if constexpr (DIM == 2) {
     if (use_pairs<FLUX, MODE>(nblocks)) {
-      launch_pair_kernel<FLUX, MODE>(nblocks, s, avg, init, out, state, a);
-      return;
+      return launch_pair_kernel<FLUX, MODE>(nblocks, s, avg, init, out, state, a);
     }
   }
   constexpr bool wide = FLUX == ALPACA_FLUX_HLLC && MODE != kModeExact;
+  unsigned groups = 0;
   with_shape<DIM>(nblocks, device_cus(), wide, [&](auto shape) {
     using S = decltype(shape);
     constexpr int tiles = exact::TileShape<DIM, S::TX, S::TY, S::TZ>::TILES;
-    launch_stage_kernel<DIM, FLUX, MODE, S::TX, S::TY, S::TZ, S::NT>(dim3(nblocks * tiles), s, avg,
-                                                                     init, out, state, a);
+    groups = unsigned(nblocks) * tiles;
+    launch_stage_kernel<DIM, FLUX, MODE, S::TX, S::TY, S::TZ, S::NT>(dim3(groups), s, avg, init, out,
+                                                                     state, a);
   });
+  return groups;
 }
 
 template <int DIM>
-void stage_fused(const alpaca_case_desc *d, int stage, const double *avg, const double *init,
+unsigned stage_fused(const alpaca_case_desc *d, int stage, const double *avg, const double *init,
                  double *out, double *init_copy, alpaca_case_state *state, int signal,
-                 hipStream_t s, bool guard = false) {
+                 hipStream_t s, bool guard = false, double *partials = nullptr) {
   int const p = d->precision;
   if (d->flux == ALPACA_FLUX_HLLC) {
     if (p == ALPACA_MIXED)
-      launch_stage_fused<DIM, ALPACA_FLUX_HLLC, kModeMixed>(d, stage, avg, init, out, init_copy, state, signal, s, guard);
-    else if (p == ALPACA_FP64_FMA)
-      launch_stage_fused<DIM, ALPACA_FLUX_HLLC, kModeFma>(d, stage, avg, init, out, init_copy, state, signal, s, guard);
-    else
-      launch_stage_fused<DIM, ALPACA_FLUX_HLLC, kModeExact>(d, stage, avg, init, out, init_copy, state, signal, s, guard);
-  } else {
-    if (p == ALPACA_MIXED)
-      launch_stage_fused<DIM, ALPACA_FLUX_ROE, kModeMixed>(d, stage, avg, init, out, init_copy, state, signal, s, guard);
-    else if (p == ALPACA_FP64_FMA)
-      launch_stage_fused<DIM, ALPACA_FLUX_ROE, kModeFma>(d, stage, avg, init, out, init_copy, state, signal, s, guard);
-    else
-      launch_stage_fused<DIM, ALPACA_FLUX_ROE, kModeExact>(d, stage, avg, init, out, init_copy, state, signal, s, guard);
+      return launch_stage_fused<DIM, ALPACA_FLUX_HLLC, kModeMixed>(d, stage, avg, init, out, init_copy, state, signal, partials, s, guard);
+    if (p == ALPACA_FP64_FMA)
+      return launch_stage_fused<DIM, ALPACA_FLUX_HLLC, kModeFma>(d, stage, avg, init, out, init_copy, state, signal, partials, s, guard);
+    return launch_stage_fused<DIM, ALPACA_FLUX_HLLC, kModeExact>(d, stage, avg, init, out, init_copy, state, signal, partials, s, guard);
   }
+  if (p == ALPACA_MIXED)
+    return launch_stage_fused<DIM, ALPACA_FLUX_ROE, kModeMixed>(d, stage, avg, init, out, init_copy, state, signal, partials, s, guard);
+  if (p == ALPACA_FP64_FMA)
+    return launch_stage_fused<DIM, ALPACA_FLUX_ROE, kModeFma>(d, stage, avg, init, out, init_copy, state, signal, partials, s, guard);
+  return launch_stage_fused<DIM, ALPACA_FLUX_ROE, kModeExact>(d, stage, avg, init, out, init_copy, state, signal, partials, s, guard);
 }
 
 template <int DIM>
@@ -851,14 +881,16 @@ int halo_table_impl(double *blocks, int nblocks, const int *nbr, const SideBc &b
 
 template <int DIM>
 int timestep_impl(const alpaca_case_desc *d, const double *avg, alpaca_case_state *state,
-                  hipStream_t s, int nblocks, BlockList list = {}, int guard = 0) {
+                  hipStream_t s, int nblocks, BlockList list = {}, int guard = 0,
+                  double *partials = nullptr) {
   ProfileScope prof(ALPACA_KERNEL_TIMESTEP, s, double(Dims<DIM>::CELLS) * nblocks);
   // Eight workgroups of four wavefronts fill a CU.
   long long const chunks = (long long)nblocks * (Dims<DIM>::CELLS / kThreads);
   unsigned const groups = (unsigned)std::min<long long>(chunks, 8LL * device_cus());
   hipLaunchKernelGGL((signal_kernel<DIM>), dim3(groups), dim3(kThreads), 0, s, avg, nblocks,
-                     d->gamma, d->background_pressure, state, list);
-  hipLaunchKernelGGL(dt_kernel, dim3(1), dim3(64), 0, s, state, d->cell_size, guard);
+                     d->gamma, d->background_pressure, state, list, partials);
+  hipLaunchKernelGGL(dt_kernel, dim3(1), dim3(kReduceThreads), 0, s, state, d->cell_size, guard,
+                     partials, partials ? (int)groups : 0);
   return hip_status(hipGetLastError());
 }
 
@@ -1232,27 +1264,30 @@ int alpaca_advance(const alpaca_case_desc *desc, double *d_u, double *d_s1, doub
     return ALPACA_ERR_INVALID;
   hipStream_t s = static_cast<hipStream_t>(stream);
   // The first step reduces the CFL signal of d_u; later steps take it from the
-  // last stage of the step before.
+  // last stage of the step before.  Both launches leave a partial signal per
+  // workgroup in d_s1, which holds nothing then (stage 0 writes every value of it
+  // that is read), for the record kernel that follows: no atomics on the record.
+  double *const partials = d_s1;
+  bool const two = desc->dim == 2;
   if (nsteps > 0) {
-    st = desc->dim == 2 ? timestep_impl<2>(desc, d_u, d_state, s, case_blocks(desc), {}, 1)
-                        : timestep_impl<3>(desc, d_u, d_state, s, case_blocks(desc), {}, 1);
+    st = two ? timestep_impl<2>(desc, d_u, d_state, s, case_blocks(desc), {}, 1, partials)
+             : timestep_impl<3>(desc, d_u, d_state, s, case_blocks(desc), {}, 1, partials);
     if (st != ALPACA_OK) return st;
   }
+  auto stage = [&](int i, const double *in, const double *init, double *out, int signal) {
+    return two ? stage_fused<2>(desc, i, in, init, out, nullptr, d_state, signal, s, true, partials)
+               : stage_fused<3>(desc, i, in, init, out, nullptr, d_state, signal, s, true, partials);
+  };
   // Steps once the record is done (its time reached t_end) do nothing: a run
   // can be advanced in chunks of steps with one read-back per chunk.
   for (int n = 0; n < nsteps; ++n) {
     bool const signal = n + 1 < nsteps;
-    if (desc->dim == 2) {
-      stage_fused<2>(desc, 0, d_u, nullptr, d_s1, nullptr, d_state, 0, s, true);
-      stage_fused<2>(desc, 1, d_s1, d_u, d_s2, nullptr, d_state, 0, s, true);
-      stage_fused<2>(desc, 2, d_s2, d_u, d_u, nullptr, d_state, signal, s, true);
-    } else {
-      stage_fused<3>(desc, 0, d_u, nullptr, d_s1, nullptr, d_state, 0, s, true);
-      stage_fused<3>(desc, 1, d_s1, d_u, d_s2, nullptr, d_state, 0, s, true);
-      stage_fused<3>(desc, 2, d_s2, d_u, d_u, nullptr, d_state, signal, s, true);
-    }
+    stage(0, d_u, nullptr, d_s1, 0);
+    stage(1, d_s1, d_u, d_s2, 0);
+    unsigned const groups = stage(2, d_s2, d_u, d_u, signal);
     if (signal)  // this step's end and the next step's dt
-      hipLaunchKernelGGL(finish_and_dt_kernel, dim3(1), dim3(64), 0, s, d_state, desc->cell_size);
+      hipLaunchKernelGGL(finish_and_dt_kernel, dim3(1), dim3(kReduceThreads), 0, s, d_state,
+                         desc->cell_size, partials, (int)groups);
     else
       hipLaunchKernelGGL(finish_step_kernel, dim3(1), dim3(64), 0, s, d_state, 1);
   }

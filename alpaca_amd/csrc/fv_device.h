@@ -130,7 +130,8 @@ struct StageArgs {
   double inv_dx;
   int nblocks;
   int stage;
-  int signal;         // reduce the CFL signal of the new state into state->smax
+  int signal;         // reduce the CFL signal of the new state into state->smax,
+  double *partials;   // or, if not null, each workgroup's into partials[blockIdx.x]
   double *init_copy;  // stage 0: also copy the Average buffer here (or null)
   int guard;          // do nothing once the case record has reached its end time
 };
@@ -150,6 +151,7 @@ struct TileJob {
   double gamma, b, inv_dx;
   int stage;
   int signal;
+  double *partials;
 };
 
 // Device description of a case held in an ensemble pool.
