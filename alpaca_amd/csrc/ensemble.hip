@@ -3,17 +3,17 @@
 //
 // Every admitted case owns a contiguous range of block slots in three pools
 // (state u, stage buffers s1, s2).  Its blocks are listed in the work list of
-// its class (flux family x arithmetic mode).  One macro step of the whole
-// ensemble is a captured hipGraph:
-//   ens_dt_kernel                 per-case CFL step (modular_algorithm_
-//                                 assembler.cpp:1932-1982) from the signal the
-//                                 previous step's last stage reduced;
-//   3 x batch_stage_kernel/class  persistent kernels over every tile of every
-//                                 listed block (fused faces + divergence + RK
-//                                 + halo push; stage 2 also reduces the next
-//                                 signal);
-//   ens_finish_kernel             per-case FinishMacroTimestep and the stop
-//                                 conditions (t_end reached, unhealthy step).
+// its class (flux family x arithmetic mode).  One macro step of a class is a
+// captured hipGraph, the classes side by side:
+//   ens_dt_kernel           per-case CFL step (modular_algorithm_assembler.cpp:
+//                           1932-1982) from the signal the previous step's last
+//                           stage reduced (a later step of a call first ends the
+//                           step before);
+//   3 x batch_stage_kernel  persistent kernels over every tile of every listed
+//                           block (fused faces + divergence + RK + halo push;
+//                           stage 2 also reduces the next signal).
+// ens_finish_kernel ends a call's last step: per-case FinishMacroTimestep and the
+// stop conditions (t_end reached, unhealthy step).
 // Work lists and case slots live in device memory, so the graph stays valid
 // while cases come and go; only the tuning (tile shape, groups per CU)
 // re-captures it.  Each case's arithmetic depends only on its own blocks and
@@ -43,10 +43,7 @@ int mode_of(int precision) {
 }
 int class_of(int flux, int precision) { return flux * 3 + mode_of(precision); }
 
-__global__ void ens_dt_kernel(const CaseSlot *slots, alpaca_case_state *states, int ncases) {
-  int const i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= ncases) return;
-  alpaca_case_state &s = states[i];
+__device__ __forceinline__ void case_dt(const CaseSlot &slot, alpaca_case_state &s) {
   int const f = s.flags;
   if (!(f & kFlagActive) || (f & kFlagsStop())) return;
   if (f & kFlagFresh) {  // admission computed the first step already
@@ -54,17 +51,14 @@ __global__ void ens_dt_kernel(const CaseSlot *slots, alpaca_case_state *states, 
     return;
   }
   double const sig = __longlong_as_double((long long)s.smax);
-  double const rate = exact::fdiv(sig, slots[i].cell_size);
+  double const rate = exact::fdiv(sig, slot.cell_size);
   double dt = rate == 0.0 ? 1.7976931348623157e308 : exact::fdiv(s.cfl, rate);
   if (s.time + dt > s.t_end) dt = exact::smax(s.t_end - s.time, 0.0);
   s.dt = dt;
   s.smax = 0;
 }
 
-__global__ void ens_finish_kernel(alpaca_case_state *states, int ncases) {
-  int const i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= ncases) return;
-  alpaca_case_state &s = states[i];
+__device__ __forceinline__ void case_finish(alpaca_case_state &s) {
   int f = s.flags;
   if (!(f & kFlagActive) || (f & kFlagsStop())) return;
   s.time += 0.0 + s.dt;
@@ -72,6 +66,22 @@ __global__ void ens_finish_kernel(alpaca_case_state *states, int ncases) {
   if (!(s.time < s.t_end)) f |= kFlagDone;
   if (s.dt < 2.220446049250313080847263336181640625e-16 && s.dt > 0.0) f |= kFlagUnhealthy;
   s.flags = f;
+}
+
+// The time steps of a class's cases; LATER: after the end of the step before.
+template <bool LATER>
+__global__ void ens_dt_kernel(const CaseSlot *slots, alpaca_case_state *states, int ncases, int cls) {
+  int const i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= ncases || slots[i].cls != cls) return;
+  alpaca_case_state s = states[i];
+  if constexpr (LATER) case_finish(s);
+  case_dt(slots[i], s);
+  states[i] = s;
+}
+
+__global__ void ens_finish_kernel(alpaca_case_state *states, int ncases) {
+  int const i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < ncases) case_finish(states[i]);
 }
 
 __global__ void ens_set_flags_kernel(alpaca_case_state *states, int i, int set, int clear) {
@@ -166,8 +176,8 @@ struct alpaca_ensemble {
   int units_per_block = 1;
   BlockPool *pool = nullptr;
   hipStream_t stream = nullptr;
-  hipStream_t aux[kClasses] = {};  // branch streams of the captured step
-  hipEvent_t fork[3] = {}, join[3][kClasses] = {};
+  hipStream_t aux[kClasses] = {};  // streams of the classes but the first
+  hipEvent_t fork = nullptr, join[kClasses] = {};
   double *u = nullptr, *s1 = nullptr, *s2 = nullptr;
   CaseSlot *d_slots = nullptr;
   alpaca_case_state *d_states = nullptr;
@@ -183,8 +193,9 @@ struct alpaca_ensemble {
   int tile_config = 0;
   int groups_per_cu = 0;  // 0: default from occupancy
   int num_cus = 256;
-  hipGraphExec_t exec[kMaxTileConfigs] = {};  // the captured step per configuration
-  hipGraph_t graph[kMaxTileConfigs] = {};
+  // A class's captured step per configuration: [0] the first of a call, [1] later.
+  hipGraphExec_t exec[kMaxTileConfigs][kClasses][2] = {};
+  hipGraph_t graph[kMaxTileConfigs][kClasses][2] = {};
   std::mutex mu;
 };
 
@@ -295,68 +306,83 @@ void launch_class(alpaca_ensemble *e, int tile_config, int c, int groups, hipStr
   }
 }
 
-// The macro step as captured: dt, then per stage the persistent kernel of
-// every enabled class -- the classes of one stage as parallel branches (a
-// fork event on the step's stream, one branch stream per further class, a
-// join before the next stage), so one class's tail overlaps the others'
-// work -- then the per-case finish.  Classes touch disjoint cases, so the
-// branches never write the same block.
-int record_step(alpaca_ensemble *e, int tile_config) {
+// A class's macro step as captured: the time steps of its cases (after the end of
+// the step before, for a later step of a call), then the three stages.
+int record_step(alpaca_ensemble *e, int tile_config, int cls, int later, hipStream_t s) {
   int const g0 = e->groups_per_cu > 0 ? e->groups_per_cu : default_groups_per_cu(e->dim, tile_config);
   int groups = g0 * e->num_cus;
   groups = (groups + 7) / 8 * 8;
   int const nc = e->max_cases;
-  hipLaunchKernelGGL(ens_dt_kernel, dim3((nc + 255) / 256), dim3(256), 0, e->stream, e->d_slots,
-                     e->d_states, nc);
-  int cls[kClasses];
-  int ncls = 0;
-  for (int c = 0; c < kClasses; ++c)
-    if (e->class_mask & (1u << c)) cls[ncls++] = c;
-  for (int stage = 0; stage < 3; ++stage) {
-    if (ncls > 1 && hipEventRecord(e->fork[stage], e->stream) != hipSuccess) return ALPACA_ERR_HIP;
-    for (int i = 0; i < ncls; ++i) {
-      int const c = cls[i];
-      hipStream_t s = i == 0 ? e->stream : e->aux[c];
-      if (i > 0 && hipStreamWaitEvent(s, e->fork[stage], 0) != hipSuccess) return ALPACA_ERR_HIP;
-      launch_class(e, tile_config, c, groups, s, stage);
-      if (i > 0 && hipEventRecord(e->join[stage][c], s) != hipSuccess) return ALPACA_ERR_HIP;
-    }
-    for (int i = 1; i < ncls; ++i)
-      if (hipStreamWaitEvent(e->stream, e->join[stage][cls[i]], 0) != hipSuccess)
-        return ALPACA_ERR_HIP;
-  }
-  hipLaunchKernelGGL(ens_finish_kernel, dim3((nc + 255) / 256), dim3(256), 0, e->stream,
-                     e->d_states, nc);
+  dim3 const grid((nc + 255) / 256), block(256);
+  if (later)
+    hipLaunchKernelGGL(ens_dt_kernel<true>, grid, block, 0, s, e->d_slots, e->d_states, nc, cls);
+  else
+    hipLaunchKernelGGL(ens_dt_kernel<false>, grid, block, 0, s, e->d_slots, e->d_states, nc, cls);
+  for (int stage = 0; stage < 3; ++stage) launch_class(e, tile_config, cls, groups, s, stage);
   return hip_ok(hipGetLastError());
 }
 
-void drop_graph(alpaca_ensemble *e, int tile_config) {
-  if (e->exec[tile_config]) (void)hipGraphExecDestroy(e->exec[tile_config]);
-  if (e->graph[tile_config]) (void)hipGraphDestroy(e->graph[tile_config]);
-  e->exec[tile_config] = nullptr;
-  e->graph[tile_config] = nullptr;
+void drop_graph(alpaca_ensemble *e, int tile_config, int cls, int later) {
+  hipGraphExec_t &exec = e->exec[tile_config][cls][later];
+  hipGraph_t &graph = e->graph[tile_config][cls][later];
+  if (exec) (void)hipGraphExecDestroy(exec);
+  if (graph) (void)hipGraphDestroy(graph);
+  exec = nullptr;
+  graph = nullptr;
 }
 void drop_graphs(alpaca_ensemble *e) {
-  for (int t = 0; t < kMaxTileConfigs; ++t) drop_graph(e, t);
+  for (int t = 0; t < kMaxTileConfigs; ++t)
+    for (int c = 0; c < kClasses; ++c)
+      for (int later = 0; later < 2; ++later) drop_graph(e, t, c, later);
 }
 
-int capture_step(alpaca_ensemble *e, int tile_config) {
-  drop_graph(e, tile_config);
-  if (hipStreamBeginCapture(e->stream, hipStreamCaptureModeThreadLocal) != hipSuccess)
+int capture_step(alpaca_ensemble *e, int tile_config, int cls, int later, hipStream_t s) {
+  drop_graph(e, tile_config, cls, later);
+  if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess)
     return ALPACA_ERR_HIP;
-  int const st = record_step(e, tile_config);
+  int const st = record_step(e, tile_config, cls, later, s);
   hipGraph_t g = nullptr;
-  hipError_t const end = hipStreamEndCapture(e->stream, &g);
+  hipError_t const end = hipStreamEndCapture(s, &g);
   if (st != ALPACA_OK || end != hipSuccess) {
     if (g) (void)hipGraphDestroy(g);
     return st != ALPACA_OK ? st : ALPACA_ERR_HIP;
   }
-  e->graph[tile_config] = g;
-  if (hipGraphInstantiate(&e->exec[tile_config], g, nullptr, nullptr, 0) != hipSuccess) {
-    drop_graph(e, tile_config);
+  e->graph[tile_config][cls][later] = g;
+  if (hipGraphInstantiate(&e->exec[tile_config][cls][later], g, nullptr, nullptr, 0) != hipSuccess) {
+    drop_graph(e, tile_config, cls, later);
     return ALPACA_ERR_HIP;
   }
   return ALPACA_OK;
+}
+
+// nsteps macro steps of the enabled classes, side by side: the first class on the
+// ensemble's stream, each further one on a stream of its own between a fork and a
+// join event, so that the ensemble's stream orders the call as a whole.  Classes
+// touch disjoint cases, blocks and records.  Two classes of 290 blocks: 151 us a
+// step with a join per stage (9 us each), 118 with one per step (25 us with the
+// records' kernel), 100 to 115 with one per call.
+int run_classes(alpaca_ensemble *e, int tile_config, int nsteps) {
+  int cls[kClasses];
+  int ncls = 0;
+  for (int c = 0; c < kClasses; ++c)
+    if (e->class_mask & (1u << c)) cls[ncls++] = c;
+  auto stream = [&](int i) { return i == 0 ? e->stream : e->aux[cls[i]]; };
+  for (int i = 0; i < ncls; ++i)
+    for (int later = 0; later < (nsteps > 1 ? 2 : 1); ++later)
+      if (!e->exec[tile_config][cls[i]][later]) {
+        int const st = capture_step(e, tile_config, cls[i], later, stream(i));
+        if (st != ALPACA_OK) return st;
+      }
+  bool ok = ncls == 1 || hipEventRecord(e->fork, e->stream) == hipSuccess;
+  for (int i = 1; ok && i < ncls; ++i) ok = hipStreamWaitEvent(stream(i), e->fork, 0) == hipSuccess;
+  for (int n = 0; ok && n < nsteps; ++n)
+    for (int i = 0; ok && i < ncls; ++i)
+      ok = hipGraphLaunch(e->exec[tile_config][cls[i]][n > 0], stream(i)) == hipSuccess;
+  // Joined after a failure too: what was queued is ordered before later calls.
+  for (int i = 1; i < ncls; ++i)
+    ok = hipEventRecord(e->join[cls[i]], stream(i)) == hipSuccess &&
+         hipStreamWaitEvent(e->stream, e->join[cls[i]], 0) == hipSuccess && ok;
+  return ok ? ALPACA_OK : ALPACA_ERR_HIP;
 }
 
 }  // namespace
@@ -415,12 +441,10 @@ int ensemble_init(alpaca_ensemble *e, BlockPool *pool, int dim, int max_cases,
     if (class_mask & (1u << c))
       ok = hipMalloc(&e->d_items[c], sizeof(WorkItem) * e->max_blocks) == hipSuccess &&
            hipStreamCreateWithFlags(&e->aux[c], hipStreamNonBlocking) == hipSuccess;
-  for (int st = 0; ok && st < 3; ++st) {
-    ok = hipEventCreateWithFlags(&e->fork[st], hipEventDisableTiming) == hipSuccess;
-    for (int c = 0; ok && c < kClasses; ++c)
-      if (class_mask & (1u << c))
-        ok = hipEventCreateWithFlags(&e->join[st][c], hipEventDisableTiming) == hipSuccess;
-  }
+  ok = ok && hipEventCreateWithFlags(&e->fork, hipEventDisableTiming) == hipSuccess;
+  for (int c = 0; ok && c < kClasses; ++c)
+    if (class_mask & (1u << c))
+      ok = hipEventCreateWithFlags(&e->join[c], hipEventDisableTiming) == hipSuccess;
   if (ok) {
     ok = hipMemsetAsync(e->d_states, 0, sizeof(alpaca_case_state) * max_cases, e->stream) ==
              hipSuccess &&
@@ -501,11 +525,9 @@ int alpaca_ensemble_destroy(alpaca_ensemble *e) {
     (void)hipFree(e->d_items[c]);
     if (e->aux[c]) (void)hipStreamDestroy(e->aux[c]);
   }
-  for (int st = 0; st < 3; ++st) {
-    if (e->fork[st]) (void)hipEventDestroy(e->fork[st]);
-    for (int c = 0; c < kClasses; ++c)
-      if (e->join[st][c]) (void)hipEventDestroy(e->join[st][c]);
-  }
+  if (e->fork) (void)hipEventDestroy(e->fork);
+  for (int c = 0; c < kClasses; ++c)
+    if (e->join[c]) (void)hipEventDestroy(e->join[c]);
   release_pool(e->pool);
   delete e;
   return ALPACA_OK;
@@ -551,6 +573,7 @@ int alpaca_ensemble_add_case(alpaca_ensemble *e, const alpaca_case_desc *desc,
   }
   cs.base = base;
   cs.nblocks = nb;
+  cs.cls = cls;
   cs.gamma = desc->gamma;
   cs.b = desc->background_pressure;
   cs.inv_dx = 1.0 / desc->cell_size;
@@ -613,10 +636,11 @@ int alpaca_ensemble_step(alpaca_ensemble *e, int nsteps) {
   size_t blocks = 0;
   for (auto const &items : e->h_items) blocks += items.size();
   int const t = e->tuned ? e->tile_config : auto_tile_config(e->dim, (long long)blocks, e->num_cus);
-  if (!e->exec[t] && (st = capture_step(e, t)) != ALPACA_OK) return st;
-  for (int n = 0; n < nsteps; ++n)
-    if (hipGraphLaunch(e->exec[t], e->stream) != hipSuccess) return ALPACA_ERR_HIP;
-  return ALPACA_OK;
+  if (nsteps == 0) return ALPACA_OK;
+  if ((st = run_classes(e, t, nsteps)) != ALPACA_OK) return st;
+  hipLaunchKernelGGL(ens_finish_kernel, dim3((e->max_cases + 255) / 256), dim3(256), 0, e->stream,
+                     e->d_states, e->max_cases);
+  return hip_ok(hipGetLastError());
 }
 
 int alpaca_ensemble_read_states(alpaca_ensemble *e, alpaca_case_state *host_out, int n) {

@@ -160,6 +160,7 @@ struct CaseSlot {
   int bc[3];
   int base;      // pool index of the case's first block
   int nblocks;
+  int cls;       // class: flux family x arithmetic mode
   double gamma, b, inv_dx, cell_size;
 };
 
