@@ -504,6 +504,9 @@ int alpaca_ensemble_create_shared(alpaca_ensemble *peer, int dim, int max_cases,
     std::lock_guard<std::mutex> lock(peer->pool->mu);
     peer->pool->refs += 1;
   }
+  // Ranges that the peer released while it had the pool alone may still be in use by
+  // steps on its stream.
+  (void)hipStreamSynchronize(peer->stream);
   e->pool = peer->pool;
   if (ensemble_init(e, peer->pool, dim, max_cases, class_mask, static_cast<hipStream_t>(stream)) !=
       ALPACA_OK) {
@@ -598,10 +601,17 @@ int alpaca_ensemble_remove_case(alpaca_ensemble *e, int case_id) {
   auto &v = e->h_items[cls];
   v.erase(std::remove_if(v.begin(), v.end(), [&](WorkItem const &w) { return w.case_id == case_id; }),
           v.end());
+  // The next step uploads the list first, and what takes over the slot and the
+  // blocks is queued on this stream after the steps that used them; an ensemble
+  // sharing the pool has a stream of its own, so the steps are waited for.  (With an
+  // upload and a wait here always, a release took 75 us.)
   e->items_dirty = true;
-  // The work list must drop the case before its slot and blocks are reused.
-  int st = upload_lists(e);
-  if (st != ALPACA_OK) return st;
+  bool shared;
+  {
+    std::lock_guard<std::mutex> pool(e->pool->mu);
+    shared = e->pool->refs > 1;
+  }
+  if (shared && hipStreamSynchronize(e->stream) != hipSuccess) return ALPACA_ERR_HIP;
   hipLaunchKernelGGL(ens_set_flags_kernel, dim3(1), dim3(64), 0, e->stream, e->d_states, case_id, 0,
                      ~0);
   free_range(e, e->h_slots[case_id].base, e->h_slots[case_id].nblocks);
