@@ -767,14 +767,14 @@ template <int FLUX, int MODE> bool use_march(int nblocks) {
 // it is ahead where the pairs are resident at once or nearly so, and where there
 // are many (exact HLLC, one stage, us, against 16x16 tiles): 1600 blocks 69 and 74,
 // 2025 71 and 91, 2500 90 and 103, 3249 127 and 123, 4900 165 and 170, 16384 529
-// and 550.  The other forms gain at many blocks only (16384: HLLC FMA 307 and
-// 325, mixed 291 and 301, Roe mixed 382 and 396); the Roe form with FMA, whose
-// registers hold 16 wavefronts a CU, loses (534 and 484).
+// and 550; Roe with FMA 2025 44 and 53, 4900 103 and 101, 16384 347 and 365.  The
+// other forms, which run 4 or 5 wavefronts per SIMD, gain at many blocks only
+// (16384: HLLC FMA 307 and 325, mixed 291 and 301, Roe mixed 382 and 396).
 template <int FLUX, int MODE> bool use_pairs(long long nblocks) {
   long long const cus = device_cus();
-  if (FLUX == ALPACA_FLUX_ROE && MODE == kModeFma) return false;
-  if (nblocks >= 32 * cus) return true;
-  return MODE == kModeExact && nblocks >= 6 * cus && (nblocks <= 10 * cus || nblocks >= 16 * cus);
+  bool const heavy = MODE == kModeExact || (FLUX == ALPACA_FLUX_ROE && MODE == kModeFma);
+  return nblocks >= 32 * cus || (MODE == kModeExact && nblocks >= 16 * cus) ||
+         (heavy && nblocks >= 6 * cus && nblocks <= 10 * cus);
 }
 
 template <int FLUX, int MODE>

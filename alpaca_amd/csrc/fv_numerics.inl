@@ -538,13 +538,10 @@ template <int NE, typename R> struct Eig {
   bool ok;
 };
 
-// Structural zeros of the Roe eigenvectors (eigendecomposition.h:238-466):
-// L rows 1 and 2 (the shear waves) hold only the mass and their own
-// transverse momentum; R leaves out the shear columns of the mass, normal
-// momentum and other transverse momentum rows.  The FP64-with-FMA form skips
-// these products (0 * x changes a sum only for a non-finite x, which that
-// form does not track); the exact form forms them, as the reference does,
-// and the mixed form keeps its measured accuracy by keeping them too.
+// Structural zeros of the left Roe eigenvectors (eigendecomposition.h:238-466):
+// rows 1 and 2 (the shear waves) hold only the mass and their own transverse
+// momentum.  The exact form leaves these products out where the stencil is
+// finite; the mixed form keeps its measured accuracy by forming them.
 template <int DIM, int DIR> __device__ __forceinline__ constexpr bool left_zero(int n, int c) {
   constexpr int Mp = kMomX + DIR, M1 = kMomX + Minor<DIR>::m1, M2 = kMomX + Minor<DIR>::m2;
   if (n == 1) return c != kMass && c != M1;
@@ -552,17 +549,6 @@ template <int DIM, int DIR> __device__ __forceinline__ constexpr bool left_zero(
   (void)Mp;
   return false;
 }
-template <int DIM, int DIR> __device__ __forceinline__ constexpr bool right_zero(int r, int c) {
-  constexpr int Mp = kMomX + DIR, M1 = kMomX + Minor<DIR>::m1, M2 = kMomX + Minor<DIR>::m2;
-  bool const shear = c >= 1 && c < DIM;  // columns 1 .. DIM-1
-  if (!shear) return false;
-  if (r == kMass || r == Mp) return true;
-  if (r == M1) return c != 1;
-  if (DIM == 3 && r == M2) return c != 2;
-  return false;
-}
-template <typename R> constexpr bool kSkipZeros = kFastArith && std::is_same<R, double>::value;
-
 // The exact FP64 finite-volume (HLLC) kernels build the right eigenvectors
 // only once the characteristic values are formed, so the 19 entries are not
 // held in registers meanwhile (it saves 20 VGPRs in 3D); without contraction
@@ -726,7 +712,7 @@ __device__ __forceinline__ void to_physical(const R *ch, const R (&Rm)[DIM + 2][
     R s = R(0.0);
 #pragma unroll
     for (int n = 1; n < NE - 1; ++n)
-      if (!(kSkipZeros<R> && right_zero<DIM, DIR>(l, n))) s += ch[n] * Rm[l][n];
+      s += ch[n] * Rm[l][n];
     s += (ch[0] * Rm[l][0] + ch[NE - 1] * Rm[l][NE - 1]);
     out[l] = s;
   }
@@ -934,17 +920,16 @@ __device__ __forceinline__ void roe_split_flux_exact(double gamma, double b,
 }
 
 // FluxSplittingScheme::ComputeFluxes + ComputeAdvection for one face
-// (flux_splitting_scheme.cpp:42-76, 185-315), added into f, in the
-// contracting forms (FP64 with FMA, mixed).  The stencil is walked cell by
-// cell -- load, advection, projection onto every field -- which keeps few
-// values live: 2 waves per SIMD for the FP64-with-FMA kernel, 3 for the mixed
-// one.  Each projection is the expression of the exact form.
-template <int DIM, int DIR, typename R, typename QS>
+// (flux_splitting_scheme.cpp:42-76, 185-315), added into f, in the mixed form.
+// The stencil is walked cell by cell -- load, advection, projection onto every
+// field -- which keeps few values live: 3 waves per SIMD.  Each projection is
+// the expression of the exact form.
+template <int DIM, int DIR, typename QS>
 __device__ __forceinline__ void roe_split_flux(double gamma64, double b64,
                                                const double *__restrict__ base, const QS &qs,
-                                               R *f) {
+                                               float *f) {
+  using R = float;
   constexpr int NE = DIM + 2;
-  constexpr bool kShift = std::is_same<R, float>::value;
   R const gamma = R(gamma64);
   auto load = [base](int m, double *c) {
 #pragma unroll
@@ -952,14 +937,14 @@ __device__ __forceinline__ void roe_split_flux(double gamma64, double b64,
       c[e] = base[e * Dims<DIM>::FIELD + (m - 2) * axis_stride<DIM, DIR>()];
   };
   Eig<NE, R> ev;
-  double adv2[NE];  // advection of cell i (FP64; mixed form only)
+  double adv2[NE];  // advection of cell i (FP64)
   R chf[NE];
   {
     double Ui[NE], Un[NE];
     load(2, Ui);
     load(3, Un);
     roe_eigensystem<DIM, DIR, R, false>(gamma, qs.left(Ui), qs.right(Un), ev);
-    if constexpr (kShift) {
+    {
       Prim<double> pd;
       cons_to_prim<DIM, double>(gamma64, b64, Ui, pd);
       advection<DIM, DIR>(Ui, pd, adv2);
@@ -971,32 +956,22 @@ __device__ __forceinline__ void roe_split_flux(double gamma64, double b64,
       load(m, Um);
       R Uc[NE];
 #pragma unroll
-      for (int e = 0; e < NE; ++e) Uc[e] = kShift ? R(Um[e] - Ui[e]) : R(Um[e]);
+      for (int e = 0; e < NE; ++e) Uc[e] = R(Um[e] - Ui[e]);
       R adv[NE];
       Prim<double> pd;
       cons_to_prim<DIM, double>(gamma64, b64, Um, pd);
-      if constexpr (kShift) {
-        // ComputeAdvection in FP64, then the difference from cell i into
-        // FP32 (see face_flux).
-        double a64[NE];
-        advection<DIM, DIR>(Um, pd, a64);
+      // ComputeAdvection in FP64, then the difference from cell i into FP32
+      // (see face_flux).
+      double a64[NE];
+      advection<DIM, DIR>(Um, pd, a64);
 #pragma unroll
-        for (int e = 0; e < NE; ++e) adv[e] = R(a64[e] - adv2[e]);
-      } else {
-        R const rho = R(pd.rho), p = R(pd.p), ud = R(pd.vel[DIR]);
-        adv[kMass] = rho * ud;
-        adv[kEnergy] = (Uc[kEnergy] + p) * ud;
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) adv[kMomX + d] = rho * (ud * R(pd.vel[d]));
-        adv[kMomX + DIR] += p;
-      }
+      for (int e = 0; e < NE; ++e) adv[e] = R(a64[e] - adv2[e]);
 #pragma unroll
       for (int n = 0; n < NE; ++n) {
         R sp = R(0.0), sn = R(0.0);
 #pragma unroll
         for (int q = 0; q < NE; ++q) {
           int const l = seq<DIM, DIR>(q);
-          if (kSkipZeros<R> && left_zero<DIM, DIR>(n, l)) continue;
           R const uct = Uc[l] * ev.L[n][l];
           R const act = adv[l] * ev.L[n][l];
           sp += (act + ev.lam[n] * uct);
@@ -1015,14 +990,9 @@ __device__ __forceinline__ void roe_split_flux(double gamma64, double b64,
   }
   R phys[NE];
   to_physical<DIM, DIR>(chf, ev.Rm, phys);
-  if constexpr (kShift) {
-    // R L (adv of cell i) = adv of cell i: the half sums of the shifts.
+  // R L (adv of cell i) = adv of cell i: the half sums of the shifts.
 #pragma unroll
-    for (int e = 0; e < NE; ++e) f[e] += R(double(phys[e]) + adv2[e]);
-  } else {
-#pragma unroll
-    for (int e = 0; e < NE; ++e) f[e] += phys[e];
-  }
+  for (int e = 0; e < NE; ++e) f[e] += R(double(phys[e]) + adv2[e]);
 }
 
 // The reconstruction of the FP64-with-FMA form: the products with the Roe
@@ -1035,72 +1005,55 @@ __device__ __forceinline__ void roe_split_flux(double gamma64, double b64,
 //   rho = a_- + a_+ + g a_e,  d = c (a_+ - a_-),  m_n = u rho + d, ...
 // The stencil is dead once Y, A, B and the shear amplitudes are formed, and no
 // eigenvector matrix is held.
-template <int DIM, int DIR, typename QS>
-__device__ __forceinline__ void fv_reconstruct_lean(double gamma, const double (&U)[6][DIM + 2],
-                                                    const QS &qs, double *cl, double *cr) {
-  constexpr int m1 = Minor<DIR>::m1, m2 = Minor<DIR>::m2;
-  constexpr int Mp = kMomX + DIR, M1 = kMomX + m1, M2 = kMomX + m2;
-  FaceQ<double> const t = qs.left(U[2]), n = qs.right(U[3]);
-  if (!(t.rho > 0.0) || !(n.rho > 0.0)) {
-    if (t.rho <= 0.0 || n.rho <= 0.0) {
-      // No eigensystem: a zero state, whose face is skipped.
-#pragma unroll
-      for (int e = 0; e < DIM + 2; ++e) cl[e] = cr[e] = 0.0;
-      return;
+template <int DIM, int DIR> struct LeanEig {
+  static constexpr int m1 = Minor<DIR>::m1, m2 = Minor<DIR>::m2;
+  static constexpr int Mp = kMomX + DIR, M1 = kMomX + m1, M2 = kMomX + m2;
+  double g, u, v, w, H, c, cc, one_cc, rho_roe, one_rho, kY, kA, kB, kBu, kv, kw;
+  // Returns false where a density is not positive: no eigensystem.
+  __device__ __forceinline__ bool form(double gamma, const FaceQ<double> &t, const FaceQ<double> &n) {
+    if (!(t.rho > 0.0) || !(n.rho > 0.0)) {
+      if (t.rho <= 0.0 || n.rho <= 0.0) return false;
+    }
+    double const rho_div = fdiv(1.0, t.sq + n.sq);
+    rho_roe = t.sq * n.sq;
+    one_rho = fdiv(1.0, rho_roe);
+    auto mean = [&](double a, double b) { return (a * t.sq + b * n.sq) * rho_div; };
+    u = mean(t.vel[DIR], n.vel[DIR]);
+    v = mean(t.vel[m1], n.vel[m1]);
+    w = DIM == 3 ? mean(t.vel[m2], n.vel[m2]) : 0.0;
+    g = gamma - 1.0;
+    H = mean(t.H, n.H);
+    double const du = t.vel[DIR] - n.vel[DIR], dv = t.vel[m1] - n.vel[m1];
+    double q2 = u * u + v * v, dq = du * du + dv * dv;
+    if constexpr (DIM == 3) {
+      double const dw = t.vel[m2] - n.vel[m2];
+      q2 += w * w;
+      dq += dw * dw;
+    }
+    cc = mean(t.psi + g * t.pod, n.psi + g * n.pod) + g * (0.5 * rho_roe * (rho_div * rho_div) * dq);
+    one_cc = fdiv(1.0, cc);
+    c = dsqrt(cc);
+    kY = q2 - H;
+    kA = 0.5 * g * one_cc;
+    kB = 0.5 * one_cc * c;
+    kBu = kB * u;
+    kv = v * one_rho;
+    kw = w * one_rho;
+    return true;
+  }
+  // Y, B and the shear amplitudes of a vector of conservatives.
+  __device__ __forceinline__ void parts(const double *U, double &Y, double &B, double &s1,
+                                        double &s2) const {
+    s1 = kv * U[kMass] - one_rho * U[M1];
+    Y = U[kEnergy] - u * U[Mp] - v * U[M1] + kY * U[kMass];
+    B = kBu * U[kMass] - kB * U[Mp];
+    if constexpr (DIM == 3) {
+      s2 = one_rho * U[M2] - kw * U[kMass];
+      Y -= w * U[M2];
     }
   }
-  double const rho_div = fdiv(1.0, t.sq + n.sq);
-  double const rho_roe = t.sq * n.sq;
-  double const one_rho = fdiv(1.0, rho_roe);
-  auto mean = [&](double a, double b) { return (a * t.sq + b * n.sq) * rho_div; };
-  double const u = mean(t.vel[DIR], n.vel[DIR]), v = mean(t.vel[m1], n.vel[m1]);
-  double const w = DIM == 3 ? mean(t.vel[m2], n.vel[m2]) : 0.0;
-  double const g = gamma - 1.0;
-  double const H = mean(t.H, n.H);
-  double const du = t.vel[DIR] - n.vel[DIR], dv = t.vel[m1] - n.vel[m1];
-  double q2 = u * u + v * v, dq = du * du + dv * dv;
-  if constexpr (DIM == 3) {
-    double const dw = t.vel[m2] - n.vel[m2];
-    q2 += w * w;
-    dq += dw * dw;
-  }
-  double const cc = mean(t.psi + g * t.pod, n.psi + g * n.pod) +
-                    g * (0.5 * rho_roe * (rho_div * rho_div) * dq);
-  double const one_cc = fdiv(1.0, cc);
-  double const c = dsqrt(cc);
-  double const kY = q2 - H, kA = 0.5 * g * one_cc, kB = 0.5 * one_cc * c;
-  double const kBu = kB * u, kv = v * one_rho, kw = w * one_rho;
-
-  double Y[6], B[6], lo[DIM + 2], hi[DIM + 2];
-  {
-    double s1[6], s2[6];
-#pragma unroll
-    for (int m = 0; m < 6; ++m) {
-      s1[m] = kv * U[m][kMass] - one_rho * U[m][M1];
-      Y[m] = U[m][kEnergy] - u * U[m][Mp] - v * U[m][M1] + kY * U[m][kMass];
-      B[m] = kBu * U[m][kMass] - kB * U[m][Mp];
-      if constexpr (DIM == 3) {
-        s2[m] = one_rho * U[m][M2] - kw * U[m][kMass];
-        Y[m] -= w * U[m][M2];
-      }
-    }
-    weno_pair_lean(s1, lo[1], hi[1]);
-    if constexpr (DIM == 3) weno_pair_lean(s2, lo[2], hi[2]);
-  }
-  double A[6], x[6];
-#pragma unroll
-  for (int m = 0; m < 6; ++m) {
-    A[m] = kA * Y[m] + 0.5 * U[m][kMass];
-    x[m] = -one_cc * Y[m];
-  }
-  weno_pair_lean(x, lo[DIM], hi[DIM]);
-#pragma unroll
-  for (int m = 0; m < 6; ++m) x[m] = A[m] + B[m];
-  weno_pair_lean(x, lo[0], hi[0]);
-#pragma unroll
-  for (int m = 0; m < 6; ++m) x[m] = A[m] - B[m];
-  weno_pair_lean(x, lo[DIM + 1], hi[DIM + 1]);
-  auto back = [&](const double *a, double *o) {
+  // Conservatives from the amplitudes.
+  __device__ __forceinline__ void back(const double *a, double *o) const {
     double const rho = a[0] + a[DIM + 1] + g * a[DIM];
     double const d = c * (a[DIM + 1] - a[0]);
     double const t1 = rho_roe * a[1];
@@ -1114,9 +1067,107 @@ __device__ __forceinline__ void fv_reconstruct_lean(double gamma, const double (
       e += w * t2;
     }
     o[kEnergy] = e;
+  }
+};
+
+template <int DIM, int DIR, typename QS>
+__device__ __forceinline__ void fv_reconstruct_lean(double gamma, const double (&U)[6][DIM + 2],
+                                                    const QS &qs, double *cl, double *cr) {
+  LeanEig<DIM, DIR> ev;
+  if (!ev.form(gamma, qs.left(U[2]), qs.right(U[3]))) {
+    // A zero state, whose face is skipped.
+#pragma unroll
+    for (int e = 0; e < DIM + 2; ++e) cl[e] = cr[e] = 0.0;
+    return;
+  }
+  double Y[6], B[6], lo[DIM + 2], hi[DIM + 2];
+  {
+    double s1[6], s2[6];
+#pragma unroll
+    for (int m = 0; m < 6; ++m) {
+      ev.parts(U[m], Y[m], B[m], s1[m], s2[m]);
+    }
+    weno_pair_lean(s1, lo[1], hi[1]);
+    if constexpr (DIM == 3) weno_pair_lean(s2, lo[2], hi[2]);
+  }
+  double A[6], x[6];
+#pragma unroll
+  for (int m = 0; m < 6; ++m) {
+    A[m] = ev.kA * Y[m] + 0.5 * U[m][kMass];
+    x[m] = -ev.one_cc * Y[m];
+  }
+  weno_pair_lean(x, lo[DIM], hi[DIM]);
+#pragma unroll
+  for (int m = 0; m < 6; ++m) x[m] = A[m] + B[m];
+  weno_pair_lean(x, lo[0], hi[0]);
+#pragma unroll
+  for (int m = 0; m < 6; ++m) x[m] = A[m] - B[m];
+  weno_pair_lean(x, lo[DIM + 1], hi[DIM + 1]);
+  ev.back(lo, cl);
+  ev.back(hi, cr);
+}
+
+// Flux splitting in the FP64-with-FMA form (roe_split_flux below): the conservatives
+// and the advection of a stencil cell are projected by the factored products, 40
+// instructions a cell with the sums and differences against 114 row by row.
+template <int DIM, int DIR, typename QS>
+__device__ __forceinline__ void roe_split_flux_lean(double gamma, double b,
+                                                    const double *__restrict__ base, const QS &qs,
+                                                    double *f) {
+  constexpr int NE = DIM + 2;
+  using E = LeanEig<DIM, DIR>;
+  auto load = [base](int m, double *c) {
+#pragma unroll
+    for (int e = 0; e < NE; ++e)
+      c[e] = base[e * Dims<DIM>::FIELD + (m - 2) * axis_stride<DIM, DIR>()];
   };
-  back(lo, cl);
-  back(hi, cr);
+  E ev;
+  {
+    double Ui[NE], Un[NE];
+    load(2, Ui);
+    load(3, Un);
+    if (!ev.form(gamma, qs.left(Ui), qs.right(Un))) return;
+  }
+  double const lam = __builtin_fabs(ev.u), lam_lo = __builtin_fabs(ev.u - ev.c),
+               lam_hi = __builtin_fabs(ev.u + ev.c);
+  double pos[NE][6], neg[NE][6];
+#pragma unroll
+  for (int m = 0; m < 6; ++m) {
+    double U[NE], adv[NE];
+    load(m, U);
+    double const one = fdiv(1.0, U[kMass]), ud = U[E::Mp] * one;
+    double k = U[E::Mp] * ud + U[E::M1] * (U[E::M1] * one);
+    if constexpr (DIM == 3) k += U[E::M2] * (U[E::M2] * one);
+    double const p = ev.g * (U[kEnergy] - 0.5 * k) - gamma * b;
+    adv[kMass] = U[E::Mp];
+    adv[kEnergy] = (U[kEnergy] + p) * ud;
+    adv[E::Mp] = U[E::Mp] * ud + p;
+    adv[E::M1] = U[E::M1] * ud;
+    if constexpr (DIM == 3) adv[E::M2] = U[E::M2] * ud;
+    double uY, uB, u1, u2, aY, aB, a1, a2;
+    ev.parts(U, uY, uB, u1, u2);
+    ev.parts(adv, aY, aB, a1, a2);
+    auto put = [&](int n, double a, double lu) {
+      pos[n][m] = a + lu;
+      neg[n][m] = a - lu;
+    };
+    double const uA = ev.kA * uY + 0.5 * U[kMass], aA = ev.kA * aY + 0.5 * adv[kMass];
+    put(0, aA + aB, lam_lo * (uA + uB));
+    put(1, a1, lam * u1);
+    if constexpr (DIM == 3) put(2, a2, lam * u2);
+    put(DIM, -ev.one_cc * aY, -ev.one_cc * (lam * uY));
+    put(DIM + 1, aA - aB, lam_hi * (uA - uB));
+  }
+  double chf[NE], phys[NE];
+#pragma unroll
+  for (int n = 0; n < NE; ++n) {
+    double wl, wr;
+    weno_pair<double>(pos[n], neg[n], wl, wr);
+    chf[n] = 0.5 * (wl + wr);
+  }
+  ev.back(chf, phys);
+#pragma unroll
+  for (int e = 0; e < NE; ++e) f[e] += phys[e];
 }
 
 // FP64 square root of a positive argument: nr_sqrt64 without its zero case.
@@ -1342,8 +1393,10 @@ __device__ __forceinline__ void face_flux(double gamma64, double b64,
     fv_face<DIM, DIR, R>(gamma64, b64, blk, off, qs, f);
   } else if constexpr (std::is_same<R, double>::value && !kFastArith) {
     roe_split_flux_exact<DIM, DIR>(gamma64, b64, blk, off, qs, f);
+  } else if constexpr (kLean<R>) {
+    roe_split_flux_lean<DIM, DIR>(gamma64, b64, base, qs, f);
   } else {
-    roe_split_flux<DIM, DIR, R>(gamma64, b64, base, qs, f);
+    roe_split_flux<DIM, DIR>(gamma64, b64, base, qs, f);
   }
 }
 

@@ -533,12 +533,12 @@ __device__ __forceinline__ void stage_march(const TileJob &j, int blk_local, int
   stage_finish<P>(j, sig, bad);
 }
 
-// Waves per SIMD the register allocator is held to.  The exact FP64 2D kernels
-// fit 3 waves without spilling; the exact 3D flux-splitting kernels need 211
-// to 217 VGPRs (2 waves).
+// Waves per SIMD the register allocator is held to.  The FP64 2D kernels fit 3
+// waves without spilling; the exact 3D flux-splitting kernels need 211 to 217
+// VGPRs (2 waves).
 template <int DIM, int FLUX, typename R>
-constexpr int kMinWaves = kFastArith || !std::is_same<R, double>::value ? 1
-                          : DIM == 2 ? 3 : (FLUX == 1 ? 2 : 1);
+constexpr int kMinWaves = !std::is_same<R, double>::value ? 1
+                          : DIM == 2 ? 3 : (FLUX == 1 && !kFastArith ? 2 : 1);
 
 // The persistent batch kernel: as above.
 template <int DIM, int FLUX, typename R>
