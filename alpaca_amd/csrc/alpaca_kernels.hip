@@ -731,7 +731,7 @@ void launch_stage_kernel(dim3 grid, hipStream_t s, const double *avg, const doub
 template <int FLUX, int MODE>
 unsigned launch_march_kernel(int nblocks, hipStream_t s, const double *avg, const double *init,
                          double *out, alpaca_case_state *state, const StageArgs &a) {
-  using R = std::conditional_t<MODE == kModeMixed, float, double>;
+  using R = double;
   using M = exact::MarchShape<R>;
   dim3 const grid(nblocks * M::SLABS), block(M::PLANE);
   if constexpr (MODE == kModeExact)
@@ -750,12 +750,14 @@ unsigned launch_march_kernel(int nblocks, hipStream_t s, const double *avg, cons
 // after the other.  So the case marches where its slabs fill the CUs at least
 // as evenly: 512 blocks 104 units against 112 (exact 1.50 ms a step against
 // 1.54 ms), but 385 blocks 104 against 91 (FMA 0.84 ms against 0.74 ms), and
-// few blocks never (64: 26 against 14).  The mixed HLLC form keeps the tiles.
+// few blocks never (64: 26 against 14).  The mixed forms keep the tiles (HLLC
+// gains nothing; Roe's FP32 faces round differently where a cell's quantities pass
+// through LDS, as other products are then fused).
 // HLLC with FMA marches from 8 blocks per CU only: below, tiles with 512 threads
 // are faster (512 blocks 290 us a stage against 307 marching, 4096 blocks 2364
 // against 2322).
 template <int FLUX, int MODE>
-constexpr bool kMarches = !(FLUX == ALPACA_FLUX_HLLC && MODE == kModeMixed);
+constexpr bool kMarches = MODE != kModeMixed;
 template <int FLUX, int MODE> bool use_march(int nblocks) {
   long long const cus = device_cus();
   if (FLUX == ALPACA_FLUX_HLLC && MODE == kModeFma && nblocks < 8 * cus) return false;

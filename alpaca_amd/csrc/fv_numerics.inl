@@ -273,59 +273,37 @@ __device__ __forceinline__ FaceQ<R> face_quantities(double gamma, double b, cons
   return f;
 }
 
-// A cell's FaceQ as NQ values.  FP64 keeps 1/rho and forms the velocities from
-// the stencil's momenta again (one exact repetition of a product each, 40
-// bytes per cell); the mixed form keeps the velocities, which are rounded
-// from FP64 products, in FP32 (28 bytes).
+// A cell's FaceQ as NQ values: 1/rho is kept and the velocities are formed from the
+// stencil's momenta again (one exact repetition of a product each).
 template <typename R> struct PackedQ {
-  static constexpr bool kF64 = std::is_same<R, double>::value;
-  static constexpr int NQ = kF64 ? 5 : 7;
+  static constexpr int NQ = 5;
+  static_assert(std::is_same<R, double>::value, "FP64 forms");
 };
 
 // Writes the FaceQ of the cell with conservatives c to q[0], q[STRIDE], ...
 template <int DIM, typename R, int STRIDE>
 __device__ __forceinline__ void store_packed(double gamma, double b, const double *c, R *q) {
-  if constexpr (PackedQ<R>::kF64) {
-    CellQ<double> w;
-    cell_quantities<DIM, double>(gamma, b, c, w);
-    q[0] = dsqrt(w.rho);
-    q[STRIDE] = w.one_rho;
-    q[2 * STRIDE] = w.psi;
-    q[3 * STRIDE] = w.H;
-    q[4 * STRIDE] = w.p * w.one_rho;
-  } else {
-    FaceQ<R> const f = face_quantities<DIM, R>(gamma, b, c);
-    q[0] = f.sq;
-    q[STRIDE] = f.vel[0];
-    q[2 * STRIDE] = f.vel[1];
-    q[3 * STRIDE] = f.vel[2];
-    q[4 * STRIDE] = f.psi;
-    q[5 * STRIDE] = f.H;
-    q[6 * STRIDE] = f.pod;
-  }
+  CellQ<double> w;
+  cell_quantities<DIM, double>(gamma, b, c, w);
+  q[0] = dsqrt(w.rho);
+  q[STRIDE] = w.one_rho;
+  q[2 * STRIDE] = w.psi;
+  q[3 * STRIDE] = w.H;
+  q[4 * STRIDE] = w.p * w.one_rho;
 }
 
 template <int DIM, typename R, int STRIDE>
 __device__ __forceinline__ FaceQ<R> load_packed(const R *q, const double *c) {
   FaceQ<R> f;
+  double const one_rho = q[STRIDE];
   f.rho = R(c[kMass]);
   f.sq = q[0];
-  if constexpr (PackedQ<R>::kF64) {
-    double const one_rho = q[STRIDE];
-    f.vel[0] = c[kMomX] * one_rho;
-    f.vel[1] = c[kMomX + 1] * one_rho;
-    f.vel[2] = DIM == 3 ? c[kMomX + DIM - 1] * one_rho : 0.0;
-    f.psi = q[2 * STRIDE];
-    f.H = q[3 * STRIDE];
-    f.pod = q[4 * STRIDE];
-  } else {
-    f.vel[0] = q[STRIDE];
-    f.vel[1] = q[2 * STRIDE];
-    f.vel[2] = q[3 * STRIDE];
-    f.psi = q[4 * STRIDE];
-    f.H = q[5 * STRIDE];
-    f.pod = q[6 * STRIDE];
-  }
+  f.vel[0] = c[kMomX] * one_rho;
+  f.vel[1] = c[kMomX + 1] * one_rho;
+  f.vel[2] = DIM == 3 ? c[kMomX + DIM - 1] * one_rho : 0.0;
+  f.psi = q[2 * STRIDE];
+  f.H = q[3 * STRIDE];
+  f.pod = q[4 * STRIDE];
   return f;
 }
 

@@ -333,14 +333,13 @@ __device__ __forceinline__ void stage_tile(int tid, const TileJob &j, int blk_lo
 // CU as the registers allow.  Before plane 0 the two Q buffers hold the
 // quantities of the cells left and right of the closing faces.
 //
-// Bound by FP64 issue with a share of L2 misses.  256^3, one step, against the
-// 8^3 tiles with the same face arithmetic: HLLC exact 12.06 -> 11.30 ms, FMA
-// 7.46 -> 6.82 ms; Roe exact 22.0 -> 21.4 ms, FMA 11.8 -> 11.0 ms, mixed 9.34 ->
-// 8.82 ms.  The mixed HLLC form gains nothing (7.0 ms both ways: it runs 3
-// waves per SIMD either way and pays the barrier) and keeps the tiles.  A
-// wavefront marching an 8^3 tile by itself, without barriers, was slower
-// (HLLC exact 13.3 ms, FMA 9.96 ms): its waves drift apart and their planes
-// no longer share the caches (1.3e8 L2 misses a launch).
+// Bound by FP64 issue with a share of L2 misses.  256^3, one stage, against the
+// 8^3 tiles: HLLC exact 4.10 -> 3.95 ms, FMA (tiles of 512 threads) 2.36 -> 2.32 ms,
+// Roe exact 5.01 -> 4.70 ms, FMA 2.84 -> 2.79 ms.  The mixed HLLC form gains nothing (it
+// runs 3 or 4 waves per SIMD either way and pays the barrier).  A wavefront
+// marching an 8^3 tile by itself, without barriers, was slower (one step, HLLC
+// exact 13.3 ms against 12.06, FMA 9.96 ms against 7.46): its waves drift apart
+// and their planes no longer share the caches (1.3e8 L2 misses a launch).
 template <typename R> struct MarchShape {
   static constexpr int SX = 8;
   static constexpr int SLABS = kIC / SX;
