@@ -341,7 +341,7 @@ int alpaca_advance(const alpaca_case_desc *desc, double *d_u, double *d_s1,
  * job).  Each case keeps its own time step, end time and stop flags; one
  * alpaca_ensemble_step advances every running case by one macro step with
  * one persistent kernel per RK stage and per enabled class (flux family x
- * arithmetic; the classes of one stage are parallel branches of the step),
+ * arithmetic; the classes run side by side through a call),
  * replayed from a captured hipGraph.  A case's results do not
  * depend on what else runs: per-case reductions only, fixed arithmetic order.
  * The ensemble owns its device memory (allocated at create).
@@ -390,7 +390,8 @@ int alpaca_ensemble_remove_case(alpaca_ensemble *e, int case_id);
 int alpaca_ensemble_cancel_case(alpaca_ensemble *e, int case_id);
 /* Tile shape (3D: 0 = 8x8x8/256 threads, 1 = 16x8x8/512; 2D: 0 = 16x16/128,
  * 1 = 16x16/256, 2 = 16x8/128) and persistent workgroups per CU (0 = the
- * occupancy default) of the stage kernels. */
+ * occupancy default) of the stage kernels.  An ensemble that was given none
+ * chooses its tiles by the number of blocks it holds. */
 int alpaca_ensemble_set_tuning(alpaca_ensemble *e, int tile_config, int groups_per_cu);
 /* Advances every running case by nsteps macro steps (asynchronous). */
 int alpaca_ensemble_step(alpaca_ensemble *e, int nsteps);
