@@ -15,11 +15,10 @@
 // Work decomposition.  A link names (child block, parent block, sibling
 // position, child level).  Averaging is one thread per two parent cells
 // written (adjacent along the fastest axis, so the child reads of neighbouring
-// threads are contiguous 16-byte accesses).  Prediction and details stage the parent's stencil window --
-// the predicted parent cells plus two on each side, at most 16 per axis
-// (32 KiB of doubles in 3D) -- in LDS once per field and let each thread
-// predict the 2^DIM children of one parent cell from it: the 3D stencil reads
-// 125 parent values per parent cell, which LDS serves instead of L1/L2.
+// threads are contiguous 16-byte accesses).  Prediction and details stage the
+// parent's stencil window -- the predicted parent cells plus two on each side, at
+// most 16 per axis (32 KiB of doubles in 3D) -- in LDS; a thread predicts the
+// children of one parent cell in 2D, of two adjacent along z in 3D.
 #include <hip/hip_runtime.h>
 
 #include <cstring>
@@ -31,7 +30,7 @@ namespace mr {
 namespace {
 
 constexpr int kThreads = 256;         // averaging
-constexpr int kStencilThreads = 192;  // prediction and details: 1728 = 9 x 192 parent cells
+constexpr int kStencilThreads = 192;  // 2D prediction of large ranges, 2D details
 constexpr int kMaxLevels = 32;
 
 // LDS layout of a parent stencil window: [W][W][W] doubles in 3D, [W][W] in
@@ -424,69 +423,43 @@ __device__ __forceinline__ void predict_range(double *s, double *__restrict__ bl
   }
 }
 
-// Predicts range r (at most 8 predicted parent cells per axis) of every
-// equation of child l.child from its parent, in one workgroup: while the
-// children of equation e are predicted from one LDS window, the parent
-// window of equation e + 1 is loaded into registers and then written to the
-// other window, so the loads overlap the stencil arithmetic.  One barrier
-// per equation; the caller's early exits are uniform over the workgroup.
-template <int DIM> using SmallLds = LdsW<DIM, 12>;
+// 2D: predicts range r (at most 8 predicted parent cells per axis) of every
+// equation of child l.child from its parent, in one workgroup of a wavefront per
+// equation: each loads its field's window (at most 144 cells) and predicts at most
+// one parent cell per lane.  The caller's early exits are uniform over the
+// workgroup.  12,000 links' internal cells 40 us, halo slabs 36 us; 56 and 71
+// with a workgroup walking the equations, a barrier each.
+constexpr int kPredict2Threads = 64 * Dims<2>::NE;
+using Lds2 = LdsW<2, 12>;
 
-template <int DIM>
-__device__ __forceinline__ void predict_range_equations(double *s, double *__restrict__ blocks,
-                                                        const alpaca_mr_link &l, const Range &r) {
-  using D = Dims<DIM>;
-  using L = SmallLds<DIM>;
-  constexpr int K = 12;  // window cells per axis at most
-  static_assert(K * K <= kStencilThreads, "one thread per window column");
-  Window<DIM> const win(r, l.position);
-  const double *parent = blocks + (size_t)l.parent * D::BLOCK;
-  double *child = blocks + (size_t)l.child * D::BLOCK;
-  // Thread (b, c) of the window's w1 x w2 plane moves the column a = 0..w0-1:
-  // field offset g + a SX, LDS offset q + a L::SX.
-  int const plane = win.w[1] * win.w[2];
-  bool const mover = int(threadIdx.x) < plane;
-  int const b = mover ? int(threadIdx.x) / win.w[2] : 0, c = mover ? int(threadIdx.x) % win.w[2] : 0;
-  int const g = win.p0[0] * D::SX + (win.p0[1] + b) * D::SY + (win.p0[2] + c);
-  int const q = b * L::SY + c;
-  int const w0 = win.w[0];
-  double pre[K];
-  auto load = [&](int e) {
-    if (!mover) return;
-    const double *src = parent + (size_t)e * D::FIELD + g;
+__device__ __forceinline__ void predict_range2(double *s, double *__restrict__ blocks,
+                                               const alpaca_mr_link &l, const Range &r) {
+  using D = Dims<2>;
+  Window<2> const win(r, l.position);
+  int const e = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  double *w = s + e * Lds2::SIZE;
+  const double *field = blocks + (size_t)l.parent * D::BLOCK + (size_t)e * D::FIELD;
+  int const n = win.w[0] * win.w[1];
+  constexpr int K = (Lds2::SIZE + 63) / 64;
+  double v[K];
 #pragma unroll
-    for (int a = 0; a < K; ++a)
-      if (a < w0) pre[a] = src[a * D::SX];
-  };
-  auto put = [&](double *w) {
-    if (!mover) return;
-#pragma unroll
-    for (int a = 0; a < K; ++a)
-      if (a < w0) w[q + a * L::SX] = pre[a];
-  };
-  load(0);
-  put(s);
-  __syncthreads();
-  int const nz = DIM == 3 ? r.count[2] : 1;
-  int const tasks = r.count[0] * r.count[1] * nz;
-#pragma unroll 1
-  for (int e = 0; e < D::NE; ++e) {
-    if (e + 1 < D::NE) load(e + 1);
-    const double *cur = s + (e & 1) * L::SIZE;
-    double *out = child + (size_t)e * D::FIELD;
-    for (int t = threadIdx.x; t < tasks; t += kStencilThreads) {
-      int const a = t / (r.count[1] * nz), b = (t / nz) % r.count[1], c = t % nz;
-      double v[1 << DIM];
-      predict_cell<L>(cur, Window<DIM>::template centre<L>(a, b, c), v);
-      int const ci = r.start[0] + 2 * a, cj = r.start[1] + 2 * b;
-      int const ck = DIM == 3 ? r.start[2] + 2 * c : 0;
-      store_children<DIM>(out + ci * D::SX + cj * D::SY + ck, v);
-    }
-    // The other window was last read by equation e - 1, before the previous
-    // barrier.
-    if (e + 1 < D::NE) put(s + ((e + 1) & 1) * L::SIZE);
-    __syncthreads();
+  for (int k = 0; k < K; ++k) {
+    int const t = lane + 64 * k;
+    if (t < n) v[k] = field[(win.p0[0] + t / win.w[1]) * D::SX + (win.p0[1] + t % win.w[1]) * D::SY];
   }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    int const t = lane + 64 * k;
+    if (t < n) w[(t / win.w[1]) * Lds2::SX + (t % win.w[1]) * Lds2::SY] = v[k];
+  }
+  __syncthreads();
+  if (lane >= r.count[0] * r.count[1]) return;
+  int const a = lane / r.count[1], b = lane % r.count[1];
+  double c[4];
+  predict_cell<Lds2>(w, Window<2>::centre<Lds2>(a, b, 0), c);
+  store_children<2>(blocks + (size_t)l.child * D::BLOCK + (size_t)e * D::FIELD +
+                        (r.start[0] + 2 * a) * D::SX + (r.start[1] + 2 * b) * D::SY,
+                    c);
 }
 
 // Ranges whose window fits the 12-cell layout: at most 8 predicted parent
@@ -495,15 +468,13 @@ __host__ __device__ inline bool small_window(const Range &r) {
   return r.count[0] <= 8 && r.count[1] <= 8 && r.count[2] <= 8;
 }
 
-// prediction_kernel<DIM, false> over ranges with small windows: one
-// workgroup per link, every equation.
-template <int DIM>
-__global__ __launch_bounds__(kStencilThreads) void prediction_small_kernel(
+// 2D ranges with small windows: one workgroup per link, every equation.
+__global__ __launch_bounds__(kPredict2Threads) void prediction2_kernel(
     double *__restrict__ blocks, int nblocks, const alpaca_mr_link *__restrict__ links, Range r) {
-  __shared__ double s[2 * SmallLds<DIM>::SIZE];
+  __shared__ double s[Dims<2>::NE * Lds2::SIZE];
   alpaca_mr_link const l = links[blockIdx.x];
-  if (!link_ok<DIM>(l, nblocks)) return;
-  predict_range_equations<DIM>(s, blocks, l, r);
+  if (!link_ok<2>(l, nblocks)) return;
+  predict_range2(s, blocks, l, r);
 }
 
 template <int DIM, bool FULL>
@@ -549,16 +520,14 @@ template <int DIM> __device__ __forceinline__ bool location_range(int loc, Range
 // UpdateMaterialJumpNoMpi (internal_halo_manager.cpp:231-262) for a batch:
 // link i's child gets the halo slab of location locations[i] predicted from
 // its parent (every equation), one workgroup per link.
-template <int DIM>
-__global__ __launch_bounds__(kStencilThreads) void jump_halo_kernel(
+__global__ __launch_bounds__(kPredict2Threads) void jump_halo2_kernel(
     double *__restrict__ blocks, int nblocks, const alpaca_mr_link *__restrict__ links,
     const int *__restrict__ locations) {
-  __shared__ double s[2 * SmallLds<DIM>::SIZE];
-  int const i = blockIdx.x;
-  alpaca_mr_link const l = links[i];
+  __shared__ double s[Dims<2>::NE * Lds2::SIZE];
+  alpaca_mr_link const l = links[blockIdx.x];
   Range r;
-  if (!link_ok<DIM>(l, nblocks) || !location_range<DIM>(locations[i], r)) return;
-  predict_range_equations<DIM>(s, blocks, l, r);
+  if (!link_ok<2>(l, nblocks) || !location_range<2>(locations[blockIdx.x], r)) return;
+  predict_range2(s, blocks, l, r);
 }
 
 // ------------------------------------------------------------ 3D predictions
@@ -688,7 +657,7 @@ __global__ __launch_bounds__((kPredictThreads<W, N>)) __attribute__((amdgpu_wave
   predict_field3<kPredictThreads<W, N>, W, N>(s, blocks, l, int(g % NE), r, threadIdx.x);
 }
 
-// The jump halos of 3D links (jump_halo_kernel): a slab has at most 64 pairs of
+// The jump halos of 3D links (jump_halo2_kernel in 2D): a slab has at most 64 pairs of
 // parent cells, so one wavefront per (link, equation).
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) void jump_halo3_kernel(double *__restrict__ blocks, int nblocks,
                                                         const alpaca_mr_link *__restrict__ links,
@@ -887,8 +856,8 @@ template <int DIM> int prediction_impl(double *blocks, int nblocks, const alpaca
       hipLaunchKernelGGL((prediction3_kernel<16, 0>), grid, dim3(kPredictThreads<16, 0>), 0, s,
                          blocks, nblocks, links, r);
   } else if (small_window(r)) {
-    hipLaunchKernelGGL((prediction_small_kernel<DIM>), dim3((unsigned)nlinks),
-                       dim3(kStencilThreads), 0, s, blocks, nblocks, links, r);
+    hipLaunchKernelGGL(prediction2_kernel, dim3((unsigned)nlinks), dim3(kPredict2Threads), 0, s,
+                       blocks, nblocks, links, r);
   } else if (all(12)) {
     hipLaunchKernelGGL((prediction_kernel<DIM, true>), grid, dim3(kStencilThreads), 0, s, blocks,
                        nblocks, links, r);
@@ -905,8 +874,8 @@ template <int DIM> int jump_halo_impl(double *blocks, int nblocks, const alpaca_
     hipLaunchKernelGGL(jump_halo3_kernel, dim3((unsigned)nlinks * Dims<3>::NE), dim3(64), 0, s, blocks,
                        nblocks, links, locations);
   else
-    hipLaunchKernelGGL((jump_halo_kernel<DIM>), dim3((unsigned)nlinks), dim3(kStencilThreads), 0, s,
-                       blocks, nblocks, links, locations);
+    hipLaunchKernelGGL(jump_halo2_kernel, dim3((unsigned)nlinks), dim3(kPredict2Threads), 0, s, blocks,
+                       nblocks, links, locations);
   return hip_status(hipGetLastError());
 }
 
