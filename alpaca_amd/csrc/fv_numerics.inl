@@ -1050,12 +1050,26 @@ template <int DIM, int DIR> struct LeanEig {
 
 template <int DIM, int DIR, typename QS>
 __device__ __forceinline__ void fv_reconstruct_lean(double gamma, const double (&U)[6][DIM + 2],
-                                                    const QS &qs, double *cl, double *cr) {
+                                                    const QS &qs, double *cl, double *cr,
+                                                    double &skipped) {
   LeanEig<DIM, DIR> ev;
   if (!ev.form(gamma, qs.left(U[2]), qs.right(U[3]))) {
-    // A zero state, whose face is skipped.
+    // Zero eigenvectors: zero states, whose face is skipped, or NaN where a value of a
+    // state's five cells is not finite (as their products with zeros are), and a flux
+    // of NaN where both states are.
+    double l = 0.0, r = 0.0;
 #pragma unroll
-    for (int e = 0; e < DIM + 2; ++e) cl[e] = cr[e] = 0.0;
+    for (int e = 0; e < DIM + 2; ++e) {
+      cl[e] = cr[e] = 0.0;
+      l += 0.0 * U[0][e];
+      r += 0.0 * U[5][e];
+#pragma unroll
+      for (int m = 1; m < 5; ++m) {
+        l += 0.0 * U[m][e];
+        r += 0.0 * U[m][e];
+      }
+    }
+    skipped = l == l ? 0.0 : r;
     return;
   }
   double Y[6], B[6], lo[DIM + 2], hi[DIM + 2];
@@ -1099,12 +1113,39 @@ __device__ __forceinline__ void roe_split_flux_lean(double gamma, double b,
     for (int e = 0; e < NE; ++e)
       c[e] = base[e * Dims<DIM>::FIELD + (m - 2) * axis_stride<DIM, DIR>()];
   };
+  // A stencil cell's conservatives and advection.
+  auto cell = [&](int m, double *U, double *adv) {
+    load(m, U);
+    double const one = fdiv(1.0, U[kMass]), ud = U[E::Mp] * one;
+    double k = U[E::Mp] * ud + U[E::M1] * (U[E::M1] * one);
+    if constexpr (DIM == 3) k += U[E::M2] * (U[E::M2] * one);
+    double const p = (gamma - 1.0) * (U[kEnergy] - 0.5 * k) - gamma * b;
+    adv[kMass] = U[E::Mp];
+    adv[kEnergy] = (U[kEnergy] + p) * ud;
+    adv[E::Mp] = U[E::Mp] * ud + p;
+    adv[E::M1] = U[E::M1] * ud;
+    if constexpr (DIM == 3) adv[E::M2] = U[E::M2] * ud;
+  };
   E ev;
   {
     double Ui[NE], Un[NE];
     load(2, Ui);
     load(3, Un);
-    if (!ev.form(gamma, qs.left(Ui), qs.right(Un))) return;
+    if (!ev.form(gamma, qs.left(Ui), qs.right(Un))) {
+      // Zero eigenvectors: no flux, or NaN where a value of the six cells is not finite
+      // (as their products with zeros are).
+      double z = 0.0;
+#pragma unroll 1
+      for (int m = 0; m < 6; ++m) {
+        double U[NE], adv[NE];
+        cell(m, U, adv);
+#pragma unroll
+        for (int e = 0; e < NE; ++e) z += 0.0 * U[e] + 0.0 * adv[e];
+      }
+#pragma unroll
+      for (int e = 0; e < NE; ++e) f[e] += z;
+      return;
+    }
   }
   double const lam = __builtin_fabs(ev.u), lam_lo = __builtin_fabs(ev.u - ev.c),
                lam_hi = __builtin_fabs(ev.u + ev.c);
@@ -1112,16 +1153,7 @@ __device__ __forceinline__ void roe_split_flux_lean(double gamma, double b,
 #pragma unroll
   for (int m = 0; m < 6; ++m) {
     double U[NE], adv[NE];
-    load(m, U);
-    double const one = fdiv(1.0, U[kMass]), ud = U[E::Mp] * one;
-    double k = U[E::Mp] * ud + U[E::M1] * (U[E::M1] * one);
-    if constexpr (DIM == 3) k += U[E::M2] * (U[E::M2] * one);
-    double const p = ev.g * (U[kEnergy] - 0.5 * k) - gamma * b;
-    adv[kMass] = U[E::Mp];
-    adv[kEnergy] = (U[kEnergy] + p) * ud;
-    adv[E::Mp] = U[E::Mp] * ud + p;
-    adv[E::M1] = U[E::M1] * ud;
-    if constexpr (DIM == 3) adv[E::M2] = U[E::M2] * ud;
+    cell(m, U, adv);
     double uY, uB, u1, u2, aY, aB, a1, a2;
     ev.parts(U, uY, uB, u1, u2);
     ev.parts(adv, aY, aB, a1, a2);
@@ -1168,11 +1200,11 @@ __device__ __forceinline__ double nr_sqrt64_pos(double x) {
 // sound speed.  Five divisions per face instead of twelve.
 template <int DIM, int DIR>
 __device__ __forceinline__ void fv_riemann_lean(double gamma, double b, const double *cl,
-                                                const double *cr, double *f) {
+                                                const double *cr, double skipped, double *f) {
   constexpr int NE = DIM + 2;
   constexpr int Mp = kMomX + DIR, M1 = kMomX + Minor<DIR>::m1, M2 = kMomX + Minor<DIR>::m2;
 #pragma unroll
-  for (int e = 0; e < NE; ++e) f[e] = 0.0;
+  for (int e = 0; e < NE; ++e) f[e] = skipped;
   double const eps = 2.220446049250313080847263336181640625e-16;  // DBL_EPSILON
   if (cl[kMass] <= eps || cr[kMass] <= eps) return;
   auto pressure = [&](const double *c, double one_rho, double &u) {
@@ -1215,12 +1247,14 @@ __device__ __forceinline__ void fv_riemann_lean(double gamma, double b, const do
 // finite_volume_scheme.cpp:160-251, with CharacteristicStateReconstruction,
 // characteristic_state_reconstruction.h:60-134) in two parts: fv_reconstruct
 // forms the states cl and cr left and right of the face from its stencil Ud
-// (FP64 conservatives of cells i-2..i+3 along DIR), fv_riemann the flux.
+// (FP64 conservatives of cells i-2..i+3 along DIR), fv_riemann the flux.  `skipped`
+// passes the flux of a face without an eigensystem.
 template <int DIM, int DIR, typename R, typename QS>
 __device__ __forceinline__ void fv_reconstruct(double gamma64, const double (&Ud)[6][DIM + 2],
-                                               const QS &qs, R *cl, R *cr) {
+                                               const QS &qs, R *cl, R *cr, R &skipped) {
+  skipped = R(0.0);
   if constexpr (kLean<R>) {
-    fv_reconstruct_lean<DIM, DIR>(gamma64, Ud, qs, cl, cr);
+    fv_reconstruct_lean<DIM, DIR>(gamma64, Ud, qs, cl, cr, skipped);
     return;
   }
   R const gamma = R(gamma64);
@@ -1311,9 +1345,9 @@ __device__ __forceinline__ void load_stencil(const BlockReader<DIM> &rd, int off
 // Writes f (zero when the reference skips the face).
 template <int DIM, int DIR, typename R>
 __device__ __forceinline__ void fv_riemann(double gamma64, double b64, const R *cl, const R *cr,
-                                           R *f) {
+                                           R skipped, R *f) {
   if constexpr (kLean<R>) {
-    fv_riemann_lean<DIM, DIR>(gamma64, b64, cl, cr, f);
+    fv_riemann_lean<DIM, DIR>(gamma64, b64, cl, cr, skipped, f);
     return;
   }
   constexpr int NE = DIM + 2;
@@ -1338,9 +1372,9 @@ __device__ __forceinline__ void fv_face(double gamma64, double b64, const double
   BlockReader<DIM> const rd(blk);
   double Ud[6][DIM + 2];
   load_stencil<DIM>(rd, off, axis_stride<DIM, DIR>(), Ud);
-  R cl[DIM + 2], cr[DIM + 2];
-  fv_reconstruct<DIM, DIR, R>(gamma64, Ud, qs, cl, cr);
-  fv_riemann<DIM, DIR, R>(gamma64, b64, cl, cr, f);
+  R cl[DIM + 2], cr[DIM + 2], skipped;
+  fv_reconstruct<DIM, DIR, R>(gamma64, Ud, qs, cl, cr, skipped);
+  fv_riemann<DIM, DIR, R>(gamma64, b64, cl, cr, skipped, f);
 }
 
 // The conservatives of one cell.

@@ -439,12 +439,12 @@ __device__ __forceinline__ void stage_march(const TileJob &j, int blk_local, int
       KeptQ<3, R, P> const qs{inner ? (yj > 0 ? q + t - kIC : HQ + p * kIC + yk) : Q + t,
                               inner ? q + t : Q + NQ * P + t};
       if constexpr (AHEAD) {
-        R cl[NE], cr[NE];
-        fv_reconstruct<3, 1, R>(j.gamma, U, qs, cl, cr);
+        R cl[NE], cr[NE], skipped;
+        fv_reconstruct<3, 1, R>(j.gamma, U, qs, cl, cr, skipped);
         int off = here(t, p) - 1;
         after(off, cl[NE - 1], cr[NE - 1]);
         load_stencil<3>(rd, off, 1, U);
-        fv_riemann<3, 1, R>(j.gamma, j.b, cl, cr, fl);
+        fv_riemann<3, 1, R>(j.gamma, j.b, cl, cr, skipped, fl);
       } else {
         int const off = inner ? here(t, p) - D::SY : closing(t, false);
         face_flux<3, 1, FLUX, R>(j.gamma, j.b, bb, off, qs, fl);
@@ -463,15 +463,15 @@ __device__ __forceinline__ void stage_march(const TileJob &j, int blk_local, int
                               inner ? q + t : Q + NQ * P + t};
       if constexpr (AHEAD) {
         if (!inner) load_stencil<3>(rd, closing(t, true), 1, U);
-        R cl[NE], cr[NE];
-        fv_reconstruct<3, 2, R>(j.gamma, U, qs, cl, cr);
+        R cl[NE], cr[NE], skipped;
+        fv_reconstruct<3, 2, R>(j.gamma, U, qs, cl, cr, skipped);
         int off = here(t, p);
         after(off, cl[NE - 1], cr[NE - 1]);
         if constexpr (COLUMN)
           load_cell<3>(rd, off + 3 * D::SX, X[5]);
         else
           load_stencil<3>(rd, off, D::SX, U);
-        fv_riemann<3, 2, R>(j.gamma, j.b, cl, cr, fl);
+        fv_riemann<3, 2, R>(j.gamma, j.b, cl, cr, skipped, fl);
       } else {
         int const off = inner ? here(t, p) - 1 : closing(t, true);
         face_flux<3, 2, FLUX, R>(j.gamma, j.b, bb, off, qs, fl);
@@ -492,8 +492,8 @@ __device__ __forceinline__ void stage_march(const TileJob &j, int blk_local, int
       KeptThenFormedQ<3, R, P> const qs{j.gamma, j.b, Q + (p & 1) * NQ * P + t,
                                         Q + ((p + 1) & 1) * NQ * P + t};
       if constexpr (AHEAD) {
-        R cl[NE], cr[NE];
-        fv_reconstruct<3, 0, R>(j.gamma, COLUMN ? X : U, qs, cl, cr);
+        R cl[NE], cr[NE], skipped;
+        fv_reconstruct<3, 0, R>(j.gamma, COLUMN ? X : U, qs, cl, cr, skipped);
         if constexpr (COLUMN) {
 #pragma unroll
           for (int m = 0; m < 5; ++m)
@@ -503,7 +503,7 @@ __device__ __forceinline__ void stage_march(const TileJob &j, int blk_local, int
         int off = here(t, p) + D::SX - D::SY;
         after(off, cl[NE - 1], cr[NE - 1]);
         load_stencil<3>(rd, off, D::SY, U);
-        fv_riemann<3, 0, R>(j.gamma, j.b, cl, cr, fh);
+        fv_riemann<3, 0, R>(j.gamma, j.b, cl, cr, skipped, fh);
       } else {
         face_flux<3, 0, FLUX, R>(j.gamma, j.b, bb, here(t, p), qs, fh);
       }
