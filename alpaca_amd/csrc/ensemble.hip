@@ -14,9 +14,9 @@
 //                           stage 2 also reduces the next signal).
 // ens_finish_kernel ends a call's last step: per-case FinishMacroTimestep and the
 // stop conditions (t_end reached, unhealthy step).
-// Work lists and case slots live in device memory, so the graph stays valid
-// while cases come and go; only the tuning (tile shape, groups per CU)
-// re-captures it.  Each case's arithmetic depends only on its own blocks and
+// Work lists and case slots live in device memory, so the graphs stay valid
+// while cases come and go: one per class and tile shape, captured on first use,
+// until the tuning changes the groups per CU.  Each case's arithmetic depends only on its own blocks and
 // record, so results are identical alone and in any mix.
 #include <hip/hip_runtime.h>
 
@@ -501,12 +501,16 @@ int alpaca_ensemble_create_shared(alpaca_ensemble *peer, int dim, int max_cases,
   auto *e = new (std::nothrow) alpaca_ensemble();
   if (!e) return ALPACA_ERR_CAPACITY;
   {
-    std::lock_guard<std::mutex> lock(peer->pool->mu);
-    peer->pool->refs += 1;
+    std::lock_guard<std::mutex> lock(peer->mu);
+    {
+      std::lock_guard<std::mutex> pool(peer->pool->mu);
+      peer->pool->refs += 1;
+    }
+    // Ranges that the peer released while it had the pool alone may still be in use by
+    // steps on its stream (which another thread's step() may be capturing unless it is
+    // held off).
+    (void)hipStreamSynchronize(peer->stream);
   }
-  // Ranges that the peer released while it had the pool alone may still be in use by
-  // steps on its stream.
-  (void)hipStreamSynchronize(peer->stream);
   e->pool = peer->pool;
   if (ensemble_init(e, peer->pool, dim, max_cases, class_mask, static_cast<hipStream_t>(stream)) !=
       ALPACA_OK) {
@@ -620,7 +624,11 @@ int alpaca_ensemble_remove_case(alpaca_ensemble *e, int case_id) {
 }
 
 int alpaca_ensemble_cancel_case(alpaca_ensemble *e, int case_id) {
-  if (!e || case_id < 0 || case_id >= e->max_cases || !e->h_active[case_id]) return ALPACA_ERR_INVALID;
+  if (!e || case_id < 0 || case_id >= e->max_cases) return ALPACA_ERR_INVALID;
+  // Under the lock, as every call that queues work: during a step() of another thread
+  // the stream's tail lies between a step's stages and its end, which alone counts it.
+  std::lock_guard<std::mutex> lock(e->mu);
+  if (!e->h_active[case_id]) return ALPACA_ERR_INVALID;
   hipLaunchKernelGGL(ens_set_flags_kernel, dim3(1), dim3(64), 0, e->stream, e->d_states, case_id,
                      kFlagCancelled, 0);
   return hip_ok(hipGetLastError());
@@ -655,24 +663,29 @@ int alpaca_ensemble_step(alpaca_ensemble *e, int nsteps) {
 
 int alpaca_ensemble_read_states(alpaca_ensemble *e, alpaca_case_state *host_out, int n) {
   if (!e || !host_out || n < 0 || n > e->max_cases) return ALPACA_ERR_INVALID;
-  if (hipMemcpyAsync(host_out, e->d_states, sizeof(alpaca_case_state) * n, hipMemcpyDeviceToHost,
-                     e->stream) != hipSuccess)
-    return ALPACA_ERR_HIP;
+  {
+    std::lock_guard<std::mutex> lock(e->mu);
+    if (hipMemcpyAsync(host_out, e->d_states, sizeof(alpaca_case_state) * n, hipMemcpyDeviceToHost,
+                       e->stream) != hipSuccess)
+      return ALPACA_ERR_HIP;
+  }
   return hip_ok(hipStreamSynchronize(e->stream));
 }
 
 int alpaca_ensemble_case_blocks(alpaca_ensemble *e, int case_id, double **d_blocks, int *nblocks) {
-  if (!e || !d_blocks || !nblocks || case_id < 0 || case_id >= e->max_cases ||
-      !e->h_active[case_id])
+  if (!e || !d_blocks || !nblocks || case_id < 0 || case_id >= e->max_cases)
     return ALPACA_ERR_INVALID;
+  std::lock_guard<std::mutex> lock(e->mu);
+  if (!e->h_active[case_id]) return ALPACA_ERR_INVALID;
   *d_blocks = e->u + (size_t)e->h_slots[case_id].base * alpaca_block_doubles(e->dim);
   *nblocks = e->h_slots[case_id].nblocks;
   return ALPACA_OK;
 }
 
 int alpaca_ensemble_copy_case(alpaca_ensemble *e, int case_id, double *d_dst) {
-  if (!e || !d_dst || case_id < 0 || case_id >= e->max_cases || !e->h_active[case_id])
-    return ALPACA_ERR_INVALID;
+  if (!e || !d_dst || case_id < 0 || case_id >= e->max_cases) return ALPACA_ERR_INVALID;
+  std::lock_guard<std::mutex> lock(e->mu);
+  if (!e->h_active[case_id]) return ALPACA_ERR_INVALID;
   CaseSlot const &cs = e->h_slots[case_id];
   return hip_ok(hipMemcpyAsync(d_dst, e->u + (size_t)cs.base * alpaca_block_doubles(e->dim),
                                block_bytes(e->dim) * cs.nblocks, hipMemcpyDeviceToDevice,

@@ -344,7 +344,9 @@ int alpaca_advance(const alpaca_case_desc *desc, double *d_u, double *d_s1,
  * arithmetic; the classes run side by side through a call),
  * replayed from a captured hipGraph.  A case's results do not
  * depend on what else runs: per-case reductions only, fixed arithmetic order.
- * The ensemble owns its device memory (allocated at create).
+ * The ensemble owns its device memory (allocated at create).  Host threads may
+ * share an ensemble: its calls take effect one after the other, each as a whole
+ * (a record read or a cancellation falls between alpaca_ensemble_step calls).
  *
  * Class bit for (flux, precision): 1 << (3*flux + m), m = 0 for ALPACA_FP64,
  * 1 for ALPACA_FP64_FMA, 2 for ALPACA_MIXED.
@@ -385,8 +387,9 @@ int alpaca_ensemble_add_case(alpaca_ensemble *e, const alpaca_case_desc *desc,
                              int *case_id);
 /* Releases a case's slot and blocks (read its blocks first). */
 int alpaca_ensemble_remove_case(alpaca_ensemble *e, int case_id);
-/* Stops a case at the next stage boundary (the ABORTFILE analogue,
- * input_output_manager.h:197-199). */
+/* Stops a case (the ABORTFILE analogue, input_output_manager.h:197-199): the
+ * steps of earlier alpaca_ensemble_step calls still run, those of later calls
+ * leave it as it is. */
 int alpaca_ensemble_cancel_case(alpaca_ensemble *e, int case_id);
 /* Tile shape (3D: 0 = 8x8x8/256 threads, 1 = 16x8x8/512; 2D: 0 = 16x16/128,
  * 1 = 16x16/256, 2 = 16x8/128) and persistent workgroups per CU (0 = the
