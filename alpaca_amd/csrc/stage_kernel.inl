@@ -693,7 +693,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kMinWaves<DI
   double *jb = jump ? jump + (size_t)blk * SURF : nullptr;
   tile_faces<DIM, FLUX, R, TX, TY, TZ, NT>(threadIdx.x, avg + (size_t)blk * D::BLOCK, x0, y0, z0, gamma,
                                            b, lds);
-  if (DIM == 2 && jb) {
+  if (DIM == 2 && jb && tile == 0) {  // one workgroup per block: others' would race
     for (int t = threadIdx.x; t < 2 * NE * kIC; t += NT) jb[4 * NE * kIC + t] += 0.0;
   }
   __syncthreads();
