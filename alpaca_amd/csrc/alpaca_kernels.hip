@@ -630,15 +630,21 @@ int stream_context(hipStream_t s, alpaca_context **out) {
   return ALPACA_OK;
 }
 
+// ALPACA_OK if the context belongs to the current device.
+int on_context_device(const alpaca_context *c) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return ALPACA_ERR_HIP;
+  return dev == c->device ? ALPACA_OK : ALPACA_ERR_INVALID;
+}
+
 // Face-flux scratch of at least `bytes` from a context on the current
 // device.  A buffer that is too small is retired, not freed: work already
 // queued on the context's stream may still read it, and freeing it here would
 // need a device synchronisation.  Growth is geometric, so the retired
 // buffers together stay below the live one.
 int context_scratch(alpaca_context *c, size_t bytes, double **out) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return ALPACA_ERR_HIP;
-  if (dev != c->device) return ALPACA_ERR_INVALID;
+  int const st = on_context_device(c);
+  if (st != ALPACA_OK) return st;
   std::lock_guard<std::mutex> lock(c->mutex);
   if (c->bytes < bytes) {
     size_t const grown = std::max(bytes, c->bytes + c->bytes / 2);
@@ -1034,6 +1040,7 @@ int alpaca_ctx_right_hand_side(alpaca_context *ctx, const alpaca_case_desc *desc
   if (st != ALPACA_OK) return st;
   if (!ctx || nblocks < 1 || nblocks > kMaxBlocks || !d_avg || !d_rhs || d_avg == d_rhs)
     return ALPACA_ERR_INVALID;
+  if ((st = on_context_device(ctx)) != ALPACA_OK) return st;
   return right_hand_side(desc, nblocks, d_avg, d_rhs, nullptr, ctx->stream);
 }
 
@@ -1045,6 +1052,7 @@ int alpaca_ctx_right_hand_side_jump_fluxes(alpaca_context *ctx, const alpaca_cas
   if (!ctx || nblocks < 1 || nblocks > kMaxBlocks || !d_avg || !d_rhs || !d_jump_fluxes ||
       d_avg == d_rhs)
     return ALPACA_ERR_INVALID;
+  if ((st = on_context_device(ctx)) != ALPACA_OK) return st;
   return right_hand_side(desc, nblocks, d_avg, d_rhs, d_jump_fluxes, ctx->stream);
 }
 
