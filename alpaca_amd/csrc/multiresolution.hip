@@ -21,6 +21,7 @@
 // children of one parent cell in 2D, of two adjacent along z in 3D.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 
 #include "fv_device.h"
@@ -836,62 +837,66 @@ template <int DIM> int average_jump_impl(double *surfaces, int nblocks, const al
   return hip_status(hipGetLastError());
 }
 
+// f(first, n) over all links in launches of at most as many as the hardware can count
+// the threads of (below 2^32), `threads` a link.
+template <typename F> void in_launches(int nlinks, int threads, const F &f) {
+  int const most = int(0xffffffffu / (unsigned)threads);
+  for (long long first = 0; first < nlinks; first += most)
+    f(int(first), (int)std::min<long long>(most, nlinks - first));
+}
+
 template <int DIM> int prediction_impl(double *blocks, int nblocks, const alpaca_mr_link *links,
                                        int nlinks, const Range &r, hipStream_t s) {
-  dim3 const grid((unsigned)nlinks * Dims<DIM>::NE);
+  constexpr int NE = Dims<DIM>::NE;
   auto all = [&r](int n) {
     return r.count[0] == n && r.count[1] == n && r.count[2] == (DIM == 3 ? n : 1);
   };
+  // `groups` workgroups of nt threads per link.
+  auto launch = [&](auto kernel, int groups, int nt) {
+    in_launches(nlinks, groups * nt, [&](int first, int n) {
+      hipLaunchKernelGGL(kernel, dim3((unsigned)n * groups), dim3(nt), 0, s, blocks, nblocks,
+                         links + first, r);
+    });
+  };
   if constexpr (DIM == 3) {
     if (all(8) && r.start[0] == kHS && r.start[1] == kHS && r.start[2] == kHS)
-      hipLaunchKernelGGL((prediction3_kernel<12, 8>), grid, dim3(kPredictThreads<12, 8>), 0, s,
-                         blocks, nblocks, links, r);
+      launch(prediction3_kernel<12, 8>, NE, kPredictThreads<12, 8>);
     else if (all(12))
-      hipLaunchKernelGGL((prediction3_kernel<16, 12>), grid, dim3(kPredictThreads<16, 12>), 0, s,
-                         blocks, nblocks, links, r);
+      launch(prediction3_kernel<16, 12>, NE, kPredictThreads<16, 12>);
     else if (small_window(r))
-      hipLaunchKernelGGL((prediction3_kernel<12, 0>), grid, dim3(kPredictThreads<12, 0>), 0, s,
-                         blocks, nblocks, links, r);
+      launch(prediction3_kernel<12, 0>, NE, kPredictThreads<12, 0>);
     else
-      hipLaunchKernelGGL((prediction3_kernel<16, 0>), grid, dim3(kPredictThreads<16, 0>), 0, s,
-                         blocks, nblocks, links, r);
+      launch(prediction3_kernel<16, 0>, NE, kPredictThreads<16, 0>);
   } else if (small_window(r)) {
-    hipLaunchKernelGGL(prediction2_kernel, dim3((unsigned)nlinks), dim3(kPredict2Threads), 0, s,
-                       blocks, nblocks, links, r);
+    launch(prediction2_kernel, 1, kPredict2Threads);
   } else if (all(12)) {
-    hipLaunchKernelGGL((prediction_kernel<DIM, true>), grid, dim3(kStencilThreads), 0, s, blocks,
-                       nblocks, links, r);
+    launch(prediction_kernel<DIM, true>, NE, kStencilThreads);
   } else {
-    hipLaunchKernelGGL((prediction_kernel<DIM, false>), grid, dim3(kStencilThreads), 0, s, blocks,
-                       nblocks, links, r);
+    launch(prediction_kernel<DIM, false>, NE, kStencilThreads);
   }
   return hip_status(hipGetLastError());
 }
 
 template <int DIM> int jump_halo_impl(double *blocks, int nblocks, const alpaca_mr_link *links,
                                       const int *locations, int nlinks, hipStream_t s) {
-  if constexpr (DIM == 3)
-    hipLaunchKernelGGL(jump_halo3_kernel, dim3((unsigned)nlinks * Dims<3>::NE), dim3(64), 0, s, blocks,
-                       nblocks, links, locations);
-  else
-    hipLaunchKernelGGL(jump_halo2_kernel, dim3((unsigned)nlinks), dim3(kPredict2Threads), 0, s, blocks,
-                       nblocks, links, locations);
+  constexpr int groups = DIM == 3 ? Dims<3>::NE : 1, nt = DIM == 3 ? 64 : kPredict2Threads;
+  in_launches(nlinks, groups * nt, [&](int first, int n) {
+    hipLaunchKernelGGL(DIM == 3 ? jump_halo3_kernel : jump_halo2_kernel, dim3((unsigned)n * groups),
+                       dim3(nt), 0, s, blocks, nblocks, links + first, locations + first);
+  });
   return hip_status(hipGetLastError());
 }
 
 template <int DIM> int details_impl(const double *blocks, int nblocks, const alpaca_mr_link *links,
                                     int nlinks, int norm, const Thresholds &th, double *details,
                                     int *decisions, hipStream_t s) {
-  dim3 const grid((unsigned)nlinks), block(kDetailThreads<DIM>);
-  if (norm == ALPACA_MR_NORM_L1)
-    hipLaunchKernelGGL((details_kernel<DIM, 1>), grid, block, 0, s, blocks, nblocks, links, th,
-                       details, decisions);
-  else if (norm == ALPACA_MR_NORM_L2)
-    hipLaunchKernelGGL((details_kernel<DIM, 2>), grid, block, 0, s, blocks, nblocks, links, th,
-                       details, decisions);
-  else
-    hipLaunchKernelGGL((details_kernel<DIM, 0>), grid, block, 0, s, blocks, nblocks, links, th,
-                       details, decisions);
+  auto kernel = norm == ALPACA_MR_NORM_L1   ? details_kernel<DIM, 1>
+                : norm == ALPACA_MR_NORM_L2 ? details_kernel<DIM, 2>
+                                            : details_kernel<DIM, 0>;
+  in_launches(nlinks, kDetailThreads<DIM>, [&](int first, int n) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)n), dim3(kDetailThreads<DIM>), 0, s, blocks, nblocks,
+                       links + first, th, details + first, decisions ? decisions + first : nullptr);
+  });
   return hip_status(hipGetLastError());
 }
 
