@@ -59,7 +59,7 @@ template <int DIM, typename F> void with_shape(long long n, long long cus, bool 
       f(ShapeTag<8, 8, 8, 512>{});
     else if (16 * n <= 3 * cus)
       f(ShapeTag<8, 8, 4, 512>{});
-    else if (wide)
+    else if (wide && n < (1 << 20))  // a launch counts fewer than 2^32 threads
       f(ShapeTag<8, 8, 8, 512>{});
     else
       f(ShapeTag<8, 8, 8, 256>{});
