@@ -638,9 +638,9 @@ __device__ __forceinline__ void predict_field3(double *s, double *__restrict__ b
 
 // One workgroup per (link, equation), the equations and siblings of a parent
 // on one XCD.  N = 8 (the internal cells): 256 threads, one pair each; N = 12 (the
-// whole block): 448 threads, two each; N = 0: any range.  A workgroup stages one
-// field, so others' arithmetic covers its loads.  Bound by the writes: without
-// them 2560 links' internal cells take 118 us.
+// whole block): 448 threads, two each; N = 0: any other of at most 8 cells per axis.
+// A workgroup stages one field, so others' arithmetic covers its loads.  Bound by the
+// writes: without them 2560 links' internal cells take 118 us.
 template <int W, int N> constexpr int kPredictThreads = W == 12 ? 256 : 448;
 
 template <int W, int N>
@@ -656,6 +656,29 @@ __global__ __launch_bounds__((kPredictThreads<W, N>)) __attribute__((amdgpu_wave
     for (int a = 0; a < 3; ++a) r.count[a] = N;
   }
   predict_field3<kPredictThreads<W, N>, W, N>(s, blocks, l, int(g % NE), r, threadIdx.x);
+}
+
+// Ranges of more than 8 predicted cells along an axis, but for the whole block: as
+// prediction3_kernel, with LDS for the part of the layout that the range's window
+// reaches.  A range of few pairs is one load, one barrier and one pair deep, and what
+// counts is how many of its workgroups a CU holds: with the whole layout (32 KB) and
+// 448 threads it held two.  960 links, us, with a workgroup of 192 threads a thread per
+// cell, with 448 threads, and so: 1 x 1 x 12 parent cells 23.4, 37.0, 20.2, 2 x 2 x 12 25.9,
+// 36.9, 19.2, 4 x 4 x 12 45.2, 47.7, 33.8, 9 x 9 x 9 190, 141, 148, 11 x 11 x 11 279, 208, 218.
+constexpr int kRangeThreads = 256;
+constexpr size_t range_lds_bytes(const Range &r) {
+  return sizeof(double) *
+         ((r.count[0] + 3) * Lds<3>::SX + (r.count[1] + 3) * Lds<3>::SY + Lds<3>::SY);
+}
+
+__global__ __launch_bounds__(kRangeThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) void prediction3_range_kernel(
+    double *__restrict__ blocks, int nblocks, const alpaca_mr_link *__restrict__ links, Range r) {
+  constexpr int NE = Dims<3>::NE;
+  extern __shared__ __align__(16) double window[];
+  unsigned const g = xcd_remap_group(blockIdx.x, gridDim.x);
+  alpaca_mr_link const l = links[g / NE];
+  if (!link_ok<3>(l, nblocks)) return;
+  predict_field3<kRangeThreads, 16, 0>(window, blocks, l, int(g % NE), r, threadIdx.x);
 }
 
 // The jump halos of 3D links (jump_halo2_kernel in 2D): a slab has at most 64 pairs of
@@ -851,10 +874,10 @@ template <int DIM> int prediction_impl(double *blocks, int nblocks, const alpaca
   auto all = [&r](int n) {
     return r.count[0] == n && r.count[1] == n && r.count[2] == (DIM == 3 ? n : 1);
   };
-  // `groups` workgroups of nt threads per link.
-  auto launch = [&](auto kernel, int groups, int nt) {
+  // `groups` workgroups of nt threads and lds bytes per link.
+  auto launch = [&](auto kernel, int groups, int nt, size_t lds = 0) {
     in_launches(nlinks, groups * nt, [&](int first, int n) {
-      hipLaunchKernelGGL(kernel, dim3((unsigned)n * groups), dim3(nt), 0, s, blocks, nblocks,
+      hipLaunchKernelGGL(kernel, dim3((unsigned)n * groups), dim3(nt), lds, s, blocks, nblocks,
                          links + first, r);
     });
   };
@@ -866,7 +889,7 @@ template <int DIM> int prediction_impl(double *blocks, int nblocks, const alpaca
     else if (small_window(r))
       launch(prediction3_kernel<12, 0>, NE, kPredictThreads<12, 0>);
     else
-      launch(prediction3_kernel<16, 0>, NE, kPredictThreads<16, 0>);
+      launch(prediction3_range_kernel, NE, kRangeThreads, range_lds_bytes(r));
   } else if (small_window(r)) {
     launch(prediction2_kernel, 1, kPredict2Threads);
   } else if (all(12)) {
