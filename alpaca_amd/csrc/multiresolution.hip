@@ -606,7 +606,7 @@ __device__ __forceinline__ void for_pairs(const Range &r, int tid, const F &f) {
   }
 }
 
-template <int NT, int W, int N>
+template <int NT, int W, int N, bool EDGES = false>
 __device__ __forceinline__ void predict_field3(double *s, double *__restrict__ blocks,
                                                const alpaca_mr_link &l, int e, const Range &r,
                                                int tid) {
@@ -614,19 +614,18 @@ __device__ __forceinline__ void predict_field3(double *s, double *__restrict__ b
   using L = LdsW<3, W>;
   Window<3> const win(r, l.position);
   double *child = blocks + (size_t)l.child * D::BLOCK + (size_t)e * D::FIELD;
-  // The internal cells of a child row cover its first and last 64-byte segment
+  // EDGES: the internal cells of a child row cover its first and last 64-byte segment
   // in part, and a partial write of a segment that is in no cache is a
-  // read-modify-write in memory, so both are read first (the values are not
-  // used).  2560 links: 343 us without, 303 us with; whole rows would take 177.
+  // read-modify-write in memory, so both are read first (the values are not used).
   double edge[2];
-  if constexpr (N == 8) {
-    static_assert(NT == kIC * kIC, "one child row per thread");
+  if constexpr (EDGES) {
+    static_assert(N == 8 && NT == kIC * kIC, "one child row per thread");
     const double *q = child + (kHS + tid / kIC) * D::SX + (kHS + tid % kIC) * D::SY;
     edge[0] = q[0];
     edge[1] = q[kTC - 1];
   }
   stage_window3<NT, N, L>(s, blocks + (size_t)l.parent * D::BLOCK + (size_t)e * D::FIELD, win, tid);
-  if constexpr (N == 8) asm volatile("" ::"v"(edge[0]), "v"(edge[1]));
+  if constexpr (EDGES) asm volatile("" ::"v"(edge[0]), "v"(edge[1]));
   __syncthreads();
   for_pairs<NT, W, N>(r, tid, [&](int a, int b, int c, int o) {
     double v[2][8];
@@ -643,7 +642,14 @@ __device__ __forceinline__ void predict_field3(double *s, double *__restrict__ b
 // writes: without them 2560 links' internal cells take 118 us.
 template <int W, int N> constexpr int kPredictThreads = W == 12 ? 256 : 448;
 
-template <int W, int N>
+// Links whose children's internal rows (16 x 16 of three 64-byte segments, five
+// equations) fill the 256 MB memory-side cache.  Above, a row's edges are read first:
+// 2400 links 329 us without, 285 us with, warm, and 1600 links 212 and 194 cold (2560 as
+// whole rows would take 177).  Below, the reads only add to the writes: 960 links 66
+// without, 97 with, warm, and 124 and 126 cold, 320 links 27 and 36, and 36 and 43.
+constexpr int kEdgeLinks = (256 << 20) / (5 * kIC * kIC * 192);
+
+template <int W, int N, bool EDGES = false>
 __global__ __launch_bounds__((kPredictThreads<W, N>)) __attribute__((amdgpu_waves_per_eu(4, 8))) void prediction3_kernel(
     double *__restrict__ blocks, int nblocks, const alpaca_mr_link *__restrict__ links, Range r) {
   constexpr int NE = Dims<3>::NE;
@@ -655,7 +661,7 @@ __global__ __launch_bounds__((kPredictThreads<W, N>)) __attribute__((amdgpu_wave
 #pragma unroll
     for (int a = 0; a < 3; ++a) r.count[a] = N;
   }
-  predict_field3<kPredictThreads<W, N>, W, N>(s, blocks, l, int(g % NE), r, threadIdx.x);
+  predict_field3<kPredictThreads<W, N>, W, N, EDGES>(s, blocks, l, int(g % NE), r, threadIdx.x);
 }
 
 // Ranges of more than 8 predicted cells along an axis, but for the whole block: as
@@ -883,7 +889,8 @@ template <int DIM> int prediction_impl(double *blocks, int nblocks, const alpaca
   };
   if constexpr (DIM == 3) {
     if (all(8) && r.start[0] == kHS && r.start[1] == kHS && r.start[2] == kHS)
-      launch(prediction3_kernel<12, 8>, NE, kPredictThreads<12, 8>);
+      launch(nlinks > kEdgeLinks ? prediction3_kernel<12, 8, true> : prediction3_kernel<12, 8>, NE,
+             kPredictThreads<12, 8>);
     else if (all(12))
       launch(prediction3_kernel<16, 12>, NE, kPredictThreads<16, 12>);
     else if (small_window(r))
