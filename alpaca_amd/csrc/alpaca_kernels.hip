@@ -22,6 +22,7 @@
 
 #include "../../include/alpaca_gpu.h"
 #include "fv_device.h"
+#include "launch_rules.h"
 #include "launch_shapes.h"
 
 // Opaque context of the per-block entries (include/alpaca_gpu.h): the HIP
@@ -749,42 +750,6 @@ unsigned launch_march_kernel(int nblocks, hipStream_t s, const double *avg, cons
   return grid.x;
 }
 
-// Whether a 3D case marches (march_stage_kernel) or runs on 8^3 tiles.  Both
-// kernels spend about the same time per unit of 64 faces and wavefront (HLLC
-// FMA 8.2 and 8.3 us, exact 13.6 and 13.5 us at 256^3), a slab taking 26
-// units and a tile 7, and a CU works through the workgroups it is dealt one
-// after the other.  So the case marches where its slabs fill the CUs at least
-// as evenly: 512 blocks 104 units against 112 (exact 1.50 ms a step against
-// 1.54 ms), but 385 blocks 104 against 91 (FMA 0.84 ms against 0.74 ms), and
-// few blocks never (64: 26 against 14).  The mixed forms keep the tiles (HLLC
-// gains nothing; Roe's FP32 faces round differently where a cell's quantities pass
-// through LDS, as other products are then fused).
-// HLLC with FMA marches from 8 blocks per CU only: below, tiles with 512 threads
-// are faster (512 blocks 290 us a stage against 307 marching, 4096 blocks 2364
-// against 2322).
-template <int FLUX, int MODE>
-constexpr bool kMarches = MODE != kModeMixed;
-template <int FLUX, int MODE> bool use_march(int nblocks) {
-  long long const cus = device_cus();
-  if (FLUX == ALPACA_FLUX_HLLC && MODE == kModeFma && nblocks < 8 * cus) return false;
-  auto rounds = [cus](long long groups) { return (groups + cus - 1) / cus; };
-  return rounds(2LL * nblocks) * 26 <= rounds(8LL * nblocks) * 7;
-}
-
-// Whether a 2D case runs on pair_stage_kernel.  Four of its workgroups fill a CU, so
-// it is ahead where the pairs are resident at once or nearly so, and where there
-// are many (exact HLLC, one stage, us, against 16x16 tiles): 1600 blocks 69 and 74,
-// 2025 71 and 91, 2500 90 and 103, 3249 127 and 123, 4900 165 and 170, 16384 529
-// and 550; Roe with FMA 2025 44 and 53, 4900 103 and 101, 16384 347 and 365.  The
-// other forms, which run 4 or 5 wavefronts per SIMD, gain at many blocks only
-// (16384: HLLC FMA 307 and 325, mixed 291 and 301, Roe mixed 382 and 396).
-template <int FLUX, int MODE> bool use_pairs(long long nblocks) {
-  long long const cus = device_cus();
-  bool const heavy = MODE == kModeExact || (FLUX == ALPACA_FLUX_ROE && MODE == kModeFma);
-  return nblocks >= 32 * cus || (MODE == kModeExact && nblocks >= 16 * cus) ||
-         (heavy && nblocks >= 6 * cus && nblocks <= 10 * cus);
-}
-
 template <int FLUX, int MODE>
 unsigned launch_pair_kernel(int nblocks, hipStream_t s, const double *avg, const double *init,
                         double *out, alpaca_case_state *state, const StageArgs &a) {
@@ -822,21 +787,18 @@ unsigned launch_stage_fused(const alpaca_case_desc *d, int stage, const double *
   a.guard = guard;
   a.init_copy = init_copy;
   ProfileScope prof(ALPACA_KERNEL_STAGE, s, double(Dims<DIM>::CELLS) * nblocks);
-  if constexpr (DIM == 3) {
-    if constexpr (kMarches<FLUX, MODE>) {
-      if (use_march<FLUX, MODE>(nblocks)) {
-        return launch_march_kernel<FLUX, MODE>(nblocks, s, avg, init, out, state, a);
-      }
-    }
+  int const cus = device_cus();
+  if constexpr (DIM == 3 && MODE != kModeMixed) {
+    if (rule_marches(FLUX, MODE, nblocks, cus))
+      return launch_march_kernel<FLUX, MODE>(nblocks, s, avg, init, out, state, a);
   }
   if constexpr (DIM == 2) {
-    if (use_pairs<FLUX, MODE>(nblocks)) {
+    if (rule_pairs(FLUX, MODE, nblocks, cus))
       return launch_pair_kernel<FLUX, MODE>(nblocks, s, avg, init, out, state, a);
-    }
   }
   constexpr bool wide = FLUX == ALPACA_FLUX_HLLC && MODE != kModeExact;
   unsigned groups = 0;
-  with_shape<DIM>(nblocks, device_cus(), wide, [&](auto shape) {
+  with_shape<DIM>(nblocks, cus, wide, [&](auto shape) {
     using S = decltype(shape);
     constexpr int tiles = exact::TileShape<DIM, S::TX, S::TY, S::TZ>::TILES;
     groups = unsigned(nblocks) * tiles;
