@@ -539,9 +539,13 @@ template <int DIM, int FLUX, typename R>
 constexpr int kMinWaves = !std::is_same<R, double>::value ? 1
                           : DIM == 2 ? 3 : (FLUX == 1 && !kFastArith ? 2 : 1);
 
-// The persistent batch kernel: as above.
-template <int DIM, int FLUX, typename R>
-constexpr int kBatchMinWaves = kMinWaves<DIM, FLUX, R>;
+// And at most, in the persistent batch kernel.  The 2D mixed flux-splitting form fits 4,
+// but with two wavefronts per workgroup its workgroups then gather on some SIMDs, four
+// wavefronts there and two on others, and a stage waits for those.  Held to 3 (one step,
+// 16x16 cells, us): 1300 blocks 167 -> 144, 1536 174 -> 149, 3072 319 -> 273, 8192 824 ->
+// 694; 1024 and fewer the same.
+template <int DIM, int FLUX, typename R, int NT>
+constexpr int kBatchMaxWaves = DIM == 2 && FLUX == 1 && std::is_same<R, float>::value && NT == 128 ? 3 : 8;
 
 // The job of a single case's stage.
 __device__ __forceinline__ TileJob stage_job(const double *avg, const double *init, double *out,
@@ -750,7 +754,7 @@ __device__ __forceinline__ double in_sgpr(double v) {
 // split into 8 contiguous ranges, one per XCD (group g runs on XCD g % 8),
 // so a case's blocks share an L2.  Units of stopped cases are skipped.
 template <int DIM, int FLUX, typename R, int TX, int TY, int TZ, int NT>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kBatchMinWaves<DIM, FLUX, R>, 8))) void batch_stage_kernel(
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kMinWaves<DIM, FLUX, R>, kBatchMaxWaves<DIM, FLUX, R, NT>))) void batch_stage_kernel(
     const double *__restrict__ avg, const double *init, double *out, const CaseSlot *slots,
     alpaca_case_state *states, const WorkItem *items, const int *n_items, int stage) {
   using T = TileShape<DIM, TX, TY, TZ>;
