@@ -176,7 +176,7 @@ struct alpaca_ensemble {
   int units_per_block = 1;
   BlockPool *pool = nullptr;
   hipStream_t stream = nullptr;
-  hipStream_t aux[kClasses] = {};  // streams of the classes but the first
+  hipStream_t aux[kClasses] = {};  // streams of the classes, if there are several
   hipEvent_t fork = nullptr, join[kClasses] = {};
   double *u = nullptr, *s1 = nullptr, *s2 = nullptr;
   CaseSlot *d_slots = nullptr;
@@ -355,18 +355,21 @@ int capture_step(alpaca_ensemble *e, int tile_config, int cls, int later, hipStr
   return ALPACA_OK;
 }
 
-// nsteps macro steps of the enabled classes, side by side: the first class on the
-// ensemble's stream, each further one on a stream of its own between a fork and a
-// join event, so that the ensemble's stream orders the call as a whole.  Classes
-// touch disjoint cases, blocks and records.  Two classes of 290 blocks: 151 us a
-// step with a join per stage (9 us each), 118 with one per step (25 us with the
-// records' kernel), 100 to 115 with one per call.
+// nsteps macro steps of the enabled classes.  One class runs on the ensemble's stream,
+// several side by side, each on a stream of its own between a fork and a join event, so
+// that the ensemble's stream orders the call as a whole.  Classes touch disjoint cases,
+// blocks and records.  Two classes of 290 blocks: 151 us a step with a join per stage (9
+// us each), 118 with one per step (25 us with the records' kernel), 100 to 115 with one
+// per call.  The classes' streams are created one after the other, which gives them
+// hardware queues of their own; with the first class on the ensemble's stream, whatever
+// queue that has, two classes shared one in one ensemble of four and ran in turn (48 2D
+// blocks in each 130 us a step instead of 74, 4 3D blocks 232 instead of 150).
 int run_classes(alpaca_ensemble *e, int tile_config, int nsteps) {
   int cls[kClasses];
   int ncls = 0;
   for (int c = 0; c < kClasses; ++c)
     if (e->class_mask & (1u << c)) cls[ncls++] = c;
-  auto stream = [&](int i) { return i == 0 ? e->stream : e->aux[cls[i]]; };
+  auto stream = [&](int i) { return ncls == 1 ? e->stream : e->aux[cls[i]]; };
   for (int i = 0; i < ncls; ++i)
     for (int later = 0; later < (nsteps > 1 ? 2 : 1); ++later)
       if (!e->exec[tile_config][cls[i]][later]) {
@@ -374,12 +377,13 @@ int run_classes(alpaca_ensemble *e, int tile_config, int nsteps) {
         if (st != ALPACA_OK) return st;
       }
   bool ok = ncls == 1 || hipEventRecord(e->fork, e->stream) == hipSuccess;
-  for (int i = 1; ok && i < ncls; ++i) ok = hipStreamWaitEvent(stream(i), e->fork, 0) == hipSuccess;
+  for (int i = 0; ok && ncls > 1 && i < ncls; ++i)
+    ok = hipStreamWaitEvent(stream(i), e->fork, 0) == hipSuccess;
   for (int n = 0; ok && n < nsteps; ++n)
     for (int i = 0; ok && i < ncls; ++i)
       ok = hipGraphLaunch(e->exec[tile_config][cls[i]][n > 0], stream(i)) == hipSuccess;
   // Joined after a failure too: what was queued is ordered before later calls.
-  for (int i = 1; i < ncls; ++i)
+  for (int i = 0; ncls > 1 && i < ncls; ++i)
     ok = hipEventRecord(e->join[cls[i]], stream(i)) == hipSuccess &&
          hipStreamWaitEvent(e->stream, e->join[cls[i]], 0) == hipSuccess && ok;
   return ok ? ALPACA_OK : ALPACA_ERR_HIP;
@@ -439,12 +443,14 @@ int ensemble_init(alpaca_ensemble *e, BlockPool *pool, int dim, int max_cases,
             hipMalloc(&e->d_counts, sizeof(int) * kClasses) == hipSuccess;
   for (int c = 0; ok && c < kClasses; ++c)
     if (class_mask & (1u << c))
-      ok = hipMalloc(&e->d_items[c], sizeof(WorkItem) * e->max_blocks) == hipSuccess &&
-           hipStreamCreateWithFlags(&e->aux[c], hipStreamNonBlocking) == hipSuccess;
-  ok = ok && hipEventCreateWithFlags(&e->fork, hipEventDisableTiming) == hipSuccess;
-  for (int c = 0; ok && c < kClasses; ++c)
-    if (class_mask & (1u << c))
-      ok = hipEventCreateWithFlags(&e->join[c], hipEventDisableTiming) == hipSuccess;
+      ok = hipMalloc(&e->d_items[c], sizeof(WorkItem) * e->max_blocks) == hipSuccess;
+  if (class_mask & (class_mask - 1)) {  // several classes
+    ok = ok && hipEventCreateWithFlags(&e->fork, hipEventDisableTiming) == hipSuccess;
+    for (int c = 0; ok && c < kClasses; ++c)
+      if (class_mask & (1u << c))
+        ok = hipStreamCreateWithFlags(&e->aux[c], hipStreamNonBlocking) == hipSuccess &&
+             hipEventCreateWithFlags(&e->join[c], hipEventDisableTiming) == hipSuccess;
+  }
   if (ok) {
     ok = hipMemsetAsync(e->d_states, 0, sizeof(alpaca_case_state) * max_cases, e->stream) ==
              hipSuccess &&
