@@ -30,6 +30,7 @@
 
 #include "../../include/alpaca_gpu.h"
 #include "fv_device.h"
+#include "launch_rules.h"
 
 using namespace alpaca;
 
@@ -94,17 +95,6 @@ __global__ void ens_set_flags_kernel(alpaca_case_state *states, int i, int set, 
 template <int DIM> constexpr int num_tiles_configs() { return DIM == 3 ? 2 : 3; }
 // And those the ensemble chooses by itself: 2D: 3 = 8x8 / 256, 4 = 16x8 / 192
 constexpr int kMaxTileConfigs = 5;
-
-// The configuration of an ensemble that was given none, from the blocks it
-// holds: as launch_shapes.h chooses for a single case (whose line for one
-// workgroup per CU does not carry over to several classes at once).  290 blocks
-// in each of two classes, exact and mixed HLLC, side by side: 49 us a stage with
-// configuration 0, 28 to 40 us with 4.
-int auto_tile_config(int dim, long long blocks, long long cus) {
-  if (dim == 3) return 0;
-  if (4 * blocks <= 5 * cus) return 3;
-  return blocks < 6 * cus ? 4 : 0;
-}
 
 template <int DIM, int FLUX, int TX, int TY, int TZ, int NT>
 void launch_batch_tile(int groups, hipStream_t s, const double *avg, const double *init,
@@ -657,9 +647,12 @@ int alpaca_ensemble_step(alpaca_ensemble *e, int nsteps) {
   std::lock_guard<std::mutex> lock(e->mu);
   int st = upload_lists(e);
   if (st != ALPACA_OK) return st;
-  size_t blocks = 0;
-  for (auto const &items : e->h_items) blocks += items.size();
-  int const t = e->tuned ? e->tile_config : auto_tile_config(e->dim, (long long)blocks, e->num_cus);
+  long long blocks = 0, largest = 0;
+  for (auto const &items : e->h_items) {
+    blocks += (long long)items.size();
+    largest = std::max(largest, (long long)items.size());
+  }
+  int const t = e->tuned ? e->tile_config : rule_ensemble_tiles(e->dim, blocks, largest, e->num_cus);
   if (nsteps == 0) return ALPACA_OK;
   if ((st = run_classes(e, t, nsteps)) != ALPACA_OK) return st;
   hipLaunchKernelGGL(ens_finish_kernel, dim3((e->max_cases + 255) / 256), dim3(256), 0, e->stream,

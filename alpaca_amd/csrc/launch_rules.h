@@ -49,4 +49,21 @@ inline bool rule_pairs(int flux, int mode, long long blocks, long long cus) {
          (heavy && blocks > 6 * cus && blocks <= 10 * cus);
 }
 
+// The tile configuration (of set_tuning, and 3 = 8x8 cells and 256 threads, 4 = 16x8 and 192)
+// of an ensemble that was given none, from all its blocks and those of its largest class.
+// 3D: 8^3 always.  2D, one step, us, configurations 0, 3 and 4:
+//   blocks                160          320          512           768           900          1400
+//   HLLC exact         95  62  70  136  86  90  140 125  96  149 184 132  147 223 180  197 315 233
+//   Roe mixed          69  50  56   95  70  67   98  98  72  102 138 101  106 165 130  144 230 173
+//   HLLC exact+mixed  100  60  58  101  69  76  104  98  87  144 129 104  147 153 117  175 214 178
+//   Roe exact+mixed   104  60  62  108  73  82  111 102  94  159 138 114  162 160 126  197 234 193
+// The line between 3 and 4 is that of a single case (launch_shapes.h).  Configuration 4
+// holds two blocks per CU at a time, and from the third on a class waits for a second
+// round, where 0 holds six; several classes fill each other's rounds.
+inline int rule_ensemble_tiles(int dim, long long blocks, long long largest, long long cus) {
+  if (dim == 3) return 0;
+  if (4 * blocks <= 5 * cus) return 3;
+  return blocks < 6 * cus && largest <= 3 * cus ? 4 : 0;
+}
+
 }  // namespace alpaca
