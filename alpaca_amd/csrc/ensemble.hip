@@ -183,9 +183,10 @@ struct alpaca_ensemble {
   int tile_config = 0;
   int groups_per_cu = 0;  // 0: default from occupancy
   int num_cus = 256;
-  // A class's captured step per configuration: [0] the first of a call, [1] later.
-  hipGraphExec_t exec[kMaxTileConfigs][kClasses][2] = {};
-  hipGraph_t graph[kMaxTileConfigs][kClasses][2] = {};
+  // A class's captured step per configuration and variant: bit 0 a later one of a call,
+  // bit 1 with no more workgroups than the default.
+  hipGraphExec_t exec[kMaxTileConfigs][kClasses][4] = {};
+  hipGraph_t graph[kMaxTileConfigs][kClasses][4] = {};
   std::mutex mu;
 };
 
@@ -250,11 +251,6 @@ void pool_capacity(alpaca_ensemble *e, int *free_blocks, int *largest) {
   *largest = (int)std::min<long long>(big, INT32_MAX);
 }
 
-int default_groups_per_cu(int dim, int tile_config) {
-  if (dim == 3) return tile_config == 1 ? 1 : 2;
-  return tile_config == 1 || tile_config == 3 ? 3 : (tile_config == 4 ? 4 : 6);
-}
-
 int upload_lists(alpaca_ensemble *e) {
   if (!e->items_dirty) return ALPACA_OK;
   int counts[kClasses];
@@ -298,13 +294,14 @@ void launch_class(alpaca_ensemble *e, int tile_config, int c, int groups, hipStr
 
 // A class's macro step as captured: the time steps of its cases (after the end of
 // the step before, for a later step of a call), then the three stages.
-int record_step(alpaca_ensemble *e, int tile_config, int cls, int later, hipStream_t s) {
-  int const g0 = e->groups_per_cu > 0 ? e->groups_per_cu : default_groups_per_cu(e->dim, tile_config);
+int record_step(alpaca_ensemble *e, int tile_config, int cls, int variant, hipStream_t s) {
+  int const dflt = rule_ensemble_default_groups(e->dim, tile_config);
+  int const g0 = e->groups_per_cu > 0 && !(variant & 2) ? e->groups_per_cu : dflt;
   int groups = g0 * e->num_cus;
   groups = (groups + 7) / 8 * 8;
   int const nc = e->max_cases;
   dim3 const grid((nc + 255) / 256), block(256);
-  if (later)
+  if (variant & 1)
     hipLaunchKernelGGL(ens_dt_kernel<true>, grid, block, 0, s, e->d_slots, e->d_states, nc, cls);
   else
     hipLaunchKernelGGL(ens_dt_kernel<false>, grid, block, 0, s, e->d_slots, e->d_states, nc, cls);
@@ -312,9 +309,9 @@ int record_step(alpaca_ensemble *e, int tile_config, int cls, int later, hipStre
   return hip_ok(hipGetLastError());
 }
 
-void drop_graph(alpaca_ensemble *e, int tile_config, int cls, int later) {
-  hipGraphExec_t &exec = e->exec[tile_config][cls][later];
-  hipGraph_t &graph = e->graph[tile_config][cls][later];
+void drop_graph(alpaca_ensemble *e, int tile_config, int cls, int variant) {
+  hipGraphExec_t &exec = e->exec[tile_config][cls][variant];
+  hipGraph_t &graph = e->graph[tile_config][cls][variant];
   if (exec) (void)hipGraphExecDestroy(exec);
   if (graph) (void)hipGraphDestroy(graph);
   exec = nullptr;
@@ -323,23 +320,23 @@ void drop_graph(alpaca_ensemble *e, int tile_config, int cls, int later) {
 void drop_graphs(alpaca_ensemble *e) {
   for (int t = 0; t < kMaxTileConfigs; ++t)
     for (int c = 0; c < kClasses; ++c)
-      for (int later = 0; later < 2; ++later) drop_graph(e, t, c, later);
+      for (int v = 0; v < 4; ++v) drop_graph(e, t, c, v);
 }
 
-int capture_step(alpaca_ensemble *e, int tile_config, int cls, int later, hipStream_t s) {
-  drop_graph(e, tile_config, cls, later);
+int capture_step(alpaca_ensemble *e, int tile_config, int cls, int variant, hipStream_t s) {
+  drop_graph(e, tile_config, cls, variant);
   if (hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal) != hipSuccess)
     return ALPACA_ERR_HIP;
-  int const st = record_step(e, tile_config, cls, later, s);
+  int const st = record_step(e, tile_config, cls, variant, s);
   hipGraph_t g = nullptr;
   hipError_t const end = hipStreamEndCapture(s, &g);
   if (st != ALPACA_OK || end != hipSuccess) {
     if (g) (void)hipGraphDestroy(g);
     return st != ALPACA_OK ? st : ALPACA_ERR_HIP;
   }
-  e->graph[tile_config][cls][later] = g;
-  if (hipGraphInstantiate(&e->exec[tile_config][cls][later], g, nullptr, nullptr, 0) != hipSuccess) {
-    drop_graph(e, tile_config, cls, later);
+  e->graph[tile_config][cls][variant] = g;
+  if (hipGraphInstantiate(&e->exec[tile_config][cls][variant], g, nullptr, nullptr, 0) != hipSuccess) {
+    drop_graph(e, tile_config, cls, variant);
     return ALPACA_ERR_HIP;
   }
   return ALPACA_OK;
@@ -360,18 +357,26 @@ int run_classes(alpaca_ensemble *e, int tile_config, int nsteps) {
   for (int c = 0; c < kClasses; ++c)
     if (e->class_mask & (1u << c)) cls[ncls++] = c;
   auto stream = [&](int i) { return ncls == 1 ? e->stream : e->aux[cls[i]]; };
-  for (int i = 0; i < ncls; ++i)
-    for (int later = 0; later < (nsteps > 1 ? 2 : 1); ++later)
-      if (!e->exec[tile_config][cls[i]][later]) {
-        int const st = capture_step(e, tile_config, cls[i], later, stream(i));
+  int fewer[kClasses];  // bit 1 of the class's variants
+  for (int i = 0; i < ncls; ++i) {
+    fewer[i] = e->groups_per_cu > rule_ensemble_default_groups(e->dim, tile_config) &&
+                       rule_ensemble_fewer_groups(e->dim, tile_config,
+                                                  (long long)e->h_items[cls[i]].size(), e->num_cus)
+                   ? 2
+                   : 0;
+    for (int v = fewer[i]; v <= fewer[i] + (nsteps > 1); ++v)
+      if (!e->exec[tile_config][cls[i]][v]) {
+        int const st = capture_step(e, tile_config, cls[i], v, stream(i));
         if (st != ALPACA_OK) return st;
       }
+  }
   bool ok = ncls == 1 || hipEventRecord(e->fork, e->stream) == hipSuccess;
   for (int i = 0; ok && ncls > 1 && i < ncls; ++i)
     ok = hipStreamWaitEvent(stream(i), e->fork, 0) == hipSuccess;
   for (int n = 0; ok && n < nsteps; ++n)
     for (int i = 0; ok && i < ncls; ++i)
-      ok = hipGraphLaunch(e->exec[tile_config][cls[i]][n > 0], stream(i)) == hipSuccess;
+      ok = hipGraphLaunch(e->exec[tile_config][cls[i]][fewer[i] | int(n > 0)], stream(i)) ==
+           hipSuccess;
   // Joined after a failure too: what was queued is ordered before later calls.
   for (int i = 0; ncls > 1 && i < ncls; ++i)
     ok = hipEventRecord(e->join[cls[i]], stream(i)) == hipSuccess &&
@@ -635,7 +640,11 @@ int alpaca_ensemble_set_tuning(alpaca_ensemble *e, int tile_config, int groups_p
   int const ntc = e->dim == 3 ? num_tiles_configs<3>() : num_tiles_configs<2>();
   if (tile_config < 0 || tile_config >= ntc) return ALPACA_ERR_INVALID;
   std::lock_guard<std::mutex> lock(e->mu);
-  if (groups_per_cu != e->groups_per_cu) drop_graphs(e);
+  if (groups_per_cu != e->groups_per_cu) {
+    // Queued steps may still run from the graphs.
+    if (hipStreamSynchronize(e->stream) != hipSuccess) return ALPACA_ERR_HIP;
+    drop_graphs(e);
+  }
   e->tuned = true;
   e->tile_config = tile_config;
   e->groups_per_cu = groups_per_cu;

@@ -66,4 +66,23 @@ inline int rule_ensemble_tiles(int dim, long long blocks, long long largest, lon
   return blocks < 6 * cus && largest <= 3 * cus ? 4 : 0;
 }
 
+// Persistent workgroups per CU of an ensemble's stage kernels with a tile configuration:
+// what fits a CU at once, and where a tuning gave none.
+inline int rule_ensemble_default_groups(int dim, int tile_config) {
+  if (dim == 3) return tile_config == 1 ? 1 : 2;
+  return tile_config == 1 || tile_config == 3 ? 3 : (tile_config == 4 ? 4 : 6);
+}
+
+// Whether a class of so many blocks takes the default where a tuning gave more.  The 2D
+// workgroups of 128 threads (configurations 0 and 2) are two wavefronts.  Up to four of
+// them with work per CU are two wavefronts on each SIMD, unless idle workgroups are dealt
+// among them, which leaves some SIMDs with three and others with one (one step, us, 6 and
+// 12 per CU: 580 blocks of exact HLLC 144 and 156, 832 146 and 189, 1024 152 and 186; mixed
+// 960 93 and 104).  Above, the idle ones are few (1100 blocks 191 and 191, 1400 199 and
+// 193), and with four wavefronts a workgroup has one on each SIMD anyway.
+inline bool rule_ensemble_fewer_groups(int dim, int tile_config, long long blocks, long long cus) {
+  if (dim != 2 || (tile_config != 0 && tile_config != 2)) return false;
+  return blocks * (tile_config == 2 ? 2 : 1) <= 4 * cus;
+}
+
 }  // namespace alpaca

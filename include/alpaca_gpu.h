@@ -393,7 +393,8 @@ int alpaca_ensemble_remove_case(alpaca_ensemble *e, int case_id);
 int alpaca_ensemble_cancel_case(alpaca_ensemble *e, int case_id);
 /* Tile shape (3D: 0 = 8x8x8/256 threads, 1 = 16x8x8/512; 2D: 0 = 16x16/128,
  * 1 = 16x16/256, 2 = 16x8/128) and persistent workgroups per CU (0 = the
- * occupancy default) of the stage kernels.  An ensemble that was given none
+ * occupancy default; in 2D a class of at most four workgroups' work per CU takes
+ * no more than that) of the stage kernels.  An ensemble that was given none
  * chooses its tiles by the number of blocks it holds. */
 int alpaca_ensemble_set_tuning(alpaca_ensemble *e, int tile_config, int groups_per_cu);
 /* Advances every running case by nsteps macro steps (asynchronous). */
