@@ -901,18 +901,22 @@ __device__ __forceinline__ void roe_split_flux_exact(double gamma, double b,
 // (flux_splitting_scheme.cpp:42-76, 185-315), added into f, in the mixed form.
 // The stencil is walked cell by cell -- load, advection, projection onto every
 // field -- which keeps few values live: 3 waves per SIMD.  Each projection is
-// the expression of the exact form.
+// the expression of the exact form.  The stencil is read through a buffer resource: with
+// 64-bit addresses 512 3D blocks took 1212 us a step, 1165 so, 4900 2D blocks 357 and 344.
 template <int DIM, int DIR, typename QS>
 __device__ __forceinline__ void roe_split_flux(double gamma64, double b64,
-                                               const double *__restrict__ base, const QS &qs,
+                                               const double *__restrict__ blk, int off, const QS &qs,
                                                float *f) {
   using R = float;
   constexpr int NE = DIM + 2;
   R const gamma = R(gamma64);
-  auto load = [base](int m, double *c) {
+  constexpr int S = axis_stride<DIM, DIR>();
+  BlockReader<DIM> const rd(blk);
+  int const off0 = (off - 2 * S) * (int)sizeof(double);
+  auto load = [&](int m, double *c) {
 #pragma unroll
     for (int e = 0; e < NE; ++e)
-      c[e] = base[e * Dims<DIM>::FIELD + (m - 2) * axis_stride<DIM, DIR>()];
+      c[e] = rd(off0, (e * Dims<DIM>::FIELD + m * S) * (int)sizeof(double));
   };
   Eig<NE, R> ev;
   double adv2[NE];  // advection of cell i (FP64)
@@ -1408,7 +1412,7 @@ __device__ __forceinline__ void face_flux(double gamma64, double b64,
   } else if constexpr (kLean<R>) {
     roe_split_flux_lean<DIM, DIR>(gamma64, b64, base, qs, f);
   } else {
-    roe_split_flux<DIM, DIR>(gamma64, b64, base, qs, f);
+    roe_split_flux<DIM, DIR>(gamma64, b64, blk, off, qs, f);
   }
 }
 
