@@ -738,14 +738,13 @@ void launch_stage_kernel(dim3 grid, hipStream_t s, const double *avg, const doub
 template <int FLUX, int MODE>
 unsigned launch_march_kernel(int nblocks, hipStream_t s, const double *avg, const double *init,
                          double *out, alpaca_case_state *state, const StageArgs &a) {
-  using R = double;
-  using M = exact::MarchShape<R>;
+  using M = exact::MarchShape;
   dim3 const grid(nblocks * M::SLABS), block(M::PLANE);
   if constexpr (MODE == kModeExact)
-    hipLaunchKernelGGL((exact::march_stage_kernel<FLUX, R>), grid, block, 0, s, avg, init, out,
+    hipLaunchKernelGGL((exact::march_stage_kernel<FLUX>), grid, block, 0, s, avg, init, out,
                        state, a);
   else
-    hipLaunchKernelGGL((fast::march_stage_kernel<FLUX, R>), grid, block, 0, s, avg, init, out, state,
+    hipLaunchKernelGGL((fast::march_stage_kernel<FLUX>), grid, block, 0, s, avg, init, out, state,
                        a);
   return grid.x;
 }

@@ -273,16 +273,13 @@ __device__ __forceinline__ FaceQ<R> face_quantities(double gamma, double b, cons
   return f;
 }
 
-// A cell's FaceQ as NQ values: 1/rho is kept and the velocities are formed from the
+// A cell's FP64 FaceQ as kPackedQ values: 1/rho is kept and the velocities are formed from the
 // stencil's momenta again (one exact repetition of a product each).
-template <typename R> struct PackedQ {
-  static constexpr int NQ = 5;
-  static_assert(std::is_same<R, double>::value, "FP64 forms");
-};
+constexpr int kPackedQ = 5;
 
 // Writes the FaceQ of the cell with conservatives c to q[0], q[STRIDE], ...
-template <int DIM, typename R, int STRIDE>
-__device__ __forceinline__ void store_packed(double gamma, double b, const double *c, R *q) {
+template <int DIM, int STRIDE>
+__device__ __forceinline__ void store_packed(double gamma, double b, const double *c, double *q) {
   CellQ<double> w;
   cell_quantities<DIM, double>(gamma, b, c, w);
   q[0] = dsqrt(w.rho);
@@ -292,11 +289,11 @@ __device__ __forceinline__ void store_packed(double gamma, double b, const doubl
   q[4 * STRIDE] = w.p * w.one_rho;
 }
 
-template <int DIM, typename R, int STRIDE>
-__device__ __forceinline__ FaceQ<R> load_packed(const R *q, const double *c) {
-  FaceQ<R> f;
+template <int DIM, int STRIDE>
+__device__ __forceinline__ FaceQ<double> load_packed(const double *q, const double *c) {
+  FaceQ<double> f;
   double const one_rho = q[STRIDE];
-  f.rho = R(c[kMass]);
+  f.rho = c[kMass];
   f.sq = q[0];
   f.vel[0] = c[kMomX] * one_rho;
   f.vel[1] = c[kMomX + 1] * one_rho;
@@ -492,12 +489,11 @@ __device__ __forceinline__ double weno_one_lean(double v1, double v2, double v3,
   return v3 + (1.0 / 6.0) * weno_lean(w, s1, s2, s3, d1, d2, d3, d4);
 }
 
-// The left reconstruction of l and the right one of r (apply_wrapper.h:48-58).
-template <typename R, bool PAIRED = true>
+// The left reconstruction of l and the right one of r (apply_wrapper.h:48-58) in the
+// contracting forms.
+template <typename R>
 __device__ __forceinline__ void weno_pair(const R *l, const R *r, R &left, R &right) {
-  if constexpr (kExact<R>) {
-    (void)weno_pair_exact<true>(l, r, left, right);
-  } else if constexpr (kLean<R>) {
+  if constexpr (kLean<R>) {
     left = weno_one_lean(l[0], l[1], l[2], l[3], l[4]);
     right = weno_one_lean(r[5], r[4], r[3], r[2], r[1]);
   } else {
@@ -521,10 +517,9 @@ template <int NE, typename R> struct Eig {
 // momentum.  The exact form leaves these products out where the stencil is
 // finite; the mixed form keeps its measured accuracy by forming them.
 template <int DIM, int DIR> __device__ __forceinline__ constexpr bool left_zero(int n, int c) {
-  constexpr int Mp = kMomX + DIR, M1 = kMomX + Minor<DIR>::m1, M2 = kMomX + Minor<DIR>::m2;
+  constexpr int M1 = kMomX + Minor<DIR>::m1, M2 = kMomX + Minor<DIR>::m2;
   if (n == 1) return c != kMass && c != M1;
   if (DIM == 3 && n == 2) return c != kMass && c != M2;
-  (void)Mp;
   return false;
 }
 // The exact FP64 finite-volume (HLLC) kernels build the right eigenvectors
@@ -1428,25 +1423,25 @@ template <int DIM, typename R> struct FormedQ {
     return face_quantities<DIM, R>(gamma, b, c);
   }
 };
-template <int DIM, typename R, int STRIDE> struct KeptQ {
-  const R *l, *r;
-  __device__ __forceinline__ FaceQ<R> left(const double *c) const {
-    return load_packed<DIM, R, STRIDE>(l, c);
+template <int DIM, int STRIDE> struct KeptQ {
+  const double *l, *r;
+  __device__ __forceinline__ FaceQ<double> left(const double *c) const {
+    return load_packed<DIM, STRIDE>(l, c);
   }
-  __device__ __forceinline__ FaceQ<R> right(const double *c) const {
-    return load_packed<DIM, R, STRIDE>(r, c);
+  __device__ __forceinline__ FaceQ<double> right(const double *c) const {
+    return load_packed<DIM, STRIDE>(r, c);
   }
 };
-template <int DIM, typename R, int STRIDE> struct KeptThenFormedQ {
+template <int DIM, int STRIDE> struct KeptThenFormedQ {
   double gamma, b;
-  const R *l;
-  R *r;
-  __device__ __forceinline__ FaceQ<R> left(const double *c) const {
-    return load_packed<DIM, R, STRIDE>(l, c);
+  const double *l;
+  double *r;
+  __device__ __forceinline__ FaceQ<double> left(const double *c) const {
+    return load_packed<DIM, STRIDE>(l, c);
   }
-  __device__ __forceinline__ FaceQ<R> right(const double *c) const {
-    store_packed<DIM, R, STRIDE>(gamma, b, c, r);
-    return load_packed<DIM, R, STRIDE>(r, c);
+  __device__ __forceinline__ FaceQ<double> right(const double *c) const {
+    store_packed<DIM, STRIDE>(gamma, b, c, r);
+    return load_packed<DIM, STRIDE>(r, c);
   }
 };
 

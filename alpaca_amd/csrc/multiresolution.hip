@@ -355,15 +355,13 @@ template <int DIM> struct Window {
   }
 };
 
-template <int DIM>
-__device__ __forceinline__ void stage_window(double *s, const double *__restrict__ field,
-                                             const Window<DIM> &win) {
-  using D = Dims<DIM>;
-  int const n = win.w[0] * win.w[1] * win.w[2];
-  for (int t = threadIdx.x; t < n; t += kStencilThreads) {
-    int const a = t / (win.w[1] * win.w[2]), b = (t / win.w[2]) % win.w[1], c = t % win.w[2];
-    s[a * Lds<DIM>::SX + b * Lds<DIM>::SY + c] =
-        field[(win.p0[0] + a) * D::SX + (win.p0[1] + b) * D::SY + (win.p0[2] + c)];
+// One 2D field's parent window into LDS.
+__device__ __forceinline__ void stage_window2(double *s, const double *__restrict__ field,
+                                              const Window<2> &win) {
+  using D = Dims<2>;
+  for (int t = threadIdx.x; t < win.w[0] * win.w[1]; t += kStencilThreads) {
+    int const a = t / win.w[1], b = t % win.w[1];
+    s[a * Lds<2>::SX + b * Lds<2>::SY] = field[(win.p0[0] + a) * D::SX + (win.p0[1] + b) * D::SY];
   }
 }
 
@@ -394,33 +392,6 @@ template <int DIM> __device__ __forceinline__ void load_children(const double *q
     double2 const a = *reinterpret_cast<const double2 *>(q);
     double2 const b = *reinterpret_cast<const double2 *>(q + D::SX);
     x[0] = a.x, x[2] = a.y, x[1] = b.x, x[3] = b.y;
-  }
-}
-
-// One workgroup per (link, equation): the child cells of the range,
-// predicted from the parent's field.  FULL: the range is the whole block
-// (12 predicted parent cells per axis, known at compile time).
-// Predicts range r of child l.child's equation e from its parent: stages the
-// parent window in s, then two children per axis per task.  The caller's
-// early exits are uniform over the workgroup, so every thread reaches the
-// barrier.
-template <int DIM>
-__device__ __forceinline__ void predict_range(double *s, double *__restrict__ blocks,
-                                              const alpaca_mr_link &l, int e, const Range &r) {
-  using D = Dims<DIM>;
-  Window<DIM> const win(r, l.position);
-  stage_window<DIM>(s, blocks + (size_t)l.parent * D::BLOCK + (size_t)e * D::FIELD, win);
-  __syncthreads();
-  double *child = blocks + (size_t)l.child * D::BLOCK + (size_t)e * D::FIELD;
-  int const nz = DIM == 3 ? r.count[2] : 1;
-  int const tasks = r.count[0] * r.count[1] * nz;
-  for (int t = threadIdx.x; t < tasks; t += kStencilThreads) {
-    int const a = t / (r.count[1] * nz), b = (t / nz) % r.count[1], c = t % nz;
-    double v[1 << DIM];
-    predict_cell(s, Window<DIM>::centre(a, b, c), v);
-    int const ci = r.start[0] + 2 * a, cj = r.start[1] + 2 * b;
-    int const ck = DIM == 3 ? r.start[2] + 2 * c : 0;
-    store_children<DIM>(child + ci * D::SX + cj * D::SY + ck, v);
   }
 }
 
@@ -478,22 +449,33 @@ __global__ __launch_bounds__(kPredict2Threads) void prediction2_kernel(
   predict_range2(s, blocks, l, r);
 }
 
-template <int DIM, bool FULL>
-__global__ __launch_bounds__(kStencilThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) void prediction_kernel(
+// 2D ranges with larger windows: one workgroup per (link, equation).  FULL: the whole
+// block (12 predicted parent cells per axis, known at compile time).
+template <bool FULL>
+__global__ __launch_bounds__(kStencilThreads) __attribute__((amdgpu_waves_per_eu(4, 8))) void prediction2_range_kernel(
     double *__restrict__ blocks, int nblocks, const alpaca_mr_link *__restrict__ links, Range r) {
-  using D = Dims<DIM>;
-  __shared__ double s[Lds<DIM>::SIZE];
+  using D = Dims<2>;
+  __shared__ double s[Lds<2>::SIZE];
   if constexpr (FULL) {
 #pragma unroll
-    for (int a = 0; a < 3; ++a) {
+    for (int a = 0; a < 2; ++a) {
       r.start[a] = 0;
-      r.count[a] = a < DIM ? kTC / 2 : 1;
+      r.count[a] = kTC / 2;
     }
   }
   int const e = blockIdx.x % D::NE;
   alpaca_mr_link const l = links[blockIdx.x / D::NE];
-  if (!link_ok<DIM>(l, nblocks)) return;
-  predict_range<DIM>(s, blocks, l, e, r);
+  if (!link_ok<2>(l, nblocks)) return;  // uniform over the workgroup
+  stage_window2(s, blocks + (size_t)l.parent * D::BLOCK + (size_t)e * D::FIELD,
+                Window<2>(r, l.position));
+  __syncthreads();
+  double *child = blocks + (size_t)l.child * D::BLOCK + (size_t)e * D::FIELD;
+  for (int t = threadIdx.x; t < r.count[0] * r.count[1]; t += kStencilThreads) {
+    int const a = t / r.count[1], b = t % r.count[1];
+    double v[4];
+    predict_cell(s, Window<2>::centre(a, b, 0), v);
+    store_children<2>(child + (r.start[0] + 2 * a) * D::SX + (r.start[1] + 2 * b) * D::SY, v);
+  }
 }
 
 // The halo slab of a location (CommunicationTypes::GetStartIndicesHaloRecv and
@@ -770,7 +752,7 @@ __global__ __launch_bounds__(kDetailThreads<DIM>) __attribute__((amdgpu_waves_pe
     if constexpr (DIM == 3)
       stage_window3<NT, H, Lds<3>>(s[e], field, win, threadIdx.x);
     else
-      stage_window<DIM>(s[e], field, win);
+      stage_window2(s[e], field, win);
   }
   __syncthreads();
   double m = 0.0;
@@ -900,9 +882,9 @@ template <int DIM> int prediction_impl(double *blocks, int nblocks, const alpaca
   } else if (small_window(r)) {
     launch(prediction2_kernel, 1, kPredict2Threads);
   } else if (all(12)) {
-    launch(prediction_kernel<DIM, true>, NE, kStencilThreads);
+    launch(prediction2_range_kernel<true>, NE, kStencilThreads);
   } else {
-    launch(prediction_kernel<DIM, false>, NE, kStencilThreads);
+    launch(prediction2_range_kernel<false>, NE, kStencilThreads);
   }
   return hip_status(hipGetLastError());
 }

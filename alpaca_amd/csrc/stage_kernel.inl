@@ -326,7 +326,7 @@ __device__ __forceinline__ void stage_tile(int tid, const TileJob &j, int blk_lo
 // cell are formed once per cell (1.5 times, with the slab's rim) instead of
 // six to seven times.
 //
-// LDS, in units of 256 values of R: Q (NQ per buffer, two buffers: the plane's
+// LDS, in units of 256 values: Q (NQ per buffer, two buffers: the plane's
 // packed cell quantities, the next plane's written by the x faces), HQ (NQ:
 // those of the halo cells at j = -1 and k = -1, all planes), FZ, EX (the closing
 // fluxes) and two buffers of FY (NE each): 70 KB in FP64, two workgroups per
@@ -340,11 +340,11 @@ __device__ __forceinline__ void stage_tile(int tid, const TileJob &j, int blk_lo
 // marching an 8^3 tile by itself, without barriers, was slower (one step, HLLC
 // exact 13.3 ms against 12.06, FMA 9.96 ms against 7.46): its waves drift apart
 // and their planes no longer share the caches (1.3e8 L2 misses a launch).
-template <typename R> struct MarchShape {
+struct MarchShape {
   static constexpr int SX = 8;
   static constexpr int SLABS = kIC / SX;
   static constexpr int PLANE = kIC * kIC;  // cells of a plane = threads
-  static constexpr int NQ = PackedQ<R>::NQ;
+  static constexpr int NQ = kPackedQ;
   static constexpr int NE = 5;
   static constexpr int LDS = (3 * NQ + 4 * NE) * PLANE;
   static_assert(SX * 2 * kIC == PLANE, "one halo cell and one closing face per thread");
@@ -359,14 +359,15 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // Makes `off` available only once a and b are formed.
-template <typename R> __device__ __forceinline__ void after(int &off, R a, R b) {
+__device__ __forceinline__ void after(int &off, double a, double b) {
   asm volatile("" : "+v"(off) : "v"(a), "v"(b));
 }
 
-template <int FLUX, typename R>
-__device__ __forceinline__ void stage_march(const TileJob &j, int blk_local, int slab, R *lds) {
+template <int FLUX>
+__device__ __forceinline__ void stage_march(const TileJob &j, int blk_local, int slab, double *lds) {
+  using R = double;
   using D = Dims<3>;
-  using M = MarchShape<R>;
+  using M = MarchShape;
   constexpr int NE = M::NE, P = M::PLANE, SX = M::SX, NQ = M::NQ;
   int const tid = threadIdx.x;
   int const wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -380,7 +381,7 @@ __device__ __forceinline__ void stage_march(const TileJob &j, int blk_local, int
     double c[NE];
 #pragma unroll
     for (int e = 0; e < NE; ++e) c[e] = rd(off * (int)sizeof(double), e * D::FIELD * (int)sizeof(double));
-    store_packed<3, R, P>(j.gamma, j.b, c, q);
+    store_packed<3, P>(j.gamma, j.b, c, q);
   };
   // Halo offset of thread t's cell in plane p, and of the cell left of its
   // closing face (threads 0-127 the y side, 128-255 the z side; plane
@@ -436,7 +437,7 @@ __device__ __forceinline__ void stage_march(const TileJob &j, int blk_local, int
       int const yj = t / kIC, yk = t % kIC;
       const R *q = Q + (p & 1) * NQ * P;
       R fl[NE];
-      KeptQ<3, R, P> const qs{inner ? (yj > 0 ? q + t - kIC : HQ + p * kIC + yk) : Q + t,
+      KeptQ<3, P> const qs{inner ? (yj > 0 ? q + t - kIC : HQ + p * kIC + yk) : Q + t,
                               inner ? q + t : Q + NQ * P + t};
       if constexpr (AHEAD) {
         R cl[NE], cr[NE], skipped;
@@ -459,7 +460,7 @@ __device__ __forceinline__ void stage_march(const TileJob &j, int blk_local, int
       int const zj = t / kIC, zk = t % kIC;
       const R *q = Q + (p & 1) * NQ * P;
       R fl[NE];
-      KeptQ<3, R, P> const qs{inner ? (zk > 0 ? q + t - 1 : HQ + P / 2 + p * kIC + zj) : Q + t,
+      KeptQ<3, P> const qs{inner ? (zk > 0 ? q + t - 1 : HQ + P / 2 + p * kIC + zj) : Q + t,
                               inner ? q + t : Q + NQ * P + t};
       if constexpr (AHEAD) {
         if (!inner) load_stencil<3>(rd, closing(t, true), 1, U);
@@ -489,7 +490,7 @@ __device__ __forceinline__ void stage_march(const TileJob &j, int blk_local, int
         keep(here(t, p), Q + NQ * P + t);
         if constexpr (AHEAD && !COLUMN) load_stencil<3>(rd, here(t, p), D::SX, U);
       }
-      KeptThenFormedQ<3, R, P> const qs{j.gamma, j.b, Q + (p & 1) * NQ * P + t,
+      KeptThenFormedQ<3, P> const qs{j.gamma, j.b, Q + (p & 1) * NQ * P + t,
                                         Q + ((p + 1) & 1) * NQ * P + t};
       if constexpr (AHEAD) {
         R cl[NE], cr[NE], skipped;
@@ -588,18 +589,18 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(kMinWaves<DI
 }
 
 // Single 3D case by plane marching: one workgroup per (block, slab).
-template <int FLUX, typename R>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMinWaves<3, FLUX, R>, 8))) void march_stage_kernel(
+template <int FLUX>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kMinWaves<3, FLUX, double>, 8))) void march_stage_kernel(
     const double *__restrict__ avg, const double *init, double *out, alpaca_case_state *state,
     StageArgs a) {
-  constexpr unsigned SLABS = MarchShape<R>::SLABS;
-  __shared__ R lds[MarchShape<R>::LDS];
+  constexpr unsigned SLABS = MarchShape::SLABS;
+  __shared__ double lds[MarchShape::LDS];
   unsigned const g = xcd_remap_group(blockIdx.x, gridDim.x);
   int const blk = g / SLABS;
   if (blk >= a.nblocks) return;  // uniform over the workgroup
   if (a.guard && (state->flags & kFlagDone)) return;
   TileJob const j = stage_job(avg, init, out, state, a);
-  stage_march<FLUX, R>(j, blk, g % SLABS, lds);
+  stage_march<FLUX>(j, blk, g % SLABS, lds);
 }
 
 // Large 2D cases: one workgroup of 192 threads per two blocks adjacent in
