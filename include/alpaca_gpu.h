@@ -73,7 +73,7 @@ typedef struct alpaca_case_desc {
   int nb[3];          /* leaf blocks per direction; nb[2] = 1 in 2D */
   int bc[3];          /* ALPACA_BC_* per direction (both sides alike) */
   int flux;           /* ALPACA_FLUX_* */
-  int precision;      /* ALPACA_FP64 / ALPACA_MIXED */
+  int precision;      /* ALPACA_FP64 / ALPACA_FP64_FMA / ALPACA_MIXED */
   double gamma;       /* stiffened-gas gamma (StiffenedGas, stiffened_gas.cpp:41) */
   double background_pressure; /* stiffened-gas B; 0 = ideal gas */
   double cell_size;   /* dx of the level-0 cells (Node::GetCellSize) */
@@ -98,11 +98,14 @@ int alpaca_abi_version(void);
 
 /* Kernel classes for the timing hooks below. */
 enum {
-  ALPACA_KERNEL_FACE_FLUX = 0, /* reconstruction + Riemann / splitting fluxes */
-  ALPACA_KERNEL_COMBINE = 1,   /* flux divergence + RK stage combination */
+  ALPACA_KERNEL_FACE_FLUX = 0, /* reconstruction + Riemann / splitting fluxes
+                                  (alpaca_convective_fluxes) */
+  ALPACA_KERNEL_COMBINE = 1,   /* flux divergence + RK stage combination as a launch of
+                                  its own: none, every path fuses it into STAGE */
   ALPACA_KERNEL_HALO = 2,      /* same-level halo fill + boundary conditions */
   ALPACA_KERNEL_TIMESTEP = 3,  /* CFL reduction */
-  ALPACA_KERNEL_STAGE = 4,     /* fused stage: faces + divergence + RK + halo */
+  ALPACA_KERNEL_STAGE = 4,     /* fused stage: faces + divergence + RK + halo; also the
+                                  right-hand sides: faces + divergence + jump fluxes */
   ALPACA_KERNEL_COUNT = 5
 };
 
@@ -111,8 +114,7 @@ enum {
  * by HIP events on its launch stream.  alpaca_profile_read synchronises on
  * the recorded events and returns the summed milliseconds, the number of
  * launches and the algorithmic work units launched (faces for FACE_FLUX,
- * cells for COMBINE, TIMESTEP and STAGE, halo cells for HALO); reset != 0
- * clears. */
+ * cells for TIMESTEP and STAGE, halo cells for HALO); reset != 0 clears. */
 int alpaca_profile_enable(int on);
 int alpaca_profile_read(int kernel, int reset, double *total_ms, long long *launches,
                         double *units);
@@ -120,26 +122,27 @@ int alpaca_profile_read(int kernel, int reset, double *total_ms, long long *laun
 /* Doubles per haloed block (NE * 24^dim). */
 size_t alpaca_block_doubles(int dim);
 
-/* Contexts of the per-block entries (i) and (ii).  The reference keeps its
- * face-flux arrays on the stack of SpaceSolver::UpdateFluxes
- * (space_solver.cpp:50-116), one set per call; here those faces go to device
- * scratch, which a context owns together with the HIP stream its calls are
- * queued on.  Use one context per host thread or stream: calls on one context
- * are ordered by its stream and share its scratch, calls on different
- * contexts never share scratch.  Scratch grows on demand without a device
- * synchronisation (outgrown buffers are kept until alpaca_context_destroy,
- * which synchronises the context's stream and frees them).  The
- * stream-argument forms (alpaca_convective_fluxes, alpaca_right_hand_side,
- * alpaca_right_hand_side_jump_fluxes) use an implicit context per (device,
- * stream), kept until the process ends; prefer an explicit context for
- * streams that are created and destroyed during the run. */
+/* Contexts of the per-block entries (i) and (ii): the HIP stream a context's
+ * calls are queued on and the device they run on (the entries over a whole array
+ * of blocks refuse another current device).  The reference keeps its face-flux arrays on the stack
+ * of SpaceSolver::UpdateFluxes (space_solver.cpp:50-116), one set per call;
+ * here the convective fluxes (i) go through device scratch that the context
+ * owns, and the right-hand sides (ii) keep their faces in LDS and use none.
+ * Use one context per host thread or stream: calls on one context are ordered
+ * by its stream and share its scratch, calls on different contexts never share
+ * scratch.  Scratch grows on demand without a device synchronisation (outgrown
+ * buffers are kept until alpaca_context_destroy, which synchronises the
+ * context's stream and frees them).  The stream-argument form
+ * alpaca_convective_fluxes uses an implicit context per (device, stream), kept
+ * until the process ends; prefer an explicit context for streams that are
+ * created and destroyed during the run. */
 typedef struct alpaca_context alpaca_context;
 /* Binds a new context to the current device and to `stream` (NULL = the
  * default stream). */
 int alpaca_context_create(void *stream, alpaca_context **out);
 int alpaca_context_destroy(alpaca_context *ctx);
-/* Grows the context's scratch to what nblocks blocks of dimension dim need,
- * so later calls up to that size allocate nothing. */
+/* Grows the context's scratch to what the convective fluxes of nblocks blocks
+ * of dimension dim need, so later calls up to that size allocate nothing. */
 int alpaca_context_reserve(alpaca_context *ctx, int dim, int nblocks);
 
 /* (i) Per-block convective fluxes.
@@ -170,8 +173,8 @@ int alpaca_right_hand_side_jump_fluxes(const alpaca_case_desc *desc, int nblocks
                                        const double *d_avg, double *d_rhs,
                                        double *d_jump_fluxes, void *stream);
 
-/* (i) and (ii) on an explicit context (its stream and scratch); the same
- * results, bit for bit, as the stream-argument forms above. */
+/* (i) and (ii) on an explicit context (its stream, device and scratch); the
+ * same results, bit for bit, as the stream-argument forms above. */
 int alpaca_ctx_convective_fluxes(alpaca_context *ctx, const alpaca_case_desc *desc,
                                  int nblocks, const double *d_avg, double *d_fluxes);
 int alpaca_ctx_right_hand_side(alpaca_context *ctx, const alpaca_case_desc *desc,
