@@ -631,9 +631,8 @@ def main():
     achieved = head["cells_per_launch"] * flop_cell_stage / avg_launch_s
     peak = PEAK_FP32 if args.precision == "mixed" else PEAK_FP64
     tag = f"stage_3d_{args.flux}_{args.precision}"
-    variant = {"fp64": "exact::", "fp64-fma": "fast::", "mixed": "fast::"}[args.precision]
-    rtype = "float" if args.precision == "mixed" else "double"
-    prof = load_profile(tag)
+    # The stage kernel is chosen by the number of blocks; the profile is of 16^3.
+    prof = load_profile(tag) if nb == 16 else {}
     bound = "valu_fp32" if args.precision == "mixed" else "valu_fp64"
     roofline = {
         "bound": bound,
@@ -642,7 +641,7 @@ def main():
         "unit": "TFLOP/s",
         "frac": achieved / peak,
         "traffic": prof.get("hbm_bytes_per_launch"),
-        "kernel": f"{variant}stage_kernel<3,{'HLLC' if flux == 0 else 'Roe'},{rtype},8,8,8,256>",
+        "kernel": prof.get("kernel") or f"stage kernel of {nb}^3 blocks, {args.flux}, {args.precision}",
         "note": (f"compute roofline (the contract's 'mfma' slot): a VALU stencil, no contraction "
                  f"maps to MFMA, so the peak is the {'FP32' if args.precision == 'mixed' else 'FP64'} "
                  f"vector figure; achieved = {flop_cell_stage:.0f} algorithmic FLOP per cell and "
