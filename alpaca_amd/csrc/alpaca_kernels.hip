@@ -2,12 +2,12 @@
 // single-phase finite-volume right-hand side.
 //
 // Kernels (one launch each, all on the caller's stream):
-//   face_flux_kernel<DIM,DIR,FLUX,R>  one thread per cell face; six-cell
+//   face_flux_kernel<DIM,DIR,FLUX,MODE>  one thread per cell face; six-cell
 //       stencil read straight from the haloed block (coalesced along k);
 //       Roe eigensystem + characteristic WENO5 + HLLC or Roe splitting.
 //       Only the per-block convective-flux entry writes face fluxes out.
-//   stage_kernel, march_stage_kernel (stage_kernel.inl)  a whole RK stage:
-//       faces, flux divergence, RK combination, halos.
+//   stage_kernel, march_stage_kernel, pair_stage_kernel (stage_kernel.inl)  a whole
+//       RK stage: faces, flux divergence, RK combination, halos.
 //   halo_kernel<DIM>  face halo slabs from neighbours / zero-gradient / symmetry.
 //   signal_kernel<DIM> + dt_kernel  CFL reduction and time step.
 #include <hip/hip_runtime.h>
